@@ -1534,9 +1534,74 @@ static void local_energy_noalloc_impl(Ctx& c, rbmhip_psi* psi, rbmhip_op* op, co
 // ===========================================================================
 // C ABI
 // ===========================================================================
+static cx<double> cxd(cd z) { return mk(z.real(), z.imag()); }
+
 // Centred, weighted S over the parameters with an O_k (the `params` entries
-// after alpha and beta), FP32 MFMA Gram blocks accumulated in FP64; returns a
-// device array of P x P complex128 (eps added on the diagonal).
+// after alpha and beta), accumulated in FP64; returns a device array of P x P
+// complex128 (eps added on the diagonal).
+//
+// From PAIR_MIN_P parameters the second moments come from pairs of spins and
+// pairs of units (k_pair_moments), an eighth of the Gram product's matrix work
+// at 36 spins and 144 units: 7.4 ms against 40.3 ms on 65 536 samples.  They
+// are also the more accurate (1.1e-7 of the largest entry against 5.6e-6, 18
+// spins, 36 units, 28 700 samples): the FP32 sums of the matrix cores round
+// toward zero, and the Gram product's longer ones lose 3.4e-6 of the diagonal
+// on average.  Divided by a small eps that difference is visible in an update
+// (up to 5e-5 of it at eps = 1e-2 below a thousand parameters), so smaller
+// models, whose Gram product takes 1.7 to 4.9 ms (32 768 samples), keep it and the
+// updates they had.
+// S_kl from pairs is a difference of two sums, <conj(O_k) O_l> -
+// conj(<O_k>) <O_l>, which loses 1 / (1 - r) of the accuracy for r =
+// |<s_p t_j>|^2 / <|t_j|^2> (1 where a unit follows one spin); beyond
+// PAIR_RATIO the O_k rows are centred before the product (k_gram_lower_bf3).
+constexpr double PAIR_RATIO = 0.9;
+constexpr int PAIR_MIN_P = 2048;
+
+template <typename T>
+static bool s_matrix_pairs(Ctx& c, rbmhip_psi* psi, const Samples& s, double n, double eps, const cx<double>* w,
+                           const std::vector<cd>& R, int P, cx<double>* S) {
+    const int N = psi->N, M = psi->M;
+    // R[r][j] = sum_s w row_r conj(col_j)
+    std::vector<cx<double>> mean((size_t)M);
+    for (int j = 0; j < M; j++) mean[(size_t)j] = cxd(std::conj(R[(size_t)j]) / n);
+    cx<double>* dmean = reinterpret_cast<cx<double>*>(c.buf("pair_mean", mean.size() * sizeof(cx<double>)));
+    c.h2d(dmean, mean.data(), mean.size() * sizeof(cx<double>));
+    const PairShape sh = pair_shape(N, M);
+    const int64_t len = (int64_t)sh.rows_p * sh.cols_p, nblk = (s.n + 31) / 32;
+    // sample splits: fill the 2048 wavefronts that run at once (two per SIMD)
+    // as evenly as possible, at least 8 blocks and at most 2 GiB in all
+    const int64_t wp = (int64_t)sh.groups * sh.col_groups, slots = 8ll * c.num_cus;
+    const int64_t zmax = std::max<int64_t>(1, std::min(std::min<int64_t>(nblk / 8, (2ll << 30) / (len * 8)), std::max<int64_t>(8, 2 * slots / wp)));
+    int splits = 1;
+    double best = 0.0;
+    for (int64_t z = 1; z <= zmax; z++) {
+        const double used = (double)(wp * z) / (double)((wp * z + slots - 1) / slots * slots);
+        if (used > 1.02 * best) { best = used; splits = (int)z; }
+    }
+    const int64_t batch = std::min<int64_t>(nblk, std::max<int64_t>(1, (1ll << 30) / ((int64_t)(M + 1) * 256)));
+    uint32_t* planes = reinterpret_cast<uint32_t*>(c.buf("okplanes", (size_t)nblk * N * sizeof(uint32_t)));
+    uint32_t* signs = reinterpret_cast<uint32_t*>(c.buf("pair_signs", (size_t)batch * sh.rows_p * sizeof(uint32_t)));
+    float* units = reinterpret_cast<float*>(c.buf("pair_units", (size_t)batch * (M + 1) * 64 * sizeof(float)));
+    double* C = reinterpret_cast<double*>(c.buf("pair_moments", (size_t)splits * len * sizeof(double)));
+    double* ratio = reinterpret_cast<double*>(c.buf("pair_ratio", 16));
+    cx<double>* first = reinterpret_cast<cx<double>*>(c.buf("pair_first", (size_t)(N + 1) * (M + 1) * sizeof(cx<double>)));
+    c.launch("s_matrix", [&] { return launch_zero(2 * splits * len, reinterpret_cast<float*>(C), c.stream); });
+    c.launch("s_matrix", [&] { return launch_spin_planes(s.n, N, s.spins, planes, c.stream); });
+    for (int64_t b0 = 0; b0 < nblk; b0 += batch) {
+        const int64_t cur = std::min(batch, nblk - b0);
+        c.launch("s_matrix", [&] { return launch_pair_planes(cur, N, sh.rows_p, planes + b0 * N, signs, c.stream); });
+        c.launch("s_matrix", [&] { return launch_pair_units<T>(b0 * 32, s.n, cur, M, s.tanh, w, dmean, units, c.stream); });
+        c.launch("s_gram", [&] { return launch_pair_moments(sh, cur, splits, M, signs, units, C, c.stream); });
+    }
+    c.launch("s_matrix", [&] { return launch_pair_finish(sh, N, M, splits, 1.0 / n, C, ratio, c.stream); });
+    double r = 0.0;
+    c.d2h(&r, ratio, sizeof(double));
+    c.sync();
+    if (!(r <= PAIR_RATIO)) return false;
+    c.launch("s_matrix", [&] { return launch_pair_assemble(sh, N, M, P, 1.0 / n, eps, dmean, C, first, S, c.stream); });
+    return true;
+}
+
 template <typename T>
 static cx<double>* s_matrix_centred(Ctx& c, rbmhip_psi* psi, rbmhip_ens* ens, const Samples& s, double eps) {
     RBM_REQUIRE(psi->kind == 0, "the centred S-matrix is built for Psi");
@@ -1549,7 +1614,11 @@ static cx<double>* s_matrix_centred(Ctx& c, rbmhip_psi* psi, rbmhip_ens* ens, co
     a.n = s.n; a.mode = 4; a.exact = ens->kind == 0; a.num_configs = (double)ens->num_configs; a.mult = s.mult;
     a.log_prefactor = std::log(psi->prefactor); a.lp = s.lp; a.coef = w;
     c.launch("coef", [&] { return launch_coef(a, c.stream); });
-    const std::vector<cd> osum = contract_params<T>(c, psi, s.n, s.tanh, s.spins, w);
+    const std::vector<cd> R = ok_contract<T>(c, N, M, s.n, s.tanh, s.spins, w);
+    cx<double>* S = reinterpret_cast<cx<double>*>(c.buf("s_centred", (size_t)P * P * sizeof(cx<double>)));
+    if (P >= PAIR_MIN_P && s_matrix_pairs<T>(c, psi, s, n, eps, w, R, P, S)) return S;
+    std::vector<cd> osum;
+    rbm_params_from_R(psi, R.data(), osum);
     std::vector<cx<float>> obar((size_t)P);
     for (int k = 0; k < P; k++) {
         // the contraction gives sum_s w conj(O_k)
@@ -1578,7 +1647,6 @@ static cx<double>* s_matrix_centred(Ctx& c, rbmhip_psi* psi, rbmhip_ens* ens, co
             return launch_gram_lower(ld2, (int)curp, O, Gd, dorder, (int)order.size(), c.stream);
         });
     }
-    cx<double>* S = reinterpret_cast<cx<double>*>(c.buf("s_centred", (size_t)P * P * sizeof(cx<double>)));
     c.launch("s_matrix", [&] { return launch_s_assemble(P, ld2, 1.0 / n, eps, Gd, S, c.stream); });
     return S;
 }
@@ -2219,7 +2287,6 @@ int rbmhip_fluctuation(rbmhip_psi* psi, rbmhip_op* op, rbmhip_ens* ens, double* 
 // virtual configurations s'_n of every sample in chunks of at most about 1 GiB
 // of records.  Both contractions accumulate in FP64.  The reference's
 // gradient (ExpectationValue.cu:243-253) is (1, -2<E>, 0, 1) / n.
-static cx<double> cxd(cd z) { return mk(z.real(), z.imag()); }
 
 template <typename T>
 static std::vector<cd> gradient_ek_sums(Ctx& c, rbmhip_psi* psi, rbmhip_op* op, rbmhip_ens* ens, const Samples& s,

@@ -1,6 +1,7 @@
-// Gram product of the S-matrix rows on the bfloat16 matrix cores (the
-// centred S of a stochastic-reconfiguration step; the reference only builds
-// S, S_matrix.cu:10-58).
+// The centred S of a stochastic-reconfiguration step on the bfloat16 matrix
+// cores (the reference only builds S, S_matrix.cu:10-58): second moments by
+// pairs of spins and pairs of units (k_pair_moments), and the Gram product of
+// the O_k rows (k_gram_lower_bf3) for models whose moments cancel.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -148,6 +149,376 @@ hipError_t launch_gram_lower(int ld, int K, const uint32_t* A, double* C, const 
     if (ld <= 0 || ld % GM_T || K <= 0 || K % (2 * GB_K) || n_order <= 0) return hipErrorInvalidValue;
     hipLaunchKernelGGL(k_gram_lower_bf3, dim3((unsigned)n_order), dim3(128), 0, stream, ld, K,
                        reinterpret_cast<const uint4*>(A), C, order);
+    return hipGetLastError();
+}
+
+// ---------------------------------------------------------------------------
+// Second moments of an RBM's log-derivatives from pairs.  With the constant
+// spin s_0 = 1, the spins s_1 .. s_N, and the constant unit t_M = 1, every
+// O_k is a product s_p T_j, so
+//   <conj(O_(p,j)) O_(p',j')> = sum_s w s_p s_p' conj(T_j) T_j'
+// depends on the pair (p, p') through s_p s_p' alone, one of 1 + N (N + 1) / 2
+// sign rows, and on the pair (j, j') through one of (M + 1)^2 real columns.
+// The product of all sign rows with all unit pairs is a GEMM of
+// N^2 / 2 x M^2 x samples with one exact +-1 operand, where the Gram product
+// of the realified O_k rows takes (2 N M)^2 / 2 x samples products of two
+// split operands: 8 times fewer matrix products at N = 36, M = 144 (three
+// part products per pair product instead of six, and each pair once).
+//
+// Operands.  A: the sign rows' bits per 32-sample block (k_pair_planes); a
+// lane takes the byte of its K quarter and a 256-entry LDS table turns it
+// into the four packed bfloat16 +-1 pairs.  B: columns 2 c + part, part (Re,
+// Im) of t_j conj(t_j') for unit pair c = j (j + 1) / 2 + j' (j >= j'), formed
+// in FP32 from the centred, sqrt(w)-scaled unit values (k_pair_units, stored
+// per 32-sample block as [unit][Re, Im][32 samples], so that a lane loads its
+// 8 samples as two 16-byte words) and split exactly into three bfloat16
+// parts; v_mfma_f32_16x16x32_bf16 sums the exact products in FP32.
+//
+// A wavefront owns RT <= 12 row tiles and CT = 3 column tiles of one sample
+// split: B is formed once for RT row tiles (about 65 vector instructions per
+// column tile and K step against RT x 3 MFMAs of 16 cycles), and the 4 RT CT
+// accumulators leave two wavefronts per SIMD.  6x6 Heisenberg, M = 144, 65 536
+// samples: 6.6 ms, 43 % of the MFMA issue rate of its 2.36 ms, and 0.8 ms for
+// the operands and the assembly, where the Gram product took 37.6 + 2.7 ms;
+// what it waits for now is the loads and vector work of B, formed again by
+// each of the 4 row groups.  Every PAIR_FLUSH blocks the FP32
+// tile is added into the split's FP64 accumulator, so the FP32 error does not
+// grow with the sample count.
+// ---------------------------------------------------------------------------
+constexpr int PAIR_CT = 3, PAIR_RT_MAX = 12, PAIR_FLUSH = 128;
+
+// bits of the sign rows: row 0 is 1, row 1 + q (q - 1) / 2 + p is s_p s_q for
+// 0 <= p < q <= N with s_0 = 1; rows past the last read as 1
+__global__ __launch_bounds__(256) void k_pair_planes(int64_t nblk, int N, int rows_p, const uint32_t* __restrict__ planes,
+                                                     uint32_t* __restrict__ out) {
+    const int rows = 1 + N * (N + 1) / 2;
+    for (int64_t b = blockIdx.x; b < nblk; b += gridDim.x)
+        for (int r = threadIdx.x; r < rows_p; r += blockDim.x) {
+            uint32_t w = 0xFFFFFFFFu;
+            if (r >= 1 && r < rows) {
+                const int t = r - 1;
+                int q = (int)((1.0f + sqrtf(1.0f + 8.0f * (float)t)) * 0.5f);
+                while (q * (q - 1) / 2 > t) q--;
+                while ((q + 1) * q / 2 <= t) q++;
+                const int p = t - q * (q - 1) / 2;
+                w = planes[b * N + q - 1];
+                if (p > 0) w = ~(w ^ planes[b * N + p - 1]);
+            }
+            out[b * rows_p + r] = w;
+        }
+}
+
+// sqrt(w) (T_j - mean_j) for unit j < M, sqrt(w) for the constant unit M, of
+// samples [s0, s0 + 32 nblk) (zero past n), in the layout above.  One workgroup
+// per block: the records are read along their rows and turned in LDS.
+template <typename T>
+__global__ __launch_bounds__(256) void k_pair_units(int64_t s0, int64_t n, int M, const cx<T>* __restrict__ Trec,
+                                                    const cx<double>* __restrict__ w, const cx<double>* __restrict__ mean,
+                                                    float* __restrict__ out) {
+    constexpr int UC = 64;   // units per LDS stage
+    __shared__ float v[2][UC][33];
+    __shared__ float sw[32];
+    const int64_t base = s0 + (int64_t)blockIdx.x * 32;
+    if (threadIdx.x < 32) sw[threadIdx.x] = base + threadIdx.x < n ? (float)sqrt(w[base + threadIdx.x].re) : 0.0f;
+    for (int j0 = 0; j0 <= M; j0 += UC) {
+        __syncthreads();
+        for (int t = threadIdx.x; t < 32 * UC; t += blockDim.x) {
+            const int jj = t & (UC - 1), k = t / UC, j = j0 + jj;
+            float re = 0.0f, im = 0.0f;
+            if (j < M && base + k < n) {
+                const cx<T> x = Trec[(base + k) * M + j];
+                re = sw[k] * (float)(x.re - (T)mean[j].re);
+                im = sw[k] * (float)(x.im - (T)mean[j].im);
+            } else if (j == M) {
+                re = sw[k];
+            }
+            v[0][jj][k] = re;
+            v[1][jj][k] = im;
+        }
+        __syncthreads();
+        for (int t = threadIdx.x; t < 64 * UC; t += blockDim.x) {
+            const int k = t & 31, part = (t >> 5) & 1, jj = t >> 6, j = j0 + jj;
+            if (j <= M) out[((int64_t)blockIdx.x * (M + 1) + j) * 64 + part * 32 + k] = v[part][jj][k];
+        }
+    }
+}
+
+RBM_DI uint32_t gb_pair(float lo, float hi) {
+    const __bf16 a = (__bf16)lo, b = (__bf16)hi;
+    return (uint32_t)__builtin_bit_cast(uint16_t, a) | ((uint32_t)__builtin_bit_cast(uint16_t, b) << 16);
+}
+
+template <int RT>
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2)))
+void k_pair_moments(int64_t nblk, int splits, int groups, int col_groups, int M, int rows_p, int cols_p,
+                    const uint32_t* __restrict__ planes, const float* __restrict__ units, double* __restrict__ C) {
+    constexpr int CT = PAIR_CT;
+    __shared__ uint4 lut[256];
+    const int lane = threadIdx.x;
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+        const uint32_t byte = (uint32_t)(lane + 64 * e);
+        uint32_t q4[4];
+#pragma unroll
+        for (int q = 0; q < 4; q++)
+            q4[q] = 0xBF80BF80u ^ (((byte >> (2 * q)) & 1u) << 15) ^ (((byte >> (2 * q + 1)) & 1u) << 31);
+        lut[byte] = make_uint4(q4[0], q4[1], q4[2], q4[3]);
+    }
+    __syncthreads();
+    const int kk = lane >> 4, ii = lane & 15;
+    // the row groups of one column group and split run next to each other and
+    // read the same unit values
+    const int grp = blockIdx.x % groups, rest = blockIdx.x / groups;
+    const int cg = rest % col_groups, z = rest / col_groups;
+    const int row0 = grp * RT * 16, col0 = cg * CT * 16;
+    const int part = ii & 1;
+    const float sgn = part ? -1.0f : 1.0f;
+    const int pairs = (M + 1) * (M + 2) / 2;
+    int oj[CT], ojp[CT];   // float offsets of units j and j' of this lane's columns within a block
+#pragma unroll
+    for (int b = 0; b < CT; b++) {
+        int c = (col0 + 16 * b + ii) >> 1;
+        if (c >= pairs) c = 0;   // padding columns repeat the first pair; they are never read
+        int j = (int)((sqrtf(8.0f * (float)c + 1.0f) - 1.0f) * 0.5f);
+        while (j * (j + 1) / 2 > c) j--;
+        while ((j + 1) * (j + 2) / 2 <= c) j++;
+        oj[b] = j * 64;
+        ojp[b] = (c - j * (j + 1) / 2) * 64;
+    }
+    const int64_t per = (nblk + splits - 1) / splits;
+    const int64_t b0 = z * per, b1 = b0 + per < nblk ? b0 + per : nblk;
+    double* Cz = C + (int64_t)z * rows_p * cols_p;
+    const int64_t ustride = (int64_t)(M + 1) * 64;
+    for (int64_t f0 = b0; f0 < b1; f0 += PAIR_FLUSH) {
+        const int64_t f1 = f0 + PAIR_FLUSH < b1 ? f0 + PAIR_FLUSH : b1;
+        gbf32x4 acc[RT][CT];
+#pragma unroll
+        for (int a = 0; a < RT; a++)
+#pragma unroll
+            for (int b = 0; b < CT; b++) acc[a][b] = gbf32x4{0.f, 0.f, 0.f, 0.f};
+        for (int64_t blk = f0; blk < f1; blk++) {
+            const float* U = units + blk * ustride + 8 * kk;
+            const uint32_t* pl = planes + blk * rows_p + row0 + ii;
+            uint32_t byte[RT];
+#pragma unroll
+            for (int a = 0; a < RT; a++) byte[a] = pl[16 * a];
+            uint4 bh[CT], bm[CT], bl[CT];
+#pragma unroll
+            for (int b = 0; b < CT; b++) {
+                float x[8], y[8], re[8], im[8];
+                const float4* px = reinterpret_cast<const float4*>(U + oj[b] + 32 * part);
+                const float4* py = reinterpret_cast<const float4*>(U + oj[b] + 32 * (1 - part));
+                const float4* pr = reinterpret_cast<const float4*>(U + ojp[b]);
+                const float4* pi = reinterpret_cast<const float4*>(U + ojp[b] + 32);
+#pragma unroll
+                for (int h = 0; h < 2; h++) {
+                    *reinterpret_cast<float4*>(x + 4 * h) = px[h];
+                    *reinterpret_cast<float4*>(y + 4 * h) = py[h];
+                    *reinterpret_cast<float4*>(re + 4 * h) = pr[h];
+                    *reinterpret_cast<float4*>(im + 4 * h) = pi[h];
+                }
+                // Re = re_j re_j' + im_j im_j',  Im = im_j re_j' - re_j im_j'
+                uint32_t hi[4], mid[4], lo[4];
+#pragma unroll
+                for (int q = 0; q < 4; q++) {
+                    float v[2];
+#pragma unroll
+                    for (int h = 0; h < 2; h++) {
+                        const int k = 2 * q + h;
+                        v[h] = __builtin_fmaf(x[k], re[k], sgn * (y[k] * im[k]));
+                    }
+                    hi[q] = gb_pair(v[0], v[1]);
+                    const float r0 = v[0] - __uint_as_float(hi[q] << 16), r1 = v[1] - __uint_as_float(hi[q] & 0xFFFF0000u);
+                    mid[q] = gb_pair(r0, r1);
+                    lo[q] = gb_pair(r0 - __uint_as_float(mid[q] << 16), r1 - __uint_as_float(mid[q] & 0xFFFF0000u));
+                }
+                bh[b] = make_uint4(hi[0], hi[1], hi[2], hi[3]);
+                bm[b] = make_uint4(mid[0], mid[1], mid[2], mid[3]);
+                bl[b] = make_uint4(lo[0], lo[1], lo[2], lo[3]);
+                // one column tile's loads at a time: registers for RT = 12
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            uint4 next = lut[(byte[0] >> (8 * kk)) & 0xFFu];
+#pragma unroll
+            for (int a = 0; a < RT; a++) {
+                const gbbf16x8 A = __builtin_bit_cast(gbbf16x8, next);
+                if (a + 1 < RT) next = lut[(byte[a + 1] >> (8 * kk)) & 0xFFu];
+#pragma unroll
+                for (int b = 0; b < CT; b++)
+                    acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A, __builtin_bit_cast(gbbf16x8, bl[b]), acc[a][b], 0, 0, 0);
+#pragma unroll
+                for (int b = 0; b < CT; b++)
+                    acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A, __builtin_bit_cast(gbbf16x8, bm[b]), acc[a][b], 0, 0, 0);
+#pragma unroll
+                for (int b = 0; b < CT; b++)
+                    acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A, __builtin_bit_cast(gbbf16x8, bh[b]), acc[a][b], 0, 0, 0);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+#pragma unroll
+        for (int a = 0; a < RT; a++) {
+            double* Ca = Cz + (int64_t)(row0 + 16 * a + 4 * kk) * cols_p + col0 + ii;
+#pragma unroll
+            for (int b = 0; b < CT; b++)
+#pragma unroll
+                for (int v = 0; v < 4; v++) Ca[(int64_t)v * cols_p + 16 * b] += (double)acc[a][b][v];
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    }
+}
+
+PairShape pair_shape(int N, int M) {
+    PairShape s;
+    const int tiles = (1 + N * (N + 1) / 2 + 15) / 16;
+    s.groups = (tiles + PAIR_RT_MAX - 1) / PAIR_RT_MAX;
+    s.rt = (tiles + s.groups - 1) / s.groups;
+    s.rows_p = s.groups * s.rt * 16;
+    s.col_groups = ((M + 1) * (M + 2) + 16 * PAIR_CT - 1) / (16 * PAIR_CT);
+    s.cols_p = s.col_groups * 16 * PAIR_CT;
+    return s;
+}
+
+hipError_t launch_pair_planes(int64_t nblk, int N, int rows_p, const uint32_t* planes, uint32_t* out, hipStream_t stream) {
+    const unsigned g = (unsigned)(nblk < 65535 ? nblk : 65535);
+    hipLaunchKernelGGL(k_pair_planes, dim3(g), dim3(256), 0, stream, nblk, N, rows_p, planes, out);
+    return hipGetLastError();
+}
+
+template <typename T>
+hipError_t launch_pair_units(int64_t s0, int64_t n, int64_t nblk, int M, const void* Trec, const cx<double>* w,
+                             const cx<double>* mean, float* out, hipStream_t stream) {
+    if (nblk <= 0 || nblk > (1ll << 30)) return hipErrorInvalidValue;
+    hipLaunchKernelGGL((k_pair_units<T>), dim3((unsigned)nblk), dim3(256), 0, stream, s0, n, M,
+                       reinterpret_cast<const cx<T>*>(Trec), w, mean, out);
+    return hipGetLastError();
+}
+template hipError_t launch_pair_units<float>(int64_t, int64_t, int64_t, int, const void*, const cx<double>*, const cx<double>*,
+                                             float*, hipStream_t);
+template hipError_t launch_pair_units<double>(int64_t, int64_t, int64_t, int, const void*, const cx<double>*, const cx<double>*,
+                                              float*, hipStream_t);
+
+hipError_t launch_pair_moments(const PairShape& s, int64_t nblk, int splits, int M, const uint32_t* planes,
+                               const float* units, double* C, hipStream_t stream) {
+    if (nblk <= 0 || splits < 1 || s.rt < 1 || s.rt > PAIR_RT_MAX) return hipErrorInvalidValue;
+    const dim3 grid((unsigned)(s.groups * s.col_groups * splits));
+#define RBM_PAIR_CASE(R_)                                                                                              \
+    case R_:                                                                                                           \
+        hipLaunchKernelGGL((k_pair_moments<R_>), grid, dim3(64), 0, stream, nblk, splits, s.groups, s.col_groups, M,   \
+                           s.rows_p, s.cols_p, planes, units, C);                                                      \
+        break;
+    switch (s.rt) {
+        RBM_PAIR_CASE(1) RBM_PAIR_CASE(2) RBM_PAIR_CASE(3) RBM_PAIR_CASE(4) RBM_PAIR_CASE(5) RBM_PAIR_CASE(6)
+        RBM_PAIR_CASE(7) RBM_PAIR_CASE(8) RBM_PAIR_CASE(9) RBM_PAIR_CASE(10) RBM_PAIR_CASE(11) RBM_PAIR_CASE(12)
+        default: return hipErrorInvalidValue;
+    }
+#undef RBM_PAIR_CASE
+    return hipGetLastError();
+}
+
+// Sum of the sample splits into split 0, in order.
+__global__ __launch_bounds__(256) void k_pair_sum(int64_t len, int splits, double* __restrict__ C) {
+    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < len; i += (int64_t)gridDim.x * blockDim.x) {
+        double s = C[i];
+        for (int z = 1; z < splits; z++) s += C[(int64_t)z * len + i];
+        C[i] = s;
+    }
+}
+
+RBM_DI int pair_row(int p, int q) {   // sign row of s_p s_q
+    if (p == q) return 0;
+    const int lo = p < q ? p : q, hi = p < q ? q : p;
+    return 1 + hi * (hi - 1) / 2 + lo;
+}
+// <conj(t_j) t_j'> of sign row r
+RBM_DI cx<double> pair_moment(const double* __restrict__ C, int cols_p, int r, int j, int jp) {
+    const int hi = j > jp ? j : jp, lo = j > jp ? jp : j;
+    const double* c = C + (int64_t)r * cols_p + 2 * (hi * (hi + 1) / 2 + lo);
+    const double im = hi == lo ? 0.0 : c[1];
+    // the column holds t_hi conj(t_lo)
+    return mk(c[0], j > jp ? -im : im);
+}
+
+// mean of O_(p,j) = <s_p t_j> + mean_j <s_p>; first[p * (M + 1) + j], times n
+__global__ __launch_bounds__(256) void k_pair_first(int N, int M, int cols_p, const cx<double>* __restrict__ mean,
+                                                    const double* __restrict__ C, cx<double>* __restrict__ first) {
+    const int e = blockIdx.x * blockDim.x + threadIdx.x;
+    if (e >= (N + 1) * (M + 1)) return;
+    const int p = e / (M + 1), j = e % (M + 1);
+    const int r = pair_row(0, p);
+    const cx<double> t = conj(pair_moment(C, cols_p, r, j, M));   // <t_j conj(t_M)>
+    first[e] = j < M ? t + pair_moment(C, cols_p, r, M, M).re * mean[j] : t;
+}
+
+// S_kl = <conj(O_k) O_l> - conj(<O_k>) <O_l> with O_(p,j) = s_p (t_j + mean_j);
+// the upper triangle is the conjugate of the lower one
+__global__ __launch_bounds__(256) void k_pair_assemble(int N, int M, int P, int cols_p, double inv, double eps,
+                                                       const cx<double>* __restrict__ mean,
+                                                       const cx<double>* __restrict__ first,
+                                                       const double* __restrict__ C, cx<double>* __restrict__ S) {
+    const int row = blockIdx.y, WN = M + N * M;
+    auto spin = [&](int k) { return k < M ? 0 : k < WN ? 1 + (k - M) / M : 1 + k - WN; };
+    auto unit = [&](int k) { return k < M ? k : k < WN ? (k - M) % M : M; };
+    const int rp = spin(row), rj = unit(row);
+    for (int col = blockIdx.x * blockDim.x + threadIdx.x; col < P; col += gridDim.x * blockDim.x) {
+        const int cp = spin(col), cj = unit(col);
+        const bool lower = row >= col;
+        const int p = lower ? rp : cp, j = lower ? rj : cj, pl = lower ? cp : rp, jl = lower ? cj : rj;
+        const int r = pair_row(p, pl);
+        cx<double> m = pair_moment(C, cols_p, r, j, jl);
+        const cx<double> mj = j < M ? conj(mean[j]) : mk(0.0, 0.0), ml = jl < M ? mean[jl] : mk(0.0, 0.0);
+        // conj(t_j) mean_l + conj(mean_j) t_l + conj(mean_j) mean_l with t_M = 1
+        if (jl < M) m = m + pair_moment(C, cols_p, r, j, M) * ml;
+        if (j < M) m = m + mj * pair_moment(C, cols_p, r, M, jl);
+        if (j < M && jl < M) m = m + pair_moment(C, cols_p, r, M, M).re * (mj * ml);
+        cx<double> v = inv * m - (inv * conj(first[p * (M + 1) + j])) * (inv * first[pl * (M + 1) + jl]);
+        if (row == col) v = mk(v.re + eps, 0.0);
+        S[(int64_t)row * P + col] = lower ? v : conj(v);
+    }
+}
+
+// *ratio = the largest |<s_p t_j>|^2 / <|t_j|^2>: 1 where a unit follows one
+// spin, whose O_k = s_p T_j then hardly varies.  One workgroup.
+__global__ __launch_bounds__(256) void k_pair_ratio(int N, int M, int cols_p, double inv, const double* __restrict__ C,
+                                                    double* __restrict__ ratio) {
+    __shared__ double red[256];
+    double m = 0.0;
+    for (int e = threadIdx.x; e < N * M; e += 256) {
+        const int p = 1 + e / M, j = e % M;
+        const cx<double> f = pair_moment(C, cols_p, pair_row(0, p), j, M);
+        const double v = pair_moment(C, cols_p, 0, j, j).re;
+        const double r = v > 0.0 ? inv * (f.re * f.re + f.im * f.im) / v : 0.0;
+        m = r > m || r != r ? r : m;   // a NaN is kept
+    }
+    red[threadIdx.x] = m;
+    __syncthreads();
+    for (int w = 128; w > 0; w >>= 1) {
+        if ((int)threadIdx.x < w) {
+            const double a = red[threadIdx.x], b = red[threadIdx.x + w];
+            red[threadIdx.x] = b > a || b != b ? b : a;
+        }
+        __syncthreads();
+    }
+    if (threadIdx.x == 0) *ratio = red[0];
+}
+
+hipError_t launch_pair_finish(const PairShape& s, int N, int M, int splits, double inv, double* C, double* ratio,
+                              hipStream_t stream) {
+    const int64_t len = (int64_t)s.rows_p * s.cols_p;
+    if (splits > 1) {
+        const unsigned g = (unsigned)((len + 255) / 256 < 8192 ? (len + 255) / 256 : 8192);
+        hipLaunchKernelGGL(k_pair_sum, dim3(g), dim3(256), 0, stream, len, splits, C);
+    }
+    hipLaunchKernelGGL(k_pair_ratio, dim3(1), dim3(256), 0, stream, N, M, s.cols_p, inv, C, ratio);
+    return hipGetLastError();
+}
+
+hipError_t launch_pair_assemble(const PairShape& s, int N, int M, int P, double inv, double eps, const cx<double>* mean,
+                                const double* C, cx<double>* first, cx<double>* S, hipStream_t stream) {
+    if (P <= 0 || P > 65535) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(k_pair_first, dim3((unsigned)(((N + 1) * (M + 1) + 255) / 256)), dim3(256), 0, stream, N, M, s.cols_p,
+                       mean, C, first);
+    hipLaunchKernelGGL(k_pair_assemble, dim3((unsigned)((P + 255) / 256), (unsigned)P), dim3(256), 0, stream, N, M, P,
+                       s.cols_p, inv, eps, mean, first, C, S);
     return hipGetLastError();
 }
 

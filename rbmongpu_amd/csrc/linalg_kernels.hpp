@@ -27,6 +27,32 @@ hipError_t launch_gram_lower(int ld, int K, const uint32_t* A, double* C, const 
 // Fills order with the workgroup-to-tile map of launch_gram_lower for ld
 // (entries (bm, bn) with bn <= bm, or (-1, -1)); returns the number of tiles.
 int gram_tile_order(int ld, std::vector<int2>& order);
+// Second moments of the O_k by pairs (gram_kernels.hip).  rows_p sign rows
+// (row 0 is 1, row 1 + q (q - 1) / 2 + p is s_p s_q for p < q <= N, s_0 = 1) in
+// `groups` groups of rt 16-row tiles, cols_p real columns (2 c + part for unit
+// pair c = j (j + 1) / 2 + j', j' <= j <= M, unit M constant).
+struct PairShape {
+    int rt, groups, rows_p, col_groups, cols_p;
+};
+PairShape pair_shape(int N, int M);
+// Sign bits of the rows per 32-sample block (nblk x rows_p words) from the
+// spin bit planes (nblk x N words)
+hipError_t launch_pair_planes(int64_t nblk, int N, int rows_p, const uint32_t* planes, uint32_t* out, hipStream_t stream);
+// sqrt(w) (T_j - mean_j) of samples [s0, s0 + 32 nblk) (zero past n) as
+// [block][unit 0..M][Re, Im][32 samples]; Trec holds cx<T>, M per sample
+template <typename T>
+hipError_t launch_pair_units(int64_t s0, int64_t n, int64_t nblk, int M, const void* Trec, const cx<double>* w,
+                             const cx<double>* mean, float* out, hipStream_t stream);
+// C[z][row][col] += sum over the blocks of split z (splits equal ranges of the nblk blocks)
+hipError_t launch_pair_moments(const PairShape& s, int64_t nblk, int splits, int M, const uint32_t* planes,
+                               const float* units, double* C, hipStream_t stream);
+// Adds the splits into C[0]; *ratio = max |<s_p t_j>|^2 / <|t_j|^2> (inv = 1 / n)
+hipError_t launch_pair_finish(const PairShape& s, int N, int M, int splits, double inv, double* C, double* ratio,
+                              hipStream_t stream);
+// S (P x P, eps added on the diagonal) from C[0]; mean holds M values, first
+// (N + 1) x (M + 1) scratch
+hipError_t launch_pair_assemble(const PairShape& s, int N, int M, int P, double inv, double eps, const cx<double>* mean,
+                                const double* C, cx<double>* first, cx<double>* S, hipStream_t stream);
 // out[z] = X_z^T Y_z (ldx x ldy) for the row ranges z = 0 .. splits - 1 of
 // length K / splits of row-major K x ldx and K x ldy operands (same MFMA
 // tiles); ldx and ldy multiples of 128, K a multiple of 16 splits.

@@ -1063,6 +1063,12 @@ void ok_mfma_shape(int N, int M, int* rows_p, int* cols_p) {
 
 bool ok_mfma_needs_planes(int N) { return ok_uses_bf3(N); }
 
+hipError_t launch_spin_planes(int64_t n, int N, const uint64_t* spins, uint32_t* planes, hipStream_t stream) {
+    const int64_t nblk = (n + 31) / 32, waves = (nblk + 1) / 2;
+    hipLaunchKernelGGL(k_spin_planes, dim3((unsigned)((waves + 3) / 4)), dim3(256), 0, stream, n, N, nblk, spins, planes);
+    return hipGetLastError();
+}
+
 hipError_t launch_ok_mfma(int64_t n, int N, int M, const void* Trec, const uint64_t* spins, const cx<double>* coef,
                           int64_t chunk, int nchunks, int rows_p, int cols_p, float* partials, uint32_t* planes,
                           hipStream_t stream) {
@@ -1081,11 +1087,7 @@ hipError_t launch_ok_mfma(int64_t n, int N, int M, const void* Trec, const uint6
     if (ok_uses_bf3(N)) {
         // chunks are whole 32-sample blocks, and the bit-planes cover them
         if (!planes || chunk % 32) return hipErrorInvalidValue;
-        const int64_t nblk = (n + 31) / 32;
-        const int64_t waves = (nblk + 1) / 2;
-        hipLaunchKernelGGL(k_spin_planes, dim3((unsigned)((waves + 3) / 4)), dim3(256), 0, stream, n, N, nblk, spins,
-                           planes);
-        const hipError_t e = hipGetLastError();
+        const hipError_t e = launch_spin_planes(n, N, spins, planes, stream);
         if (e != hipSuccess) return e;
 #define RBM_MF_ROW(R_)                                                                                             \
     RBM_MF_CASE(k_ok_mfma_bf3, R_, 2, planes) RBM_MF_CASE(k_ok_mfma_bf3, R_, 3, planes)                            \

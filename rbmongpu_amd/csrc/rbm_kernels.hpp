@@ -126,6 +126,8 @@ constexpr int MFMA_SUM_SPLIT = 16;   // FP64 partial-sum groups (Psum holds MFMA
 // bit-planes: planes must hold ceil(n / 32) x N uint32 and chunk be a multiple
 // of 32; smaller N ignore planes (may be null).
 bool ok_mfma_needs_planes(int N);
+// spin bit planes: planes[blk * N + i] bit k = spin i of sample 32 blk + k is up
+hipError_t launch_spin_planes(int64_t n, int N, const uint64_t* spins, uint32_t* planes, hipStream_t stream);
 hipError_t launch_ok_mfma(int64_t n, int N, int M, const void* Trec, const uint64_t* spins, const cx<double>* coef,
                           int64_t chunk, int nchunks, int rows_p, int cols_p, float* partials, uint32_t* planes,
                           hipStream_t stream);
