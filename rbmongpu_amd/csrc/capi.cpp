@@ -1261,7 +1261,7 @@ static Scalars reduce_scalars(Ctx& c, int64_t n, const double* sc) {
 // R[r][col] = sum_s coef[s] row_r(s) conj(col(s)) for the RBM rows
 // {1, s_0..s_{N-1}} and columns {T_0..T_{M-1}, 1}: FP32 arithmetic on the
 // bfloat16 matrix cores (exact three-part split) for complex64 records, chunk
-// partials added in FP64; FP64 VALU on complex128 records.
+// partials added in FP64; FP64 matrix cores on complex128 records.
 template <typename T>
 static std::vector<cd> ok_contract(Ctx& c, int N, int M, int64_t n, const void* tanh, const uint64_t* spins,
                                    const cx<double>* coef, bool fp64_sums = false) {
@@ -1286,11 +1286,9 @@ static std::vector<cd> ok_contract(Ctx& c, int N, int M, int64_t n, const void* 
         });
         c.launch("partials_sum", [&] { return launch_mfma_finish((int)nch, N, M, rows_p, cols_p, part, psum, out, c.stream); });
     } else {
-        int64_t nb = std::min<int64_t>(1024, std::max<int64_t>(1, (256ll << 20) / (plen * 16)));
-        nb = std::min<int64_t>(nb, std::max<int64_t>(1, (n + 63) / 64));
-        const int64_t chunk = (n + nb - 1) / nb;
+        const int64_t chunk = ok_reduce_chunk(n, N, M), nb = (n + chunk - 1) / chunk;
         cx<double>* part = reinterpret_cast<cx<double>*>(c.buf("okpart", (size_t)(nb * plen) * sizeof(cx<double>)));
-        c.launch("ok_reduce", [&] { return launch_ok_reduce<T>(n, N, M, tanh, spins, coef, 1, chunk, (int)nb, part, c.stream); });
+        c.launch("ok_reduce", [&] { return launch_ok_reduce<T>(n, N, M, tanh, spins, coef, chunk, part, c.stream); });
         c.launch("partials_sum", [&] { return launch_partials_sum((int)nb, plen, part, out, c.stream); });
     }
     std::vector<cd> h((size_t)plen);

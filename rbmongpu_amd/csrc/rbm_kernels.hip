@@ -685,54 +685,88 @@ __global__ __launch_bounds__(256) void k_lse_partials(int64_t n, const cx<double
 }
 
 // ---------------------------------------------------------------------------
-// O_k contractions.  With rows r = {1, s_0 .. s_{N-1}} and columns
+// O_k contractions in FP64 (complex128 models, and the E_k estimators of
+// either precision).  With rows r = {1, s_0 .. s_{N-1}} and columns
 // c = {T_0 .. T_{M-1}, 1} (T_j = my_tanh(theta_j)):
-//   R[q][r][c] = sum_s coef_q[s] * row_r(s) * conj(col_c(s))
+//   R[r][c] = sum_s coef[s] * row_r(s) * conj(col_c(s))
 // covers sum w conj(O_b), sum w conj(O_W), sum w O_a and sum w (c = M, r = 0).
-// Each block reduces a contiguous chunk of samples in FP64 and writes its
-// partials; k_partials_sum adds blocks in fixed order (deterministic).
+// As the FP32 contraction below it is a real GEMM over the samples, here on
+// v_mfma_f64_16x16x4f64: A = the +-1 rows, B = column 2 c + part (Re, Im) of
+// coef conj(col_c); lane l supplies A[l % 16][l / 16] and B[l / 16][l % 16],
+// accumulator v of lane l is row l / 16 + 4 v, column l % 16.  One wavefront
+// owns RT row tiles and CT column tiles of one sample chunk, so that a record
+// is read once per RT rows; each chunk's partials are added in FP64 by
+// k_partials_sum in a fixed order.  N = 16, M = 64, 65 536 samples: 30 us, of
+// which the 77 MB of complex128 records and spins are 17 at the rate of a large
+// copy (76 us with one thread per 8 rows and column on the vector units).
 // ---------------------------------------------------------------------------
-template <typename T>
-__global__ __launch_bounds__(256) void k_ok_reduce(int64_t n, int N, int M, const cx<T>* __restrict__ Trec,
-                                                   const uint64_t* __restrict__ spins,
-                                                   const cx<double>* __restrict__ coef, int nc, int64_t chunk,
-                                                   cx<double>* __restrict__ partials) {
-    constexpr int RB = OK_ROWS_PER_THREAD;
+typedef double doublex4 __attribute__((ext_vector_type(4)));
+
+template <typename T, int RT, int CT>
+__global__ __launch_bounds__(64) void k_ok_mfma_f64(int64_t n, int N, int M, const cx<T>* __restrict__ Trec,
+                                                    const uint64_t* __restrict__ spins,
+                                                    const cx<double>* __restrict__ coef, int64_t chunk, int ry, int cz,
+                                                    cx<double>* __restrict__ partials) {
+    const int lane = threadIdx.x;
+    const int kk = lane >> 4, ii = lane & 15;
+    const int tile = blockIdx.x % (ry * cz);
+    const int64_t chunk_id = blockIdx.x / (ry * cz);
+    const int rt0 = (tile % ry) * RT, ct0 = (tile / ry) * CT;
     const int R = N + 1, C = M + 1;
-    const int nrb = (R + RB - 1) / RB;
-    const int nwork = nrb * C;
-    const int64_t s_begin = (int64_t)blockIdx.x * chunk;
+    doublex4 acc[RT][CT];
+#pragma unroll
+    for (int a = 0; a < RT; a++)
+#pragma unroll
+        for (int b = 0; b < CT; b++) acc[a][b] = doublex4{0.0, 0.0, 0.0, 0.0};
+    const int part = ii & 1;
+    int coff[CT];
+    double cload[CT], cfix[CT];
+#pragma unroll
+    for (int b = 0; b < CT; b++) {
+        const int j = (16 * (ct0 + b) + ii) >> 1;
+        coff[b] = j < M ? j : 0;               // clamped: always a valid load
+        cload[b] = j < M ? 1.0 : 0.0;          // take the loaded value
+        cfix[b] = j == M ? 1.0 : 0.0;          // the constant column
+    }
+    const int64_t s_begin = chunk_id * chunk;
     const int64_t s_end = s_begin + chunk < n ? s_begin + chunk : n;
-    const int64_t plen = (int64_t)nc * R * C;
-    for (int w0 = 0; w0 < nwork; w0 += blockDim.x) {
-        const int w = w0 + threadIdx.x;
-        if (w >= nwork) break;
-        const int col = w % C, rb = w / C;
-        cx<double> acc[2][RB];
+#pragma unroll 2
+    for (int64_t s0 = s_begin; s0 < s_end; s0 += 4) {
+        const int64_t s = s0 + kk;
+        const bool ok = s < s_end;
+        const int64_t sc = ok ? s : s_begin;
+        const cx<double> c = coef[sc];
+        const uint64_t w0 = spins[2 * sc], w1 = spins[2 * sc + 1];
+        const double cre = ok ? c.re : 0.0, cim = ok ? c.im : 0.0;
+        // Re(c conj t) = cre tr + cim ti,  Im(c conj t) = cim tr - cre ti
+        const double p = part ? cim : cre, q = part ? -cre : cim;
+        const cx<T>* Tr = Trec + sc * M;
+        double bv[CT];
 #pragma unroll
-        for (int q = 0; q < 2; q++)
+        for (int b = 0; b < CT; b++) {
+            const cx<T> t = Tr[coff[b]];
+            bv[b] = fm(p, fm((double)t.re, cload[b], cfix[b]), q * ((double)t.im * cload[b]));
+        }
 #pragma unroll
-            for (int r = 0; r < RB; r++) acc[q][r] = mk(0.0, 0.0);
-        for (int64_t s = s_begin; s < s_end; s++) {
-            const cx<double> tv = col < M ? conj(to_d(Trec[s * M + col])) : mk(1.0, 0.0);
-            const uint64_t s0 = spins[2 * s], s1 = spins[2 * s + 1];
-            const cx<double> y0 = coef[s] * tv;
-            const cx<double> y1 = nc > 1 ? coef[n + s] * tv : mk(0.0, 0.0);
+        for (int a = 0; a < RT; a++) {
+            const int r = 16 * (rt0 + a) + ii;
+            const double av = r == 0 ? 1.0 : (r <= N ? spin_of<double>(w0, w1, (r - 1) & 127) : 0.0);
 #pragma unroll
-            for (int r = 0; r < RB; r++) {
-                const int row = rb * RB + r;
-                const double sg = row == 0 ? 1.0 : spin_of<double>(s0, s1, row - 1);
-                acc[0][r] = acc[0][r] + sg * y0;
-                acc[1][r] = acc[1][r] + sg * y1;
+            for (int b = 0; b < CT; b++) acc[a][b] = __builtin_amdgcn_mfma_f64_16x16x4f64(av, bv[b], acc[a][b], 0, 0, 0);
+        }
+    }
+    double* out = reinterpret_cast<double*>(partials + chunk_id * R * C);
+#pragma unroll
+    for (int a = 0; a < RT; a++)
+#pragma unroll
+        for (int b = 0; b < CT; b++) {
+            const int col = 16 * (ct0 + b) + ii;
+#pragma unroll
+            for (int v = 0; v < 4; v++) {
+                const int r = 16 * (rt0 + a) + kk + 4 * v;
+                if (r < R && col < 2 * C) out[(int64_t)r * 2 * C + col] = acc[a][b][v];
             }
         }
-        for (int q = 0; q < nc; q++)
-#pragma unroll
-            for (int r = 0; r < RB; r++) {
-                const int row = rb * RB + r;
-                if (row < R) partials[(int64_t)blockIdx.x * plen + ((int64_t)q * R + row) * C + col] = acc[q][r];
-            }
-    }
 }
 
 // ---------------------------------------------------------------------------
@@ -1119,12 +1153,29 @@ hipError_t launch_mfma_finish(int nchunks, int N, int M, int rows_p, int cols_p,
     return hipGetLastError();
 }
 
+// out[i] = sum_b partials[b][i].  A workgroup takes 16 consecutive elements
+// (256 contiguous bytes a row) with 16 threads each, thread y adding rows
+// y, y + 16, ...; the 16 sums are added in order.  (One thread per element,
+// each adding 1024 rows one after the other: 259 us for 17 x 65 elements,
+// now 12.)
 __global__ __launch_bounds__(256) void k_partials_sum(int nblocks, int64_t len, const cx<double>* __restrict__ partials,
                                                       cx<double>* __restrict__ out) {
-    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < len; i += (int64_t)gridDim.x * blockDim.x) {
+    __shared__ cx<double> red[16][17];
+    const int x = threadIdx.x & 15, y = threadIdx.x >> 4;
+    for (int64_t i0 = (int64_t)blockIdx.x * 16; i0 < len; i0 += (int64_t)gridDim.x * 16) {
+        const int64_t i = i0 + x;
         cx<double> s = mk(0.0, 0.0);
-        for (int b = 0; b < nblocks; b++) s = s + partials[(int64_t)b * len + i];
-        out[i] = s;
+        if (i < len) {
+#pragma unroll 4
+            for (int b = y; b < nblocks; b += 16) s = s + partials[(int64_t)b * len + i];
+        }
+        red[y][x] = s;
+        __syncthreads();
+        if (y == 0 && i < len) {
+            for (int k = 1; k < 16; k++) s = s + red[k][x];
+            out[i] = s;
+        }
+        __syncthreads();
     }
 }
 
@@ -1402,17 +1453,54 @@ hipError_t launch_eval(const RbmDev<T>& md, const OpDev& op, int has_op, int64_t
     return hipGetLastError();
 }
 
+// Tiling of the FP64 contraction: all row tiles up to 5 in one wavefront with 3
+// column tiles (2 beyond: 9 row tiles at N = 128), the accumulators taking
+// 8 RT CT registers.
+static void f64_tiling(int N, int M, int& RT, int& CT, int& ry, int& cz) {
+    const int rt = (N + 1 + 15) / 16, ct = (2 * (M + 1) + 15) / 16;
+    ry = (rt + 4) / 5;
+    RT = (rt + ry - 1) / ry;
+    CT = ct < 3 ? ct : 3;
+    cz = (ct + CT - 1) / CT;
+}
+
+int64_t ok_reduce_chunk(int64_t n, int N, int M) {
+    int RT, CT, ry, cz;
+    f64_tiling(N, M, RT, CT, ry, cz);
+    // about 4096 wavefronts, at least 32 samples each, at most 256 MiB of partials
+    const int64_t bytes = (int64_t)(N + 1) * (M + 1) * 16;
+    int64_t nb = 4096 / ((int64_t)ry * cz);
+    if (nb > (256ll << 20) / bytes) nb = (256ll << 20) / bytes;
+    if (nb > (n + 31) / 32) nb = (n + 31) / 32;
+    if (nb < 1) nb = 1;
+    return ((n + nb - 1) / nb + 3) / 4 * 4;   // whole 4-sample K steps
+}
+
 template <typename T>
 hipError_t launch_ok_reduce(int64_t n, int N, int M, const void* Trec, const uint64_t* spins, const cx<double>* coef,
-                            int nc, int64_t chunk, int nblocks, cx<double>* partials, hipStream_t stream) {
-    hipLaunchKernelGGL((k_ok_reduce<T>), dim3(nblocks), dim3(256), 0, stream, n, N, M,
-                       reinterpret_cast<const cx<T>*>(Trec), spins, coef, nc, chunk, partials);
-    return hipGetLastError();
+                            int64_t chunk, cx<double>* partials, hipStream_t stream) {
+    if (n <= 0 || chunk <= 0 || chunk % 4) return hipErrorInvalidValue;
+    int RT, CT, ry, cz;
+    f64_tiling(N, M, RT, CT, ry, cz);
+    const int64_t nb = (n + chunk - 1) / chunk;
+    const dim3 grid((unsigned)(nb * ry * cz));
+    const cx<T>* Tr = reinterpret_cast<const cx<T>*>(Trec);
+#define RBM_F64_CASE(R_, C_)                                                                                           \
+    if (RT == R_ && CT == C_) {                                                                                        \
+        hipLaunchKernelGGL((k_ok_mfma_f64<T, R_, C_>), grid, dim3(64), 0, stream, n, N, M, Tr, spins, coef, chunk, ry,  \
+                           cz, partials);                                                                              \
+        return hipGetLastError();                                                                                      \
+    }
+#define RBM_F64_ROW(R_) RBM_F64_CASE(R_, 1) RBM_F64_CASE(R_, 2) RBM_F64_CASE(R_, 3)
+    RBM_F64_ROW(1) RBM_F64_ROW(2) RBM_F64_ROW(3) RBM_F64_ROW(4) RBM_F64_ROW(5)
+#undef RBM_F64_ROW
+#undef RBM_F64_CASE
+    return hipErrorInvalidValue;
 }
 
 hipError_t launch_partials_sum(int nblocks, int64_t len, const cx<double>* partials, cx<double>* out, hipStream_t stream) {
-    int64_t g = (len + 255) / 256;
-    if (g > 4096) g = 4096;
+    int64_t g = (len + 15) / 16;
+    if (g > 65536) g = 65536;
     hipLaunchKernelGGL(k_partials_sum, dim3((unsigned)g), dim3(256), 0, stream, nblocks, len, partials, out);
     return hipGetLastError();
 }
@@ -1785,8 +1873,8 @@ template hipError_t launch_mc<float>(const RbmDev<float>&, const McParams&, uint
 template hipError_t launch_mc<double>(const RbmDev<double>&, const McParams&, uint64_t*, uint32_t*, bool, size_t, hipStream_t);
 template hipError_t launch_eval<float>(const RbmDev<float>&, const OpDev&, int, int64_t, const uint64_t*, uint64_t, const Records&, bool, size_t, int, hipStream_t);
 template hipError_t launch_eval<double>(const RbmDev<double>&, const OpDev&, int, int64_t, const uint64_t*, uint64_t, const Records&, bool, size_t, int, hipStream_t);
-template hipError_t launch_ok_reduce<float>(int64_t, int, int, const void*, const uint64_t*, const cx<double>*, int, int64_t, int, cx<double>*, hipStream_t);
-template hipError_t launch_ok_reduce<double>(int64_t, int, int, const void*, const uint64_t*, const cx<double>*, int, int64_t, int, cx<double>*, hipStream_t);
+template hipError_t launch_ok_reduce<float>(int64_t, int, int, const void*, const uint64_t*, const cx<double>*, int64_t, cx<double>*, hipStream_t);
+template hipError_t launch_ok_reduce<double>(int64_t, int, int, const void*, const uint64_t*, const cx<double>*, int64_t, cx<double>*, hipStream_t);
 template hipError_t launch_s_matrix_ref<float>(int64_t, int, int, int, const void*, const uint64_t*, double, cx<double>*, hipStream_t);
 template hipError_t launch_s_matrix_ref<double>(int64_t, int, int, int, const void*, const uint64_t*, double, cx<double>*, hipStream_t);
 

@@ -69,7 +69,6 @@ constexpr int MC_DRAW_BLOCK = 32;
 constexpr int MC_RESYNC_SWEEPS = 16;
 
 constexpr int SC_STRIDE = 4;
-constexpr int OK_ROWS_PER_THREAD = 8;
 
 struct CoefArgs {
     int64_t n;
@@ -113,9 +112,12 @@ template <typename T>
 hipError_t launch_rbm_log_ratio(const RbmDev<T>& md, const void* dW, const void* db, const cx<double>* da, int64_t n,
                                 const uint64_t* configs, uint64_t index_base, const cx<double>* lp, cx<double>* lp2,
                                 int max_blocks, hipStream_t stream);
+// FP64 contraction R[r][c] = sum_s coef[s] row_r(s) conj(col_c(s)) in chunks of
+// ok_reduce_chunk samples; partials holds ceil(n / chunk) x (N + 1) x (M + 1)
+int64_t ok_reduce_chunk(int64_t n, int N, int M);
 template <typename T>
 hipError_t launch_ok_reduce(int64_t n, int N, int M, const void* Trec, const uint64_t* spins, const cx<double>* coef,
-                            int nc, int64_t chunk, int nblocks, cx<double>* partials, hipStream_t stream);
+                            int64_t chunk, cx<double>* partials, hipStream_t stream);
 // FP32 MFMA contraction (complex64 records): P[m][n] = sum_s A_m(s) B_n(s)
 // with m = 2r + part (rows {1, s_i}, Re/Im of the coefficient) and
 // n = 2j + part (columns {T_j, 1}, Re/Im); per-chunk FP32 partials.
