@@ -2514,7 +2514,18 @@ int rbmhip_s_matrix(rbmhip_psi* psi, rbmhip_ens* ens, double* out) {
             Samples s = sample<T>(c, psi, nullptr, ens, true, true);
             cx<double>* S = reinterpret_cast<cx<double>*>(c.buf("smat", (size_t)(P * P) * sizeof(cx<double>)));
             const double inv = 1.0 / (double)ens->num_steps();
-            c.launch("s_matrix", [&] { return launch_s_matrix_ref<T>(s.n, psi->N, psi->M, psi->has_a, s.tanh, s.spins, inv, S, c.stream); });
+            const PairShape sh = pair_shape_f64(psi->N, psi->M);
+            // sample splits of whole 4-sample steps: about a wavefront per SIMD,
+            // at least 32 samples each and at most 2 GiB of moments
+            const int64_t wp = (int64_t)sh.groups * sh.col_groups, len = (int64_t)sh.rows_p * sh.cols_p;
+            int64_t splits = std::min<int64_t>(std::min<int64_t>(4ll * c.num_cus / wp, s.n / 32), (2ll << 30) / (len * 8));
+            splits = std::max<int64_t>(1, splits);
+            const int64_t per = ((s.n + splits - 1) / splits + 3) / 4 * 4;
+            splits = (s.n + per - 1) / per;
+            double* C = reinterpret_cast<double*>(c.buf("pair_moments", (size_t)(splits * len) * sizeof(double)));
+            c.launch("s_matrix", [&] {
+                return launch_s_matrix_ref<T>(sh, s.n, (int)splits, psi->N, psi->M, (int)P, s.tanh, s.spins, inv, C, S, c.stream);
+            });
             c.d2h(out, S, (size_t)(P * P) * sizeof(cx<double>));
             c.sync();
         });

@@ -522,4 +522,150 @@ hipError_t launch_pair_assemble(const PairShape& s, int N, int M, int P, double 
     return hipGetLastError();
 }
 
+// ---------------------------------------------------------------------------
+// get_S_matrix (source/network_functions/S_matrix.cu:10-58, CPU semantics),
+// S_kl = inv sum_s O_k(s) conj(O_l(s)), unweighted and uncentred, in FP64: the
+// same sign rows and unit pairs as k_pair_moments (T_j as they are, no
+// weights), the product on v_mfma_f64_16x16x4f64 (lane l supplies
+// A[l % 16][l / 16] and B[l / 16][l % 16], accumulator v is row l / 16 + 4 v).
+// A wavefront owns RT <= 4 row tiles and 2 column tiles of one sample split.
+// N = 10, M = 20 (1024 states, 240 x 240): moments, sum and assembly 30 us, where
+// one thread per entry running down all states took 608.
+// ---------------------------------------------------------------------------
+typedef double gbf64x4 __attribute__((ext_vector_type(4)));
+constexpr int PAIR64_RT_MAX = 4, PAIR64_CT = 2;
+
+template <typename T, int RT>
+__global__ __launch_bounds__(64) void k_pair_moments_f64(int64_t n, int64_t per, int N, int M, int groups, int col_groups,
+                                                         int rows_p, int cols_p, const cx<T>* __restrict__ Trec,
+                                                         const uint64_t* __restrict__ spins, double* __restrict__ C) {
+    constexpr int CT = PAIR64_CT;
+    const int lane = threadIdx.x, kk = lane >> 4, ii = lane & 15;
+    const int grp = blockIdx.x % groups, rest = blockIdx.x / groups;
+    const int cg = rest % col_groups, z = rest / col_groups;
+    const int row0 = grp * RT * 16, col0 = cg * CT * 16;
+    const int rows = 1 + N * (N + 1) / 2, pairs = (M + 1) * (M + 2) / 2;
+    uint64_t m0[RT], m1[RT];   // the spins of each sign row (rows past the last read as 1)
+#pragma unroll
+    for (int a = 0; a < RT; a++) {
+        const int r = row0 + 16 * a + ii;
+        m0[a] = m1[a] = 0;
+        if (r >= 1 && r < rows) {
+            const int t = r - 1;
+            int q = (int)((1.0f + sqrtf(1.0f + 8.0f * (float)t)) * 0.5f);
+            while (q * (q - 1) / 2 > t) q--;
+            while ((q + 1) * q / 2 <= t) q++;
+            const int p = t - q * (q - 1) / 2;
+            flip_bit(m0[a], m1[a], q - 1);
+            if (p > 0) flip_bit(m0[a], m1[a], p - 1);
+        }
+    }
+    const int part = ii & 1;
+    int jh[CT], jl[CT];
+#pragma unroll
+    for (int b = 0; b < CT; b++) {
+        int c = (col0 + 16 * b + ii) >> 1;
+        if (c >= pairs) c = 0;   // padding columns repeat the first pair; they are never read
+        int j = (int)((sqrtf(8.0f * (float)c + 1.0f) - 1.0f) * 0.5f);
+        while (j * (j + 1) / 2 > c) j--;
+        while ((j + 1) * (j + 2) / 2 <= c) j++;
+        jh[b] = j;
+        jl[b] = c - j * (j + 1) / 2;
+    }
+    gbf64x4 acc[RT][CT];
+#pragma unroll
+    for (int a = 0; a < RT; a++)
+#pragma unroll
+        for (int b = 0; b < CT; b++) acc[a][b] = gbf64x4{0.0, 0.0, 0.0, 0.0};
+    const int64_t s_begin = z * per, s_end = s_begin + per < n ? s_begin + per : n;
+#pragma unroll 2
+    for (int64_t s0 = s_begin; s0 < s_end; s0 += 4) {
+        const int64_t s = s0 + kk;
+        const bool ok = s < s_end;
+        const int64_t sc = ok ? s : s_begin;
+        const uint64_t w0 = ~spins[2 * sc], w1 = ~spins[2 * sc + 1];
+        const cx<T>* Tr = Trec + sc * M;
+        double bv[CT];
+#pragma unroll
+        for (int b = 0; b < CT; b++) {
+            const cx<double> th = jh[b] < M ? to_d(Tr[jh[b] < M ? jh[b] : 0]) : mk(1.0, 0.0);
+            const cx<double> tl = jl[b] < M ? to_d(Tr[jl[b] < M ? jl[b] : 0]) : mk(1.0, 0.0);
+            // Re, Im of t_j conj(t_j')
+            const double v = part ? fm(th.im, tl.re, -(th.re * tl.im)) : fm(th.re, tl.re, th.im * tl.im);
+            bv[b] = ok ? v : 0.0;
+        }
+#pragma unroll
+        for (int a = 0; a < RT; a++) {
+            const int par = (__popcll(m0[a] & w0) + __popcll(m1[a] & w1)) & 1;
+            const double av = par ? -1.0 : 1.0;
+#pragma unroll
+            for (int b = 0; b < CT; b++) acc[a][b] = __builtin_amdgcn_mfma_f64_16x16x4f64(av, bv[b], acc[a][b], 0, 0, 0);
+        }
+    }
+    double* Cz = C + (int64_t)z * rows_p * cols_p;
+#pragma unroll
+    for (int a = 0; a < RT; a++)
+#pragma unroll
+        for (int b = 0; b < CT; b++)
+#pragma unroll
+            for (int v = 0; v < 4; v++)
+                Cz[(int64_t)(row0 + 16 * a + kk + 4 * v) * cols_p + col0 + 16 * b + ii] = acc[a][b][v];
+}
+
+// rows and columns below 2N (alpha, beta) are zero
+__global__ __launch_bounds__(256) void k_s_ref_assemble(int N, int M, int P, int cols_p, double inv,
+                                                        const double* __restrict__ C, cx<double>* __restrict__ S) {
+    const int row = blockIdx.y, WN = M + N * M;
+    auto spin = [&](int k) { return k < M ? 0 : k < WN ? 1 + (k - M) / M : 1 + k - WN; };
+    auto unit = [&](int k) { return k < M ? k : k < WN ? (k - M) % M : M; };
+    const int k = row - 2 * N;
+    for (int col = blockIdx.x * blockDim.x + threadIdx.x; col < P; col += gridDim.x * blockDim.x) {
+        const int l = col - 2 * N;
+        cx<double> v = mk(0.0, 0.0);
+        if (k >= 0 && l >= 0) v = inv * conj(pair_moment(C, cols_p, pair_row(spin(k), spin(l)), unit(k), unit(l)));
+        S[(int64_t)row * P + col] = v;
+    }
+}
+
+PairShape pair_shape_f64(int N, int M) {
+    PairShape s;
+    const int tiles = (1 + N * (N + 1) / 2 + 15) / 16;
+    s.groups = (tiles + PAIR64_RT_MAX - 1) / PAIR64_RT_MAX;
+    s.rt = (tiles + s.groups - 1) / s.groups;
+    s.rows_p = s.groups * s.rt * 16;
+    s.col_groups = ((M + 1) * (M + 2) + 16 * PAIR64_CT - 1) / (16 * PAIR64_CT);
+    s.cols_p = s.col_groups * 16 * PAIR64_CT;
+    return s;
+}
+
+template <typename T>
+hipError_t launch_s_matrix_ref(const PairShape& s, int64_t n, int splits, int N, int M, int P, const void* Trec,
+                               const uint64_t* spins, double inv, double* C, cx<double>* S, hipStream_t stream) {
+    if (n <= 0 || splits < 1 || P <= 0 || P > 65535 || s.rt < 1 || s.rt > PAIR64_RT_MAX) return hipErrorInvalidValue;
+    const dim3 grid((unsigned)(s.groups * s.col_groups * splits));
+    const int64_t per = ((n + splits - 1) / splits + 3) / 4 * 4;
+    if (per * (splits - 1) >= n) return hipErrorInvalidValue;   // every split has samples
+#define RBM_PAIR64_CASE(R_)                                                                                            \
+    case R_:                                                                                                           \
+        hipLaunchKernelGGL((k_pair_moments_f64<T, R_>), grid, dim3(64), 0, stream, n, per, N, M, s.groups,             \
+                           s.col_groups, s.rows_p, s.cols_p, reinterpret_cast<const cx<T>*>(Trec), spins, C);           \
+        break;
+    switch (s.rt) {
+        RBM_PAIR64_CASE(1) RBM_PAIR64_CASE(2) RBM_PAIR64_CASE(3) RBM_PAIR64_CASE(4)
+        default: return hipErrorInvalidValue;
+    }
+#undef RBM_PAIR64_CASE
+    const int64_t len = (int64_t)s.rows_p * s.cols_p;
+    if (splits > 1)
+        hipLaunchKernelGGL(k_pair_sum, dim3((unsigned)((len + 255) / 256 < 8192 ? (len + 255) / 256 : 8192)), dim3(256), 0,
+                           stream, len, splits, C);
+    hipLaunchKernelGGL(k_s_ref_assemble, dim3((unsigned)((P + 255) / 256), (unsigned)P), dim3(256), 0, stream, N, M, P,
+                       s.cols_p, inv, C, S);
+    return hipGetLastError();
+}
+template hipError_t launch_s_matrix_ref<float>(const PairShape&, int64_t, int, int, int, int, const void*, const uint64_t*,
+                                               double, double*, cx<double>*, hipStream_t);
+template hipError_t launch_s_matrix_ref<double>(const PairShape&, int64_t, int, int, int, int, const void*, const uint64_t*,
+                                                double, double*, cx<double>*, hipStream_t);
+
 }  // namespace rbmhip

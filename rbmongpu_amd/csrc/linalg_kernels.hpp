@@ -53,6 +53,13 @@ hipError_t launch_pair_finish(const PairShape& s, int N, int M, int splits, doub
 // (N + 1) x (M + 1) scratch
 hipError_t launch_pair_assemble(const PairShape& s, int N, int M, int P, double inv, double eps, const cx<double>* mean,
                                 const double* C, cx<double>* first, cx<double>* S, hipStream_t stream);
+// S_kl = inv sum_s O_k conj(O_l) in FP64 (P x P with the 2N zero rows and
+// columns of the axis angles first) over n samples in `splits` equal ranges of
+// whole 4-sample steps, none of them empty; C holds splits x rows_p x cols_p
+PairShape pair_shape_f64(int N, int M);
+template <typename T>
+hipError_t launch_s_matrix_ref(const PairShape& s, int64_t n, int splits, int N, int M, int P, const void* Trec,
+                               const uint64_t* spins, double inv, double* C, cx<double>* S, hipStream_t stream);
 // out[z] = X_z^T Y_z (ldx x ldy) for the row ranges z = 0 .. splits - 1 of
 // length K / splits of row-major K x ldx and K x ldy operands (same MFMA
 // tiles); ldx and ldy multiples of 128, K a multiple of 16 splits.

@@ -1179,38 +1179,6 @@ __global__ __launch_bounds__(256) void k_partials_sum(int nblocks, int64_t len, 
     }
 }
 
-// get_S_matrix (source/network_functions/S_matrix.cu:10-58, CPU semantics):
-// S[k][k'] = inv * sum_s O_k(s) conj(O_k'(s)), unweighted and uncentred;
-// rows/columns below 2N (alpha, beta) stay zero.
-template <typename T>
-__global__ __launch_bounds__(256) void k_s_matrix_ref(int64_t n, int N, int M, int has_a,
-                                                      const cx<T>* __restrict__ Trec,
-                                                      const uint64_t* __restrict__ spins, double inv,
-                                                      cx<double>* __restrict__ S) {
-    const int64_t P = 2 * (int64_t)N + M + (int64_t)N * M + (has_a ? N : 0);
-    for (int64_t e = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; e < P * P; e += (int64_t)gridDim.x * blockDim.x) {
-        const int64_t k = e / P - 2 * N, kp = e % P - 2 * N;
-        cx<double> acc = mk(0.0, 0.0);
-        if (k >= 0 && kp >= 0) {
-            for (int64_t s = 0; s < n; s++) {
-                const uint64_t s0 = spins[2 * s], s1 = spins[2 * s + 1];
-                const cx<T>* Tr = Trec + s * M;
-                auto ok = [&](int64_t kk) -> cx<double> {
-                    if (kk < M) return to_d(Tr[kk]);
-                    if (kk < M + (int64_t)N * M) {
-                        const int64_t i = (kk - M) / M, j = (kk - M) % M;
-                        return spin_of<double>(s0, s1, (int)i) * to_d(Tr[j]);
-                    }
-                    return mk(spin_of<double>(s0, s1, (int)(kk - M - (int64_t)N * M)), 0.0);
-                };
-                acc = acc + ok(k) * conj(ok(kp));
-            }
-            acc = inv * acc;
-        }
-        S[e] = acc;
-    }
-}
-
 __global__ void k_activation(int64_t n, const cx<double>* __restrict__ z, cx<double>* __restrict__ out, int deriv) {
     for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
         out[i] = deriv ? dlogcosh(z[i]) : logcosh(z[i]);
@@ -1570,17 +1538,6 @@ hipError_t launch_lse_partials(int64_t n, const cx<double>* lp, double log_prefa
     return hipGetLastError();
 }
 
-template <typename T>
-hipError_t launch_s_matrix_ref(int64_t n, int N, int M, int has_a, const void* Trec, const uint64_t* spins, double inv,
-                               cx<double>* S, hipStream_t stream) {
-    const int64_t P = 2 * (int64_t)N + M + (int64_t)N * M + (has_a ? N : 0);
-    int64_t g = (P * P + 255) / 256;
-    if (g > 8192) g = 8192;
-    hipLaunchKernelGGL((k_s_matrix_ref<T>), dim3((unsigned)g), dim3(256), 0, stream, n, N, M, has_a,
-                       reinterpret_cast<const cx<T>*>(Trec), spins, inv, S);
-    return hipGetLastError();
-}
-
 // ---------------------------------------------------------------------------
 // log psi of n configurations (RBM without visible bias), theta = b + W^T s on
 // the bfloat16 matrix cores with FP32 arithmetic: the +-1 spins are exact in
@@ -1875,7 +1832,5 @@ template hipError_t launch_eval<float>(const RbmDev<float>&, const OpDev&, int, 
 template hipError_t launch_eval<double>(const RbmDev<double>&, const OpDev&, int, int64_t, const uint64_t*, uint64_t, const Records&, bool, size_t, int, hipStream_t);
 template hipError_t launch_ok_reduce<float>(int64_t, int, int, const void*, const uint64_t*, const cx<double>*, int64_t, cx<double>*, hipStream_t);
 template hipError_t launch_ok_reduce<double>(int64_t, int, int, const void*, const uint64_t*, const cx<double>*, int64_t, cx<double>*, hipStream_t);
-template hipError_t launch_s_matrix_ref<float>(int64_t, int, int, int, const void*, const uint64_t*, double, cx<double>*, hipStream_t);
-template hipError_t launch_s_matrix_ref<double>(int64_t, int, int, int, const void*, const uint64_t*, double, cx<double>*, hipStream_t);
 
 }  // namespace rbmhip

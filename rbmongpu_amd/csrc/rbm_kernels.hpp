@@ -159,9 +159,6 @@ hipError_t launch_axis_contract(int64_t n, int N, const uint64_t* configs, uint6
 hipError_t launch_scalar_partials(int64_t n, const double* sc, int nblocks, double* partials, hipStream_t stream);
 hipError_t launch_lse_partials(int64_t n, const cx<double>* lp, double log_prefactor, int nblocks, double* partials,
                                hipStream_t stream);
-template <typename T>
-hipError_t launch_s_matrix_ref(int64_t n, int N, int M, int has_a, const void* Trec, const uint64_t* spins, double inv,
-                               cx<double>* S, hipStream_t stream);
 hipError_t launch_activation(int64_t n, const cx<double>* z, cx<double>* out, int deriv, hipStream_t stream);
 // Centred S-matrix pieces: realified, weighted, centred O rows of samples
 // [s0, s0 + nb) (rows nb .. nbp zero; columns [Re (P) | Im (P) | 0 .. ld2)),
