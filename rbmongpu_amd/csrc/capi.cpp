@@ -61,8 +61,17 @@ struct ApiRange {
     ApiRange& operator=(const ApiRange&) = delete;
 };
 
+// The context that the calling thread's current call holds (set by ctx()),
+// released when the call ends.
+struct Ctx;
+thread_local Ctx* g_held = nullptr;
+struct CallLock {
+    ~CallLock();
+};
+
 template <class F>
 int guard(F&& f) {
+    CallLock lock;
     try {
         f();
         return RBMHIP_OK;
@@ -103,6 +112,9 @@ struct DevBuf {
 };
 
 struct Ctx {
+    // held by a compute call from ctx() to its end (CallLock): the stream, the
+    // workspaces and the staging buffer serve one call at a time
+    std::mutex busy;
     int device = 0;
     hipStream_t stream = nullptr;
     size_t max_lds = 65536;
@@ -147,8 +159,49 @@ struct Ctx {
         pending.push_back(p);
     }
 
+    // Pinned staging for copies between the host's arrays and the device.  A
+    // copy from or to pageable memory goes through the runtime's own staging
+    // and blocks (10-20 us each, and an exact gradient of 10 spins makes 8); a
+    // copy of at most STAGE_COPY bytes goes through this buffer instead and is
+    // ordered by the stream alone: h2d takes its bytes at once, d2h delivers
+    // them at the next sync().  The buffer is used from its start again after
+    // each sync(); when it is full, and for larger copies, the runtime's path
+    // is taken.  Allocated on first use and kept, one per device.
+    static constexpr size_t STAGE_BYTES = 8u << 20, STAGE_COPY = 4u << 20;
+    unsigned char* stage = nullptr;
+    size_t stage_used = 0;
+    struct Delivery {
+        void* dst;
+        const void* src;
+        size_t bytes;
+    };
+    std::vector<Delivery> deliveries;
+
+    void* stage_take(size_t bytes) {
+        if (bytes == 0 || bytes > STAGE_COPY) return nullptr;
+        if (!stage && hipHostMalloc(reinterpret_cast<void**>(&stage), STAGE_BYTES, hipHostMallocDefault) != hipSuccess) {
+            (void)hipGetLastError();
+            stage = nullptr;
+            return nullptr;
+        }
+        const size_t at = (stage_used + 255) & ~(size_t)255;
+        if (at + bytes > STAGE_BYTES) return nullptr;
+        stage_used = at + bytes;
+        return stage + at;
+    }
+    // Forgets what a call that failed half-way left in the staging buffer.
+    void stage_reset() {
+        if (stage_used == 0) return;
+        (void)hipStreamSynchronize(stream);
+        deliveries.clear();
+        stage_used = 0;
+    }
+
     void sync() {
         RBM_HIPCHK(hipStreamSynchronize(stream));
+        for (const Delivery& d : deliveries) std::memcpy(d.dst, d.src, d.bytes);
+        deliveries.clear();
+        stage_used = 0;
         for (auto& p : pending) {
             float ms = 0.f;
             RBM_HIPCHK(hipEventElapsedTime(&ms, p.a, p.b));
@@ -162,18 +215,48 @@ struct Ctx {
     }
 
     void d2h(void* dst, const void* src, size_t bytes) {
+        if (void* s = stage_take(bytes)) {
+            RBM_HIPCHK(hipMemcpyAsync(s, src, bytes, hipMemcpyDeviceToHost, stream));
+            deliveries.push_back({dst, s, bytes});
+            return;
+        }
         RBM_HIPCHK(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, stream));
     }
     void h2d(void* dst, const void* src, size_t bytes) {
+        if (void* s = stage_take(bytes)) {
+            std::memcpy(s, src, bytes);
+            RBM_HIPCHK(hipMemcpyAsync(dst, s, bytes, hipMemcpyHostToDevice, stream));
+            return;
+        }
         RBM_HIPCHK(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, stream));
     }
+    // n values of V at dst, formed by fill(V*)
+    template <class V, class F>
+    void upload(void* dst, size_t n, F&& fill) {
+        if (n == 0) return;
+        if (void* s = stage_take(n * sizeof(V))) {
+            fill(reinterpret_cast<V*>(s));
+            RBM_HIPCHK(hipMemcpyAsync(dst, s, n * sizeof(V), hipMemcpyHostToDevice, stream));
+            return;
+        }
+        std::vector<V> h(n);
+        fill(h.data());
+        RBM_HIPCHK(hipMemcpyAsync(dst, h.data(), n * sizeof(V), hipMemcpyHostToDevice, stream));
+        RBM_HIPCHK(hipStreamSynchronize(stream));
+    }
 };
+
+CallLock::~CallLock() {
+    if (!g_held) return;
+    g_held->busy.unlock();
+    g_held = nullptr;
+}
 
 static std::mutex g_mu;
 static int g_device = 0;
 static std::map<int, std::unique_ptr<Ctx>> g_ctx;
 
-static Ctx& ctx() {
+static Ctx& find_ctx() {
     std::lock_guard<std::mutex> lk(g_mu);
     int count = 0;
     if (hipGetDeviceCount(&count) != hipSuccess || count <= 0)
@@ -198,6 +281,19 @@ static Ctx& ctx() {
     Ctx& ref = *c;
     g_ctx[g_device] = std::move(c);
     return ref;
+}
+
+// The current device's context, held for the calling thread until its call ends.
+static Ctx& ctx() {
+    Ctx& c = find_ctx();
+    if (g_held != &c) {
+        if (g_held) g_held->busy.unlock();
+        g_held = nullptr;
+        c.busy.lock();
+        g_held = &c;
+        c.stage_reset();
+    }
+    return c;
 }
 
 }  // namespace rbmhip
@@ -253,11 +349,10 @@ struct rbmhip_psi {
 
 template <typename T>
 static void upload_cx(Ctx& c, DevBuf& buf, const std::vector<cd>& v) {
-    std::vector<cx<T>> h(v.size());
-    for (size_t i = 0; i < v.size(); i++) h[i] = mk<T>((T)v[i].real(), (T)v[i].imag());
-    buf.ensure(sizeof(cx<T>) * h.size());
-    if (!h.empty()) RBM_HIPCHK(hipMemcpy(buf.p, h.data(), sizeof(cx<T>) * h.size(), hipMemcpyHostToDevice));
-    (void)c;
+    buf.ensure(sizeof(cx<T>) * v.size());
+    c.upload<cx<T>>(buf.p, v.size(), [&](cx<T>* h) {
+        for (size_t i = 0; i < v.size(); i++) h[i] = mk<T>((T)v[i].real(), (T)v[i].imag());
+    });
 }
 
 template <typename T>
@@ -266,12 +361,18 @@ static RbmDev<T> rbm_dev(Ctx& c, rbmhip_psi* psi) {
     const int ld = rbm_padded_width(psi->M);
     if (d.version != psi->version || d.precision != psi->precision) {
         // W and b padded with zero columns to ld hidden units
-        std::vector<cd> Wp((size_t)psi->N * ld, cd(0, 0)), bp((size_t)ld, cd(0, 0));
-        for (int i = 0; i < psi->N; i++)
-            for (int j = 0; j < psi->M; j++) Wp[(size_t)i * ld + j] = psi->W[(size_t)i * psi->M + j];
-        for (int j = 0; j < psi->M; j++) bp[j] = psi->b[j];
-        upload_cx<T>(c, d.W, Wp);
-        upload_cx<T>(c, d.b, bp);
+        const int N = psi->N, M = psi->M;
+        auto rows = [&](cx<T>* h, const cd* src, int n) {
+            for (int i = 0; i < n; i++)
+                for (int j = 0; j < ld; j++, h++) {
+                    const cd z = j < M ? src[(size_t)i * M + j] : cd(0, 0);
+                    *h = mk<T>((T)z.real(), (T)z.imag());
+                }
+        };
+        d.W.ensure(sizeof(cx<T>) * (size_t)N * ld);
+        d.b.ensure(sizeof(cx<T>) * (size_t)ld);
+        c.upload<cx<T>>(d.W.p, (size_t)N * ld, [&](cx<T>* h) { rows(h, psi->W.data(), N); });
+        c.upload<cx<T>>(d.b.p, (size_t)ld, [&](cx<T>* h) { rows(h, psi->b.data(), 1); });
         if (psi->has_a) upload_cx<T>(c, d.a, psi->a);
         d.version = psi->version;
         d.precision = psi->precision;
@@ -1475,7 +1576,7 @@ struct ScratchTables {
                     "the model and operator need more than the " + std::to_string(NOALLOC_TABLE_BYTES >> 20) +
                         " MiB of table space of the allocation-free entry point");
         used = at + bytes;
-        if (bytes) c.h2d(base + at, v.data(), bytes);
+        if (bytes) RBM_HIPCHK(hipMemcpyAsync(base + at, v.data(), bytes, hipMemcpyHostToDevice, c.stream));
         return base + at;
     }
 };
@@ -1520,11 +1621,11 @@ static void local_energy_noalloc_impl(Ctx& c, rbmhip_psi* psi, rbmhip_op* op, co
     uint64_t* ds = reinterpret_cast<uint64_t*>(base + NOALLOC_TABLE_BYTES);
     cx<double>* lp = reinterpret_cast<cx<double>*>(base + NOALLOC_TABLE_BYTES + region);
     cx<double>* el = reinterpret_cast<cx<double>*>(base + NOALLOC_TABLE_BYTES + 2 * region);
-    c.h2d(ds, spins, (size_t)n * 2 * sizeof(uint64_t));
+    RBM_HIPCHK(hipMemcpyAsync(ds, spins, (size_t)n * 2 * sizeof(uint64_t), hipMemcpyHostToDevice, c.stream));
     const size_t lds = rbm_w_bytes<T>(psi);
     Records rec{nullptr, lp, el, nullptr};
     RBM_HIPCHK(launch_eval<T>(md, od, 1, n, ds, 0, rec, lds <= c.max_lds, lds, c.num_cus * 8, c.stream));
-    c.d2h(out, el, (size_t)n * sizeof(cx<double>));
+    RBM_HIPCHK(hipMemcpyAsync(out, el, (size_t)n * sizeof(cx<double>), hipMemcpyDeviceToHost, c.stream));
     // the host staging vectors above stay alive until the copies are done
     RBM_HIPCHK(hipStreamSynchronize(c.stream));
 }
@@ -2647,20 +2748,17 @@ static int hs_distance_impl(rbmhip_psi* psi, rbmhip_psi* psi_prime, rbmhip_op* o
                 using T = decltype(tag);
                 const RbmDev<T> md = rbm_dev<T>(c, psi);
                 const int Nn = psi->N, Mm = psi->M, ld = md.ld;
-                std::vector<cx<T>> hw((size_t)Nn * ld, mk<T>(0, 0)), hb((size_t)ld, mk<T>(0, 0));
-                for (int i = 0; i < Nn; i++)
-                    for (int j = 0; j < Mm; j++) {
-                        const cd d = psi_prime->W[(size_t)i * Mm + j] - psi->W[(size_t)i * Mm + j];
-                        hw[(size_t)i * ld + j] = mk<T>((T)d.real(), (T)d.imag());
-                    }
-                for (int j = 0; j < Mm; j++) {
-                    const cd d = psi_prime->b[j] - psi->b[j];
-                    hb[j] = mk<T>((T)d.real(), (T)d.imag());
-                }
-                void* dW = c.buf("hs_dW", hw.size() * sizeof(cx<T>));
-                void* db = c.buf("hs_db", hb.size() * sizeof(cx<T>));
-                RBM_HIPCHK(hipMemcpy(dW, hw.data(), hw.size() * sizeof(cx<T>), hipMemcpyHostToDevice));
-                RBM_HIPCHK(hipMemcpy(db, hb.data(), hb.size() * sizeof(cx<T>), hipMemcpyHostToDevice));
+                void* dW = c.buf("hs_dW", (size_t)Nn * ld * sizeof(cx<T>));
+                void* db = c.buf("hs_db", (size_t)ld * sizeof(cx<T>));
+                auto rows = [&](cx<T>* h, const cd* x, const cd* y, int n) {
+                    for (int i = 0; i < n; i++)
+                        for (int j = 0; j < ld; j++, h++) {
+                            const cd d = j < Mm ? x[(size_t)i * Mm + j] - y[(size_t)i * Mm + j] : cd(0, 0);
+                            *h = mk<T>((T)d.real(), (T)d.imag());
+                        }
+                };
+                c.upload<cx<T>>(dW, (size_t)Nn * ld, [&](cx<T>* h) { rows(h, psi_prime->W.data(), psi->W.data(), Nn); });
+                c.upload<cx<T>>(db, (size_t)ld, [&](cx<T>* h) { rows(h, psi_prime->b.data(), psi->b.data(), 1); });
                 cx<double>* da = nullptr;
                 if (psi->has_a || psi_prime->has_a) {
                     std::vector<cx<double>> ha((size_t)Nn);
@@ -2669,7 +2767,8 @@ static int hs_distance_impl(rbmhip_psi* psi, rbmhip_psi* psi_prime, rbmhip_op* o
                         ha[i] = mk(d.real(), d.imag());
                     }
                     da = reinterpret_cast<cx<double>*>(c.buf("hs_da", ha.size() * sizeof(cx<double>)));
-                    RBM_HIPCHK(hipMemcpy(da, ha.data(), ha.size() * sizeof(cx<double>), hipMemcpyHostToDevice));
+                    c.h2d(da, ha.data(), ha.size() * sizeof(cx<double>));
+                    c.sync();
                 }
                 c.launch("hs_log_ratio", [&] {
                     return launch_rbm_log_ratio<T>(md, dW, db, da, s.n, configs, 0, s.lp, lp2, c.num_cus * 8, c.stream);
