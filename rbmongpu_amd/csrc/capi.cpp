@@ -843,35 +843,27 @@ static MadeInf made_inf(Ctx& c, rbmhip_made* md) {
     return mi;
 }
 
-// Forward and backward pass of loss = -(1/B) sum_s log q(x_s) over B rows of X
-// (Bp = padded rows).  Leaves the gradient in md->grad and the per-tile log-q
-// partials in `partials`.
-// Launch extents of one training step (gather, forward and backward GEMMs,
-// bias column sums, Adam): for every buffer a kernel of the step touches, the
-// largest element offset its launch arguments allow, against the size the
-// step allocates for that buffer.  Pure host arithmetic, run before every
-// training call and by rbmhip_made_check_launches without a GPU.
-static int made_splits(int Bp) {
-    int splits = 1;
-    while (splits < 64 && Bp % (16 * splits * 2) == 0 && Bp / (splits * 2) >= 64) splits *= 2;
-    return splits;
-}
-
+// Launch extents of one training step (pass, weight gradients, update): for
+// every buffer a kernel of the step touches, the largest element offset its
+// launch arguments allow, against the size the step allocates for that buffer.
+// Pure host arithmetic, run before every training call and by
+// rbmhip_made_check_launches without a GPU.
 struct MadeStepPlan {
-    int N, H, Np, Hp, B, Bp, splits, tiles;
+    MadeShape s;
+    int B, Bp, tiles, splits;
     int64_t n, off_b1, off_W2, off_b2, padded;
 };
 
 static MadeStepPlan made_plan(int N, int H, int64_t n, int batch) {
     MadeStepPlan p{};
-    p.N = N; p.H = H; p.Np = made_pad(N); p.Hp = made_pad(H);
+    p.s.N = N; p.s.H = H; p.s.Np = made_pad(N); p.s.Hp = made_pad(H);
     p.B = batch; p.Bp = made_pad(batch); p.n = n;
-    p.splits = made_splits(p.Bp);
-    p.tiles = (p.Np / 64) * (p.Bp / 64);
-    p.off_b1 = (int64_t)p.Hp * p.Np;
-    p.off_W2 = p.off_b1 + p.Hp;
-    p.off_b2 = p.off_W2 + (int64_t)p.Np * p.Hp;
-    p.padded = p.off_b2 + p.Np;
+    p.tiles = p.Bp / 16;
+    p.splits = made_wgrad_splits(p.s, p.tiles);
+    p.off_b1 = (int64_t)p.s.Hp * p.s.Np;
+    p.off_W2 = p.off_b1 + p.s.Hp;
+    p.off_b2 = p.off_W2 + (int64_t)p.s.Np * p.s.Hp;
+    p.padded = p.off_b2 + p.s.Np;
     return p;
 }
 
@@ -881,84 +873,55 @@ static void made_check_extents(const MadeStepPlan& p) {
             throw Error(RBMHIP_ERR_ARG, std::string("launch extent exceeds its buffer: ") + what + " touches " +
                                             std::to_string(touched) + " elements of " + std::to_string(size));
     };
-    // k_gemm<EPI> over an M x N output, K deep, split `splits` ways: A at
-    // (m sam + k sak), B at (k sbk + n sbn), C at (z M ldc + m ldc + n)
-    auto gemm = [&](const char* what, int M, int N, int K, int64_t sam, int64_t sak, int64_t a_size, int64_t sbk,
-                    int64_t sbn, int64_t b_size, int64_t ldc, int64_t c_size, int splits) {
-        RBM_REQUIRE(M % 64 == 0 && N % 64 == 0 && K % (16 * splits) == 0, std::string("GEMM shape: ") + what);
-        need((M - 1) * sam + (K - 1) * sak + 1, a_size, what);
-        need((K - 1) * sbk + (N - 1) * sbn + 1, b_size, what);
-        need((int64_t)(splits - 1) * M * ldc + (M - 1) * ldc + N, c_size, what);
-    };
-    const int64_t X = (int64_t)p.Bp * p.Np, HB = (int64_t)p.Bp * p.Hp, W = (int64_t)p.Np * p.Hp;
-    // minibatch indices and the gather of Bp rows of Np inputs
-    need(p.B, p.B, "batch indices");
-    need(X, X, "gathered inputs");
+    const int64_t Np = p.s.Np, Hp = p.s.Hp, Bp = p.Bp, W = Np * Hp;
+    RBM_REQUIRE((Np == 64 || Np == 128) && Hp >= 64 && Hp <= 512 && Hp % 64 == 0, "padded shape of the training pass");
+    RBM_REQUIRE(p.B <= p.Bp && p.tiles * 16 == p.Bp, "sample tiles");
+    // pass: tile blk of 16 samples
+    const int64_t last = 15;
     need(2 * p.n, 2 * p.n, "spin words");
-    // a = X W1^T + b1 (W1: Hp x Np at 0, b1 at off_b1), h = relu(a)
-    gemm("a = X W1^T", p.Bp, p.Hp, p.Np, p.Np, 1, X, 1, p.Np, p.off_b1, p.Hp, HB, 1);
-    need(p.off_b1 + p.Hp, p.padded, "b1");
-    // l = h W2^T + b2 (W2: Np x Hp at off_W2), loss partials per tile
-    gemm("l = h W2^T", p.Bp, p.Np, p.Hp, p.Hp, 1, HB, 1, p.Hp, W, p.Np, X, 1);
-    need(p.off_W2 + W, p.padded, "W2");
-    need(p.off_b2 + p.Np, p.padded, "b2");
-    need((p.Bp / 64) * (p.Np / 64), p.tiles, "loss partials");
-    // dW2 = dl^T h split over K, reduced into G at off_W2
-    gemm("dW2 = dl^T h", p.Np, p.Hp, p.Bp, 1, p.Np, X, p.Hp, 1, HB, p.Hp, (int64_t)p.splits * W, p.splits);
-    // dh = (dl W2) relu'(a)
-    gemm("dh = dl W2", p.Bp, p.Hp, p.Np, p.Np, 1, X, p.Hp, 1, W, p.Hp, HB, 1);
-    // dW1 = dh^T X split over K, reduced into G at 0
-    gemm("dW1 = dh^T X", p.Hp, p.Np, p.Bp, 1, p.Hp, HB, p.Np, 1, X, p.Np, (int64_t)p.splits * W, p.splits);
-    // bias gradients: column sums of dh (Hp columns) and dl (Np columns)
-    need((int64_t)COLSUM_SLICES * std::max(p.Hp, p.Np), (int64_t)COLSUM_SLICES * std::max(p.Hp, p.Np), "column-sum slices");
-    need(p.off_b1 + p.Hp, p.padded, "db1");
-    need(p.off_b2 + p.Np, p.padded, "db2");
+    need(((Hp / 16 - 1) * (Np / 16) + Np / 16 - 1) * 256 + 4 * 63 + 4, W, "W1 and W2 transposed, packed");
+    need(((Np / 16 - 1) * (Hp / 16) + Hp / 16 - 1) * 256 + 4 * 63 + 4, W, "W2, packed");
+    need(p.off_b1 + Hp, p.off_W2, "b1");
+    need(p.off_b2 + Np, p.padded, "b2");
+    need((p.tiles - 1) * Hp * 16 + 256 * (Hp / 16 - 1) + 16 * 3 + 64 * 3 + last + 1, Hp * Bp, "hidden activations");
+    need((p.tiles - 1) * Np * 16 + 256 * (Np / 16 - 1) + 16 * 3 + 64 * 3 + last + 1, Np * Bp, "logit derivatives");
+    need((p.tiles - 1) * Np + Np, p.tiles * Np, "input bits");
+    need((p.tiles - 1) * (Hp + Np) + Hp + Np, p.tiles * (Hp + Np), "bias sums");
+    // weight gradients: 64 x 64 blocks, sample tiles z, z + splits, ...
+    RBM_REQUIRE(p.splits >= 1 && p.splits <= p.tiles, "an empty split of the weight gradients");
+    need(((p.tiles - 1) * Hp + Hp - 64 + 48 + last) * 16 + 4 * 3 + 4, Hp * Bp, "rows of the weight gradients");
+    need((int64_t)(p.splits - 1) * p.padded + p.off_W2 + W, (int64_t)p.splits * p.padded, "weight-gradient partials");
 }
 
-static void made_forward_backward(Ctx& c, rbmhip_made* md, int B, int Bp, const float* X, double* partials) {
-    const int N = md->s.N, H = md->s.H, Np = md->s.Np, Hp = md->s.Hp;
-    float* Apre = reinterpret_cast<float*>(c.buf("made_apre", (size_t)Bp * Hp * sizeof(float)));
-    float* Hh = reinterpret_cast<float*>(c.buf("made_h", (size_t)Bp * Hp * sizeof(float)));
-    float* dL = reinterpret_cast<float*>(c.buf("made_dl", (size_t)Bp * Np * sizeof(float)));
-    float* dH = reinterpret_cast<float*>(c.buf("made_dh", (size_t)Bp * Hp * sizeof(float)));
+// The step's buffers and constant arguments.
+static MadeStep made_step_args(Ctx& c, rbmhip_made* md, const MadeStepPlan& p, const uint64_t* spins, double* loss_part) {
+    const int64_t Np = p.s.Np, Hp = p.s.Hp;
+    MadeStep a{};
+    a.N = p.s.N; a.B = p.B; a.Bp = p.Bp; a.n = p.n;
+    a.spins = spins;
     const float* P = md->P();
-    float* G = md->G();
-    const float* W1 = P;
-    const float* W2 = P + md->off_W2;
-    GemmEpiArgs e{};
-    // a = X W1^T + b1, h = relu(a)
-    e.bias = P + md->off_b1; e.C2 = Hh;
-    c.launch("made_gemm", [&] { return launch_gemm(EPI_BIAS_RELU, Bp, Hp, Np, X, Np, 1, W1, 1, Np, Apre, Hp, e, c.stream); });
-    // l = h W2^T + b2 -> dl = (sigmoid(l) - x) / B
-    e = GemmEpiArgs{};
-    e.bias = P + md->off_b2; e.aux = X; e.ld_aux = Np; e.n_live = N; e.m_live = B; e.inv_batch = 1.0f / (float)B;
-    e.partials = partials;
-    c.launch("made_gemm", [&] { return launch_gemm(EPI_LOGITS, Bp, Np, Hp, Hh, Hp, 1, W2, 1, Hp, dL, Np, e, c.stream); });
-    // weight gradients: small outputs with the batch as K, split over workgroups
-    const int splits = made_splits(Bp);
-    float* splitk = reinterpret_cast<float*>(c.buf("made_splitk", (size_t)splits * Np * Hp * sizeof(float)));
-    // dW2 = dl^T h (masked)
-    e = GemmEpiArgs{};
-    e.m_live = N; e.n_live = H;
-    c.launch("made_gemm", [&] {
-        return launch_gemm_splitk(EPI_MASK_W2, Np, Hp, Bp, dL, 1, Np, Hh, Hp, 1, G + md->off_W2, Hp, e, splits, splitk, c.stream);
-    });
-    // dh = (dl W2) * [a > 0]
-    e = GemmEpiArgs{};
-    e.aux = Apre; e.ld_aux = Hp;
-    c.launch("made_gemm", [&] { return launch_gemm(EPI_RELU_GRAD, Bp, Hp, Np, dL, Np, 1, W2, Hp, 1, dH, Hp, e, c.stream); });
-    // dW1 = dh^T X (masked)
-    e = GemmEpiArgs{};
-    e.m_live = H; e.n_live = N;
-    c.launch("made_gemm", [&] {
-        return launch_gemm_splitk(EPI_MASK_W1, Hp, Np, Bp, dH, 1, Hp, X, Np, 1, G, Np, e, splits, splitk, c.stream);
-    });
-    float* part = reinterpret_cast<float*>(c.buf("made_colsum", (size_t)COLSUM_SLICES * (Hp > Np ? Hp : Np) * sizeof(float)));
-    c.launch("made_colsum", [&] { return launch_colsum(Bp, Hp, H, dH, G + md->off_b1, part, c.stream); });
-    c.launch("made_colsum", [&] { return launch_colsum(Bp, Np, N, dL, G + md->off_b2, part, c.stream); });
+    float* packed = reinterpret_cast<float*>(c.buf("made_packed", (size_t)(3 * Np * Hp) * sizeof(float)));
+    a.W1 = packed; a.b1 = P + p.off_b1; a.W2 = packed + Np * Hp; a.b2 = P + p.off_b2; a.W2t = packed + 2 * Np * Hp;
+    a.inv_batch = 1.0f / (float)p.B;
+    a.hT = reinterpret_cast<float*>(c.buf("made_h", (size_t)(Hp * p.Bp) * sizeof(float)));
+    a.daT = reinterpret_cast<float*>(c.buf("made_da", (size_t)(Hp * p.Bp) * sizeof(float)));
+    a.dlT = reinterpret_cast<float*>(c.buf("made_dl", (size_t)(Np * p.Bp) * sizeof(float)));
+    a.xbits = reinterpret_cast<uint16_t*>(c.buf("made_x", (size_t)(p.tiles * Np) * sizeof(uint16_t)));
+    a.bias_part = reinterpret_cast<float*>(c.buf("made_bias", (size_t)(p.tiles * (Hp + Np)) * sizeof(float)));
+    a.loss_part = loss_part;
+    a.wgrad_part = reinterpret_cast<float*>(c.buf("made_wgrad", (size_t)(p.splits * p.padded) * sizeof(float)));
+    a.off_b1 = p.off_b1; a.off_W2 = p.off_W2; a.off_b2 = p.off_b2; a.padded = p.padded;
+    c.launch("made_pack", [&] { return launch_made_pack(p.s, P, P + p.off_W2, packed, c.stream); });
+    return a;
 }
 
-static int made_loss_tiles(const rbmhip_made* md, int Bp) { return (md->s.Np / 64) * (Bp / 64); }
+static void made_step(Ctx& c, const MadeStepPlan& p, const MadeStep& a, const MadeUpdate& u) {
+    c.launch("made_pass", [&] { return launch_made_pass(p.s, a, c.stream); });
+    c.launch("made_wgrad", [&] { return launch_made_wgrad(p.s, a, p.splits, c.stream); });
+    c.launch("made_update", [&] {
+        return launch_made_update(p.s, u, a, p.splits, const_cast<float*>(a.W1), c.stream);
+    });
+}
 
 // ---------------------------------------------------------------------------
 // ensembles
@@ -2992,15 +2955,17 @@ int rbmhip_made_loss_grad(rbmhip_made* made, const uint64_t* spins, int64_t n, d
         RBM_REQUIRE(n <= (1 << 24), "batch too large");
         Ctx& c = ctx();
         made_check_device(c, made);
-        const int B = (int)n, Bp = made_pad(B);
-        made_check_extents(made_plan(made->s.N, made->s.H, n, B));
+        const int B = (int)n;
+        const MadeStepPlan plan = made_plan(made->s.N, made->s.H, n, B);
+        made_check_extents(plan);
         uint64_t* ds = reinterpret_cast<uint64_t*>(c.buf("made_in", (size_t)n * 2 * sizeof(uint64_t)));
         c.h2d(ds, spins, (size_t)n * 2 * sizeof(uint64_t));
-        float* X = reinterpret_cast<float*>(c.buf("made_x", (size_t)Bp * made->s.Np * sizeof(float)));
-        c.launch("made_gather", [&] { return launch_made_gather(Bp, B, made->s.N, made->s.Np, ds, nullptr, X, c.stream); });
-        const int tiles = made_loss_tiles(made, Bp);
+        const int tiles = plan.tiles;
         double* part = reinterpret_cast<double*>(c.buf("made_part", (size_t)tiles * sizeof(double)));
-        made_forward_backward(c, made, B, Bp, X, part);
+        const MadeStep a = made_step_args(c, made, plan, ds, part);
+        MadeUpdate u{};
+        u.grad = made->G();
+        made_step(c, plan, a, u);
         std::vector<double> hp((size_t)tiles);
         std::vector<float> dev((size_t)made->padded);
         c.d2h(hp.data(), part, hp.size() * sizeof(double));
@@ -3025,28 +2990,29 @@ int rbmhip_made_train(rbmhip_made* made, const uint64_t* spins, int64_t n, int s
         Ctx& c = ctx();
         made_check_device(c, made);
         if (steps == 0) return;
-        const int B = batch, Bp = made_pad(B);
-        made_check_extents(made_plan(made->s.N, made->s.H, n, B));
-        const bool full = (int64_t)batch == n;   // the whole sample set, in order, every step
+        const int B = batch;
+        const MadeStepPlan plan = made_plan(made->s.N, made->s.H, n, B);
+        made_check_extents(plan);
         uint64_t* ds = reinterpret_cast<uint64_t*>(c.buf("made_train_in", (size_t)n * 2 * sizeof(uint64_t)));
         c.h2d(ds, spins, (size_t)n * 2 * sizeof(uint64_t));
-        float* X = reinterpret_cast<float*>(c.buf("made_x", (size_t)Bp * made->s.Np * sizeof(float)));
-        int64_t* idx = full ? nullptr : reinterpret_cast<int64_t*>(c.buf("made_idx", (size_t)B * sizeof(int64_t)));
-        const int tiles = made_loss_tiles(made, Bp);
+        const int tiles = plan.tiles;
         double* part = reinterpret_cast<double*>(c.buf("made_train_part", (size_t)steps * tiles * sizeof(double)));
+        MadeStep a = made_step_args(c, made, plan, ds, part);
+        a.draw = (int64_t)batch != n;   // else the whole sample set, in order, every step
+        a.seed_lo = (uint32_t)seed;
+        a.seed_hi = (uint32_t)(seed >> 32);
+        MadeUpdate u{};
+        u.params = made->P();
+        u.m = reinterpret_cast<float*>(made->m.p);
+        u.v = reinterpret_cast<float*>(made->v.p);
+        u.lr = (float)lr; u.beta1 = 0.9f; u.beta2 = 0.999f; u.eps = 1e-8f;
         for (int st = 0; st < steps; st++) {
-            if (!full) {
-                c.launch("made_batch", [&] {
-                    return launch_made_batch_index(B, n, (uint32_t)(made->t + st), (uint32_t)seed, (uint32_t)(seed >> 32), idx, c.stream);
-                });
-            }
-            c.launch("made_gather", [&] { return launch_made_gather(Bp, B, made->s.N, made->s.Np, ds, idx, X, c.stream); });
-            made_forward_backward(c, made, B, Bp, X, part + (size_t)st * tiles);
             const int t = made->t + st + 1;
-            c.launch("made_adam", [&] {
-                return launch_adam(made->padded, made->P(), made->G(), reinterpret_cast<float*>(made->m.p),
-                                   reinterpret_cast<float*>(made->v.p), t, (float)lr, 0.9f, 0.999f, 1e-8f, c.stream);
-            });
+            a.step = (uint32_t)(made->t + st);
+            a.loss_part = part + (size_t)st * tiles;
+            u.c1 = (float)(1.0 / (1.0 - std::pow((double)u.beta1, t)));
+            u.c2 = (float)(1.0 / (1.0 - std::pow((double)u.beta2, t)));
+            made_step(c, plan, a, u);
         }
         made->t += steps;
         made->inf_valid = false;

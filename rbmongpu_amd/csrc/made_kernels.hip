@@ -1,9 +1,6 @@
 // gfx950 kernels of the masked autoregressive proposal (MADE):
-//   k_gemm<EPI>           FP32 MFMA GEMM (v_mfma_f32_16x16x4f32) with fused epilogues
-//                         for the training forward and backward passes
-//   k_made_gather         spin words -> 0/1 input rows
-//   k_made_batch_index    Philox-drawn minibatch indices
-//   k_colsum_part/_finish, k_adam   bias gradients and the Adam update
+//   k_made_pass           forward and backward pass of a training step (FP32 MFMA)
+//   k_made_wgrad, k_made_update   weight gradients, bias sums and Adam
 //   k_made_inf_weights    bfloat16 inference copies of W1 (transposed) and W2
 //   k_made_sample<HPL,S,W1F>  autoregressive sampling / scoring, weights in LDS
 //   k_imh                 independent Metropolis-Hastings over precomputed proposals
@@ -15,245 +12,395 @@ typedef float floatx4 __attribute__((ext_vector_type(4)));
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 
 // ---------------------------------------------------------------------------
-// GEMM.  A 256-thread workgroup computes a 64 x 64 tile of C as 2 x 2 waves of
-// 32 x 32, each 2 x 2 MFMA 16x16x4 tiles; K advances 16 at a time through LDS.
-// MFMA operand layout (16x16x4 f32): lane l supplies A[l % 16][l / 16] and
-// B[l / 16][l % 16]; accumulator element v of lane l is D[4 (l / 16) + v][l % 16].
+// Training.  One step of loss = -(1/B) sum_s log q(x_s) is three launches:
+//   k_made_pass     forward and backward pass of 16 samples per workgroup
+//   k_made_wgrad    weight gradients, split over the batch
+//   k_made_update   sums of the splits, masks, Adam
+// All products are FP32 MFMA (v_mfma_f32_16x16x4f32: lane l supplies
+// A[l % 16][l / 16] and B[l / 16][l % 16], accumulator v of lane l is
+// D[4 (l / 16) + v][l % 16]), with the same FP32 values as a GEMM per product.
+//
+// In k_made_pass the samples are the columns of D, so a lane's four
+// accumulators of one 16-unit tile are four units of one sample: exactly what
+// it supplies as B operands (k = l / 16 of four MFMAs, one per v) to the next
+// layer when the weights of MFMA v are those of units 16 t + 4 (l / 16) + v,
+// which a lane reads as one 16-byte word.  Activations therefore stay in
+// registers from the drawn sample to its back-propagated derivative, and the
+// inputs come straight from the spin bits.  The pass leaves the activations,
+// derivatives and bits that the weight gradients contract, 16 samples of a unit
+// in 64 bytes, units of a tile one after the other, so that there a lane's four
+// samples are one 16-byte word and 16 units 1 KiB in a row.
+//
+// N = 100, H = 256, batch 16 384: a step takes 83 us (pass 48, weight
+// gradients 27, update 8); the three matrix products of the pass alone are 20
+// at the FP32 matrix rate, those of the gradients 14, and the logits' FP32
+// functions and bias sums 18 of vector instructions.  It took 257 as 12
+// launches (index, gather, five tiled GEMMs through LDS at 34 TFLOP/s, column
+// sums, Adam), 86 of them in column sums whose few workgroups ran down the
+// batch one row after the other.
 // ---------------------------------------------------------------------------
-constexpr int GT = 64, GK = 16;
-
 RBM_DI float sigmoidf_acc(float l) { return 1.0f / (1.0f + expf(-l)); }
 RBM_DI float softplusf_acc(float l) { return fmaxf(l, 0.0f) + log1pf(expf(-fabsf(l))); }
 
-template <int EPI>
-__global__ __launch_bounds__(256) void k_gemm(int M, int N, int K, const float* __restrict__ A, long sam, long sak,
-                                              const float* __restrict__ B, long sbk, long sbn, float* __restrict__ C,
-                                              long ldc, GemmEpiArgs e) {
-    __shared__ float As[GK][GT + 4];
-    __shared__ float Bs[GK][GT + 4];
-    __shared__ double red[256];
-    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-    const int m0 = blockIdx.y * GT, n0 = blockIdx.x * GT;
-    if (e.lower_only && n0 > m0) return;   // uniform per workgroup, before any barrier
-    const int wm = (wave >> 1) * 32, wn = (wave & 1) * 32;
-    // split K: workgroup z covers [z K / gridDim.z, (z + 1) K / gridDim.z) and
-    // writes its partial product at C + z M ldc
-    const int kspan = K / gridDim.z;
-    const int kbeg = blockIdx.z * kspan, kend = kbeg + kspan;
-    C += (long)blockIdx.z * M * ldc;
-    floatx4 acc[2][2];
+// Weights in the order in which k_made_pass reads them: 16 x 16 tiles, tile
+// (m, t) of a matrix with T tiles a row at 256 (m T + t), in it lane l's four
+// weights, row l % 16, columns 4 (l / 16) .., at 4 l.  A load is 1 KiB in a row;
+// read from the row-major parameters, 64 bytes of 16 rows a power of two apart,
+// the pass took 55 us instead of 48 (N = 100, H = 256, 16 384 samples).
+RBM_DI int64_t made_packed(int row, int col, int tiles) {
+    return ((int64_t)(row >> 4) * tiles + (col >> 4)) * 256 + ((row & 15) + ((col & 12) << 2)) * 4 + (col & 3);
+}
+
+// w[m] = this lane's weights of tile (m0 + m, t)
+template <int R> RBM_DI void made_tiles(floatx4* w, const float* __restrict__ W, int tiles, int m0, int t) {
+    const float* q = W + (m0 * tiles + t) * 256 + (threadIdx.x & 63) * 4;
 #pragma unroll
-    for (int i = 0; i < 2; i++)
-#pragma unroll
-        for (int j = 0; j < 2; j++) acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
-    for (int k0 = kbeg; k0 < kend; k0 += GK) {
-#pragma unroll
-        for (int r = 0; r < 4; r++) {
-            const int idx = tid + 256 * r;
-            int mm, kk;
-            if (sak == 1) { kk = idx & 15; mm = idx >> 4; } else { mm = idx & 63; kk = idx >> 6; }
-            As[kk][mm] = A[(long)(m0 + mm) * sam + (long)(k0 + kk) * sak];
-            int nn, kb;
-            if (sbn == 1) { nn = idx & 63; kb = idx >> 6; } else { kb = idx & 15; nn = idx >> 4; }
-            Bs[kb][nn] = B[(long)(k0 + kb) * sbk + (long)(n0 + nn) * sbn];
+    for (int m = 0; m < R; m++) w[m] = *reinterpret_cast<const floatx4*>(q + m * tiles * 256);
+}
+
+// A workgroup of 4 wavefronts takes 16 samples; wavefront q has the hidden
+// tiles q HT / 4 ..: its part of a, the part of l these units give (summed over
+// the wavefronts in order through LDS), and its part of da.  The logits' losses
+// and derivatives, a long chain of FP32 functions, are shared out the same way,
+// so four wavefronts a SIMD overlap them with the others' matrix instructions
+// (63 us a pass of 16 384 samples at one wavefront per 16 samples).
+// NT, HT: 16-wide tiles of the padded inputs and hidden units.
+template <int NT, int HT>
+__global__ __launch_bounds__(256, HT <= 16 ? 4 : 2) void k_made_pass(MadeStep p) {
+    constexpr int Np = 16 * NT, Hp = 16 * HT, HW = HT / 4, NW = NT / 4;
+    __shared__ floatx4 lpart[4][NT][64];
+    auto& dls = lpart[0];   // a wavefront replaces the sums it alone has read
+    __shared__ double lsum[4];
+    const int lane = threadIdx.x & 63, g = lane >> 4, r = lane & 15;
+    const int q = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int blk = blockIdx.x, s = 16 * blk + r;
+    const bool valid = s < p.B;
+    uint64_t w0 = 0, w1 = 0;
+    if (valid) {
+        int64_t src = s;
+        if (p.draw) {
+            const u32x4 x = philox(p.step, (uint32_t)s, 0u, 4u, p.seed_lo, p.seed_hi);
+            src = (int64_t)(((double)x.x + 0.5) * (1.0 / 4294967296.0) * (double)p.n);
+            src = src < p.n ? src : p.n - 1;
         }
-        __syncthreads();
-#pragma unroll
-        for (int kq = 0; kq < GK; kq += 4) {
-            float af[2], bf[2];
-#pragma unroll
-            for (int i = 0; i < 2; i++) af[i] = As[kq + (lane >> 4)][wm + 16 * i + (lane & 15)];
-#pragma unroll
-            for (int j = 0; j < 2; j++) bf[j] = Bs[kq + (lane >> 4)][wn + 16 * j + (lane & 15)];
-#pragma unroll
-            for (int i = 0; i < 2; i++)
-#pragma unroll
-                for (int j = 0; j < 2; j++)
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(af[i], bf[j], acc[i][j], 0, 0, 0);
-        }
-        __syncthreads();
+        w0 = p.spins[2 * src];
+        w1 = p.spins[2 * src + 1];
+        mask_words(w0, w1, p.N);
     }
-    double part = 0.0;
+    {   // input bits of the 16 samples by spin, a quarter of the spins each
+        const uint64_t w = (q * (Np / 4) < 64 ? w0 : w1) >> (q * (Np / 4) & 63);
+        uint32_t mine = 0;
+        for (int k = 0; k < Np / 4; k++) {
+            const uint32_t m = (uint32_t)__ballot((int)((w >> k) & 1u)) & 0xFFFFu;
+            mine = lane == k ? m : mine;
+        }
+        if (lane < Np / 4) p.xbits[(int64_t)blk * Np + q * (Np / 4) + lane] = (uint16_t)mine;
+    }
+    // a = W1 x + b1.  Of every product the weights of the next 16 inputs are
+    // requested before the matrix instructions of the present ones.
+    floatx4 a[HW];
 #pragma unroll
-    for (int i = 0; i < 2; i++)
+    for (int m = 0; m < HW; m++) a[m] = *reinterpret_cast<const floatx4*>(p.b1 + 16 * (q * HW + m) + 4 * g);
+    {
+        floatx4 w[2][HW];
+        made_tiles<HW>(w[0], p.W1, NT, q * HW, 0);
 #pragma unroll
-        for (int j = 0; j < 2; j++)
+        for (int t = 0; t < NT; t++) {
+            if (t + 1 < NT) made_tiles<HW>(w[(t + 1) & 1], p.W1, NT, q * HW, t + 1);
+            __builtin_amdgcn_sched_barrier(0);
+            const uint32_t nib = (uint32_t)((t < 4 ? w0 >> (16 * t + 4 * g) : w1 >> (16 * t - 64 + 4 * g)) & 15u);
 #pragma unroll
             for (int v = 0; v < 4; v++) {
-                const int m = m0 + wm + 16 * i + 4 * (lane >> 4) + v;
-                const int n = n0 + wn + 16 * j + (lane & 15);
-                const float x = acc[i][j][v];
-                float* out = C + (long)m * ldc + n;
-                if (EPI == EPI_STORE) {
-                    *out = x;
-                } else if (EPI == EPI_BIAS_RELU) {
-                    const float a = x + e.bias[n];
-                    *out = a;
-                    e.C2[(long)m * ldc + n] = fmaxf(a, 0.0f);
-                } else if (EPI == EPI_LOGITS) {
-                    const float l = x + e.bias[n];
-                    const float xv = e.aux[(long)m * e.ld_aux + n];
-                    const bool live = m < e.m_live && n < e.n_live;
-                    *out = live ? (sigmoidf_acc(l) - xv) * e.inv_batch : 0.0f;
-                    if (live) part += (double)(xv * l) - (double)softplusf_acc(l);
-                } else if (EPI == EPI_MASK_W2) {
-                    const bool ok = m < e.m_live && n < e.n_live && made_degree(n, e.m_live) <= m;
-                    *out = ok ? x : 0.0f;
-                } else if (EPI == EPI_MASK_W1) {
-                    const bool ok = m < e.m_live && n < e.n_live && n < made_degree(m, e.n_live);
-                    *out = ok ? x : 0.0f;
-                } else if (EPI == EPI_RELU_GRAD) {
-                    *out = e.aux[(long)m * e.ld_aux + n] > 0.0f ? x : 0.0f;
-                }
+                const float x = (nib >> v) & 1u ? 1.0f : 0.0f;
+#pragma unroll
+                for (int m = 0; m < HW; m++)
+                    a[m] = __builtin_amdgcn_mfma_f32_16x16x4f32(w[t & 1][m][v], x, a[m], 0, 0, 0);
             }
-    if (EPI == EPI_LOGITS) {
-        red[tid] = part;
-        __syncthreads();
-        if (tid == 0) {
-            double s = 0.0;
-            for (int k = 0; k < 256; k++) s += red[k];
-            e.partials[blockIdx.y * gridDim.x + blockIdx.x] = s;
         }
     }
-}
-
-// Split-K reduction: C = epilogue(sum over the splits of the partial products).
-template <int EPI>
-__global__ __launch_bounds__(256) void k_splitk_reduce(int M, int N, int splits, const float* __restrict__ part,
-                                                       float* __restrict__ C, long ldc, GemmEpiArgs e) {
-    const int64_t total = (int64_t)M * N;
-    for (int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; t < total; t += (int64_t)gridDim.x * blockDim.x) {
-        const int m = (int)(t / N), n = (int)(t % N);
-        float x = 0.0f;
-        for (int z = 0; z < splits; z++) x += part[(int64_t)z * total + t];
-        bool ok = true;
-        if (EPI == EPI_MASK_W2) ok = m < e.m_live && n < e.n_live && made_degree(n, e.m_live) <= m;
-        if (EPI == EPI_MASK_W1) ok = m < e.m_live && n < e.n_live && n < made_degree(m, e.n_live);
-        C[(long)m * ldc + n] = ok ? x : 0.0f;
-    }
-}
-
-hipError_t launch_gemm_splitk(int epi, int M, int N, int K, const float* A, long sam, long sak, const float* B,
-                              long sbk, long sbn, float* C, long ldc, const GemmEpiArgs& e, int splits, float* scratch,
-                              hipStream_t stream) {
-    if (M % GT || N % GT || M <= 0 || N <= 0 || K <= 0 || splits < 1 || K % (GK * splits)) return hipErrorInvalidValue;
-    hipLaunchKernelGGL((k_gemm<EPI_STORE>), dim3(N / GT, M / GT, splits), dim3(256), 0, stream, M, N, K, A, sam, sak, B,
-                       sbk, sbn, scratch, (long)N, e);
-    hipError_t err = hipGetLastError();
-    if (err != hipSuccess) return err;
-    const int64_t total = (int64_t)M * N;
-    const unsigned blocks = (unsigned)((total + 255) / 256 < 2048 ? (total + 255) / 256 : 2048);
-    switch (epi) {
-        case EPI_STORE: hipLaunchKernelGGL((k_splitk_reduce<EPI_STORE>), dim3(blocks), dim3(256), 0, stream, M, N, splits, scratch, C, ldc, e); break;
-        case EPI_MASK_W1: hipLaunchKernelGGL((k_splitk_reduce<EPI_MASK_W1>), dim3(blocks), dim3(256), 0, stream, M, N, splits, scratch, C, ldc, e); break;
-        case EPI_MASK_W2: hipLaunchKernelGGL((k_splitk_reduce<EPI_MASK_W2>), dim3(blocks), dim3(256), 0, stream, M, N, splits, scratch, C, ldc, e); break;
-        default: return hipErrorInvalidValue;
-    }
-    return hipGetLastError();
-}
-
-hipError_t launch_gemm(int epi, int M, int N, int K, const float* A, long sam, long sak, const float* B, long sbk,
-                       long sbn, float* C, long ldc, const GemmEpiArgs& e, hipStream_t stream) {
-    if (M % GT || N % GT || K % GK || M <= 0 || N <= 0 || K <= 0) return hipErrorInvalidValue;
-    const dim3 grid(N / GT, M / GT), block(256);
-#define RBM_GEMM_CASE(E) \
-    case E: hipLaunchKernelGGL((k_gemm<E>), grid, block, 0, stream, M, N, K, A, sam, sak, B, sbk, sbn, C, ldc, e); break;
-    switch (epi) {
-        RBM_GEMM_CASE(EPI_STORE)
-        RBM_GEMM_CASE(EPI_BIAS_RELU)
-        RBM_GEMM_CASE(EPI_LOGITS)
-        RBM_GEMM_CASE(EPI_MASK_W2)
-        RBM_GEMM_CASE(EPI_MASK_W1)
-        RBM_GEMM_CASE(EPI_RELU_GRAD)
-        default: return hipErrorInvalidValue;
-    }
-#undef RBM_GEMM_CASE
-    return hipGetLastError();
-}
-
-// ---------------------------------------------------------------------------
-// Training helpers
-// ---------------------------------------------------------------------------
-__global__ __launch_bounds__(256) void k_made_gather(int64_t rows, int n_live, int N, int Np,
-                                                     const uint64_t* __restrict__ spins,
-                                                     const int64_t* __restrict__ idx, float* __restrict__ X) {
-    const int64_t total = rows * Np;
-    for (int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; t < total; t += (int64_t)gridDim.x * blockDim.x) {
-        const int64_t s = t / Np;
-        const int i = (int)(t - s * Np);
-        float v = 0.0f;
-        if (s < n_live && i < N) {
-            const int64_t src = idx ? idx[s] : s;
-            v = (float)bit_of(spins[2 * src], spins[2 * src + 1], i);
+    // l = W2 relu(a) + b2
+    {
+        floatx4 l[NT];
+#pragma unroll
+        for (int m = 0; m < NT; m++) l[m] = floatx4{0.f, 0.f, 0.f, 0.f};
+        float* hT = p.hT + ((int64_t)blk * Hp + 16 * q * HW) * 16 + 64 * g + r;
+        floatx4 w[2][4];
+        made_tiles<4>(w[0], p.W2, HT, 0, q * HW);
+#pragma unroll
+        for (int k = 0; k < HW * NW; k++) {   // four output tiles of one hidden tile
+            const int t = k / NW, m0 = 4 * (k % NW);
+            if (k + 1 < HW * NW) made_tiles<4>(w[(k + 1) & 1], p.W2, HT, 4 * ((k + 1) % NW), q * HW + (k + 1) / NW);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int v = 0; v < 4; v++) {
+                const float h = fmaxf(a[t][v], 0.0f);
+                if (m0 == 0) hT[256 * t + 16 * v] = h;
+#pragma unroll
+                for (int m = 0; m < 4; m++)
+                    l[m0 + m] = __builtin_amdgcn_mfma_f32_16x16x4f32(w[k & 1][m][v], h, l[m0 + m], 0, 0, 0);
+            }
         }
-        X[t] = v;
+#pragma unroll
+        for (int m = 0; m < NT; m++) lpart[q][m][lane] = l[m];
     }
-}
-
-hipError_t launch_made_gather(int64_t rows, int n_live, int N, int Np, const uint64_t* spins, const int64_t* idx,
-                              float* X, hipStream_t stream) {
-    const int64_t total = rows * Np;
-    int64_t blocks = (total + 255) / 256;
-    if (blocks > 4096) blocks = 4096;
-    hipLaunchKernelGGL(k_made_gather, dim3((unsigned)blocks), dim3(256), 0, stream, rows, n_live, N, Np, spins, idx, X);
-    return hipGetLastError();
-}
-
-__global__ __launch_bounds__(256) void k_made_batch_index(int B, int64_t n, uint32_t step, uint32_t seed_lo,
-                                                          uint32_t seed_hi, int64_t* __restrict__ idx) {
-    const int s = blockIdx.x * blockDim.x + threadIdx.x;
-    if (s >= B) return;
-    const u32x4 r = philox(step, (uint32_t)s, 0u, 4u, seed_lo, seed_hi);
-    const double u = ((double)r.x + 0.5) * (1.0 / 4294967296.0);
-    int64_t k = (int64_t)(u * (double)n);
-    idx[s] = k < n ? k : n - 1;
-}
-
-hipError_t launch_made_batch_index(int B, int64_t n, uint32_t step, uint32_t seed_lo, uint32_t seed_hi, int64_t* idx,
-                                   hipStream_t stream) {
-    hipLaunchKernelGGL(k_made_batch_index, dim3((B + 255) / 256), dim3(256), 0, stream, B, n, step, seed_lo, seed_hi,
-                       idx);
-    return hipGetLastError();
-}
-
-// Column sums of the rows x cols matrix G (the bias gradients: sums over the
-// batch), columns >= n_live zero.  Two deterministic stages: the 256-thread
-// workgroup (x, y) owns columns [64 x, 64 x + 64) of row slice y (rows
-// [y R, (y + 1) R), R = ceil(rows / COLSUM_SLICES)); its 4 row groups of 64
-// threads stride over the slice with coalesced 64-wide reads and are added in
-// a fixed order into part[y][c]; k_colsum_finish then adds the slices in
-// order.  part holds COLSUM_SLICES x cols.
-__global__ __launch_bounds__(256) void k_colsum_part(int rows, int cols, int n_live, const float* __restrict__ G,
-                                                     float* __restrict__ part) {
-    __shared__ float red[4][64];
-    const int cl = threadIdx.x & 63, grp = threadIdx.x >> 6;
-    const int c = blockIdx.x * 64 + cl;
-    const int per = (rows + (int)gridDim.y - 1) / (int)gridDim.y;
-    const int r0 = (int)blockIdx.y * per, r1 = r0 + per < rows ? r0 + per : rows;
-    float s = 0.0f;
-    if (c < cols && c < n_live)
-        for (int r = r0 + grp; r < r1; r += 4) s += G[(long)r * cols + c];
-    red[grp][cl] = s;
     __syncthreads();
-    if (grp == 0 && c < cols) part[(long)blockIdx.y * cols + c] = ((red[0][cl] + red[1][cl]) + red[2][cl]) + red[3][cl];
+    // dl = (sigmoid(l) - x) / B, log q
+    double loss = 0.0;
+    float* dlT = p.dlT + (int64_t)blk * Np * 16 + 64 * g + r;
+#pragma unroll
+    for (int k = 0; k < NW; k++) {
+        const int m = q * NW + k;
+        floatx4 l = *reinterpret_cast<const floatx4*>(p.b2 + 16 * m + 4 * g);
+#pragma unroll
+        for (int z = 0; z < 4; z++) l += lpart[z][m][lane];
+#pragma unroll
+        for (int v = 0; v < 4; v++) {
+            const int j = 16 * m + 4 * g + v;
+            const float x = bit_of(w0, w1, j) ? 1.0f : 0.0f;
+            const bool live = valid && j < p.N;
+            const float lv = l[v];
+            if (live) loss += (double)(x * lv) - (double)softplusf_acc(lv);
+            const float d = live ? (sigmoidf_acc(lv) - x) * p.inv_batch : 0.0f;
+            l[v] = d;
+            dlT[256 * m + 16 * v] = d;
+            const float sum = row_sum16(d);
+            if (r == 0) p.bias_part[(int64_t)blk * (Hp + Np) + Hp + j] = sum;
+        }
+        dls[m][lane] = l;
+    }
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) loss += __shfl_xor(loss, off);
+    if (lane == 0) lsum[q] = loss;
+    __syncthreads();
+    if (threadIdx.x == 0) p.loss_part[blk] = ((lsum[0] + lsum[1]) + lsum[2]) + lsum[3];
+    // da = (W2^T dl) [a > 0]
+    floatx4 w[2][HW], d[HW];
+#pragma unroll
+    for (int m = 0; m < HW; m++) d[m] = floatx4{0.f, 0.f, 0.f, 0.f};
+    made_tiles<HW>(w[0], p.W2t, NT, q * HW, 0);
+#pragma unroll
+    for (int t = 0; t < NT; t++) {
+        if (t + 1 < NT) made_tiles<HW>(w[(t + 1) & 1], p.W2t, NT, q * HW, t + 1);
+        __builtin_amdgcn_sched_barrier(0);
+        const floatx4 l = dls[t][lane];
+#pragma unroll
+        for (int v = 0; v < 4; v++)
+#pragma unroll
+            for (int m = 0; m < HW; m++) d[m] = __builtin_amdgcn_mfma_f32_16x16x4f32(w[t & 1][m][v], l[v], d[m], 0, 0, 0);
+    }
+    float* daT = p.daT + ((int64_t)blk * Hp + 16 * q * HW) * 16 + 64 * g + r;
+#pragma unroll
+    for (int m = 0; m < HW; m++)
+#pragma unroll
+        for (int v = 0; v < 4; v++) {
+            const float da = a[m][v] > 0.0f ? d[m][v] : 0.0f;
+            daT[256 * m + 16 * v] = da;
+            const float sum = row_sum16(da);
+            if (r == 0) p.bias_part[(int64_t)blk * (Hp + Np) + 16 * (q * HW + m) + 4 * g + v] = sum;
+        }
 }
 
-__global__ __launch_bounds__(256) void k_colsum_finish(int cols, int slices, const float* __restrict__ part,
-                                                       float* __restrict__ out) {
-    const int c = blockIdx.x * blockDim.x + threadIdx.x;
-    if (c >= cols) return;
-    float t = 0.0f;
-    for (int y = 0; y < slices; y++) t += part[(long)y * cols + c];
-    out[c] = t;
+// dW1 = da^T x and dW2 = dl^T h.  A workgroup owns a 64 x 64 block of either
+// and sample tiles z, z + splits, ..., in turn for its wavefronts, which read 16 samples of 64 + 64 rows per step (64 MFMAs), the
+// next step's before them, and add their sums through LDS; part[z] holds both
+// gradients at their places in the parameters.  Four wavefronts to a workgroup
+// also keep the SIMDs evenly loaded: as single wavefronts they took 28 to 40 us
+// (N = 100, H = 256, 16 384 samples) with where the launch before had left room.
+template <bool FIRST>
+RBM_DI void made_wgrad(const MadeStep& p, int Np, int Hp, int row0, int col0, int t0, int dt, int tiles, float* __restrict__ out,
+                       floatx4 (*sums)[16][64]) {
+    const int lane = threadIdx.x & 63, g = lane >> 4, r = lane & 15;
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int rows = FIRST ? Hp : Np, cols = FIRST ? Np : Hp;
+    const float* A = (FIRST ? p.daT : p.dlT) + (row0 + r) * 16 + 4 * g;
+    const float* Bm = p.hT + (col0 + r) * 16 + 4 * g;
+    const uint16_t* X = p.xbits + col0 + r;
+    floatx4 acc[4][4];
+#pragma unroll
+    for (int i = 0; i < 4; i++)
+#pragma unroll
+        for (int j = 0; j < 4; j++) acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
+    floatx4 fa[2][4], fb[2][4];
+    uint32_t xb[2][4];
+    auto fetch = [&](int k, int t) {
+#pragma unroll
+        for (int i = 0; i < 4; i++) fa[k][i] = *reinterpret_cast<const floatx4*>(A + ((int64_t)t * rows + 16 * i) * 16);
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            if (FIRST) xb[k][j] = X[(int64_t)t * cols + 16 * j];
+            else fb[k][j] = *reinterpret_cast<const floatx4*>(Bm + ((int64_t)t * cols + 16 * j) * 16);
+        }
+    };
+    auto step = [&](int k) {
+        if (FIRST) {
+#pragma unroll
+            for (int j = 0; j < 4; j++)
+#pragma unroll
+                for (int v = 0; v < 4; v++) fb[k][j][v] = (xb[k][j] >> (4 * g + v)) & 1u ? 1.0f : 0.0f;
+        }
+#pragma unroll
+        for (int v = 0; v < 4; v++)
+#pragma unroll
+            for (int i = 0; i < 4; i++)
+#pragma unroll
+                for (int j = 0; j < 4; j++)
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(fa[k][i][v], fb[k][j][v], acc[i][j], 0, 0, 0);
+    };
+    int t = t0 + wave * dt;
+    dt *= 4;
+    if (t < tiles) fetch(0, t);
+    for (; t < tiles; t += 2 * dt) {
+        if (t + dt < tiles) fetch(1, t + dt);
+        __builtin_amdgcn_sched_barrier(0);
+        step(0);
+        if (t + 2 * dt < tiles) fetch(0, t + 2 * dt);
+        __builtin_amdgcn_sched_barrier(0);
+        if (t + dt < tiles) step(1);
+    }
+#pragma unroll
+    for (int i = 0; i < 4; i++)
+#pragma unroll
+        for (int j = 0; j < 4; j++) sums[wave][4 * i + j][lane] = acc[i][j];
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        floatx4 x = sums[0][4 * wave + j][lane];
+#pragma unroll
+        for (int z = 1; z < 4; z++) x += sums[z][4 * wave + j][lane];
+#pragma unroll
+        for (int v = 0; v < 4; v++) out[(int64_t)(row0 + 16 * wave + 4 * g + v) * cols + col0 + 16 * j + r] = x[v];
+    }
 }
 
-hipError_t launch_colsum(int rows, int cols, int n_live, const float* G, float* out, float* part, hipStream_t stream) {
-    if (rows <= 0 || cols <= 0) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(k_colsum_part, dim3((cols + 63) / 64, COLSUM_SLICES), dim3(256), 0, stream, rows, cols, n_live, G,
-                       part);
-    hipError_t err = hipGetLastError();
-    if (err != hipSuccess) return err;
-    hipLaunchKernelGGL(k_colsum_finish, dim3((cols + 255) / 256), dim3(256), 0, stream, cols, COLSUM_SLICES, part, out);
+// Workgroups go to the 8 dies in turn: all blocks of a split to one die, which
+// so reads its samples from memory once, and with a multiple of 8 splits to the
+// die whose workgroups of k_made_pass wrote them.
+__global__ __launch_bounds__(256) void k_made_wgrad(MadeStep p, int Np, int Hp, int tiles, int splits) {
+    __shared__ floatx4 sums[4][16][64];
+    const int half = (Np / 64) * (Hp / 64);   // blocks of each gradient
+    const int b = ((int)blockIdx.x / 8) % (2 * half), z = (int)blockIdx.x / (16 * half) * 8 + (int)blockIdx.x % 8;
+    if (z >= splits) return;
+    const bool first = b < half;              // dW1: Hp x Np, dW2: Np x Hp
+    const int q = first ? b : b - half, cols = first ? Np / 64 : Hp / 64;
+    const int row0 = 64 * (q / cols), col0 = 64 * (q % cols);
+    float* out = p.wgrad_part + (int64_t)z * p.padded;
+    if (first) made_wgrad<true>(p, Np, Hp, row0, col0, z, splits, tiles, out, sums);
+    else made_wgrad<false>(p, Np, Hp, row0, col0, z, splits, tiles, out + p.off_W2, sums);
+}
+
+// Gradient of every parameter (the splits and the sample tiles' bias sums
+// added in a fixed order, masked entries zero), then Adam (Kingma & Ba 2015),
+// or the gradient alone when u.grad is set.  Weights: one thread per
+// parameter; biases: workgroups past the weights' take 16 of them with 16
+// threads each.
+RBM_DI void made_apply(const MadeUpdate& u, int64_t e, float gk) {
+    if (u.grad) { u.grad[e] = gk; return; }
+    const float mk_ = u.beta1 * u.m[e] + (1.0f - u.beta1) * gk;
+    const float vk = u.beta2 * u.v[e] + (1.0f - u.beta2) * gk * gk;
+    u.m[e] = mk_;
+    u.v[e] = vk;
+    u.params[e] -= u.lr * (mk_ * u.c1) / (sqrtf(vk * u.c2) + u.eps);
+}
+
+// One weight into the packed copies: W1, W2 and W2 transposed, Np Hp floats each
+RBM_DI void made_pack(const MadeShape& sh, bool first, int row, int col, float x, float* __restrict__ packed) {
+    const int64_t W = (int64_t)sh.Np * sh.Hp;
+    if (first) {
+        packed[made_packed(row, col, sh.Np / 16)] = x;
+    } else {
+        packed[W + made_packed(row, col, sh.Hp / 16)] = x;
+        packed[2 * W + made_packed(col, row, sh.Np / 16)] = x;
+    }
+}
+
+__global__ __launch_bounds__(256) void k_made_update(MadeShape sh, MadeUpdate u, int splits, int tiles, int64_t off_b1,
+                                                     int64_t off_W2, int64_t off_b2, int64_t padded, int weight_blocks,
+                                                     const float* __restrict__ wpart, const float* __restrict__ bpart,
+                                                     float* __restrict__ packed) {
+    const int N = sh.N, H = sh.H, Np = sh.Np, Hp = sh.Hp;
+    if ((int)blockIdx.x < weight_blocks) {
+        const int64_t k = (int64_t)blockIdx.x * 256 + threadIdx.x;
+        const int64_t W = (int64_t)Np * Hp;
+        if (k >= 2 * W) return;
+        const bool first = k < W;
+        const int64_t e = first ? k : off_W2 + (k - W);
+        float x = 0.0f;
+#pragma unroll 16
+        for (int z = 0; z < splits; z++) x += wpart[(int64_t)z * padded + e];
+        const int row = first ? (int)(k / Np) : (int)((k - W) / Hp), col = first ? (int)(k % Np) : (int)((k - W) % Hp);
+        const bool ok = first ? row < H && col < N && col < made_degree(row, N) : row < N && col < H && made_degree(col, N) <= row;
+        made_apply(u, e, ok ? x : 0.0f);
+        if (!u.grad) made_pack(sh, first, row, col, u.params[e], packed);
+        return;
+    }
+    __shared__ float red[16][17];
+    const int x = threadIdx.x & 15, y = threadIdx.x >> 4;
+    const int k = ((int)blockIdx.x - weight_blocks) * 16 + x;   // b1, then b2
+    float s = 0.0f;
+#pragma unroll 16
+    for (int t = y; t < tiles; t += 16) s += bpart[(int64_t)t * (Hp + Np) + k];
+    red[y][x] = s;
+    __syncthreads();
+    if (y == 0) {
+        for (int q = 1; q < 16; q++) s += red[q][x];
+        const bool ok = k < Hp ? k < H : k - Hp < N;
+        made_apply(u, k < Hp ? off_b1 + k : off_b2 + (k - Hp), ok ? s : 0.0f);
+    }
+}
+
+__global__ __launch_bounds__(256) void k_made_pack(MadeShape sh, const float* __restrict__ W1, const float* __restrict__ W2,
+                                                   float* __restrict__ packed) {
+    const int64_t W = (int64_t)sh.Np * sh.Hp;
+    for (int64_t k = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; k < 2 * W; k += (int64_t)gridDim.x * blockDim.x) {
+        if (k < W) made_pack(sh, true, (int)(k / sh.Np), (int)(k % sh.Np), W1[k], packed);
+        else made_pack(sh, false, (int)((k - W) / sh.Hp), (int)((k - W) % sh.Hp), W2[k - W], packed);
+    }
+}
+
+hipError_t launch_made_pack(const MadeShape& s, const float* W1, const float* W2, float* packed, hipStream_t stream) {
+    hipLaunchKernelGGL(k_made_pack, dim3(256), dim3(256), 0, stream, s, W1, W2, packed);
+    return hipGetLastError();
+}
+
+int made_wgrad_splits(const MadeShape& s, int tiles) {
+    // two workgroups a compute unit, at least 4 sample tiles a workgroup
+    const int blocks = 2 * (s.Np / 64) * (s.Hp / 64);
+    int z = 512 / blocks;
+    if (z > tiles / 4) z = tiles / 4;
+    if (z > 8) z -= z % 8;
+    return z < 1 ? 1 : z;
+}
+
+hipError_t launch_made_pass(const MadeShape& sh, const MadeStep& p, hipStream_t stream) {
+    if (p.Bp <= 0 || p.Bp % 64 || sh.Np % 64 || sh.Hp % 64) return hipErrorInvalidValue;
+    const dim3 grid((unsigned)(p.Bp / 16)), block(256);
+#define RBM_PASS_CASE(NT_, HT_)                                                                  \
+    if (sh.Np == 16 * NT_ && sh.Hp == 16 * HT_) {                                                \
+        hipLaunchKernelGGL((k_made_pass<NT_, HT_>), grid, block, 0, stream, p);                  \
+        return hipGetLastError();                                                                \
+    }
+#define RBM_PASS_ROW(HT_) RBM_PASS_CASE(4, HT_) RBM_PASS_CASE(8, HT_)
+    RBM_PASS_ROW(4) RBM_PASS_ROW(8) RBM_PASS_ROW(12) RBM_PASS_ROW(16) RBM_PASS_ROW(20) RBM_PASS_ROW(24) RBM_PASS_ROW(28)
+    RBM_PASS_ROW(32)
+#undef RBM_PASS_ROW
+#undef RBM_PASS_CASE
+    return hipErrorInvalidValue;
+}
+
+hipError_t launch_made_wgrad(const MadeShape& sh, const MadeStep& p, int splits, hipStream_t stream) {
+    const int tiles = p.Bp / 16;
+    if (splits < 1 || splits > tiles) return hipErrorInvalidValue;
+    const int blocks = 2 * (sh.Np / 64) * (sh.Hp / 64);
+    hipLaunchKernelGGL(k_made_wgrad, dim3((unsigned)(blocks * ((splits + 7) / 8 * 8))), dim3(256), 0, stream, p, sh.Np,
+                       sh.Hp, tiles, splits);
+    return hipGetLastError();
+}
+
+hipError_t launch_made_update(const MadeShape& sh, const MadeUpdate& u, const MadeStep& p, int splits, float* packed,
+                              hipStream_t stream) {
+    const int weight_blocks = (int)((2ll * sh.Np * sh.Hp + 255) / 256), bias_blocks = (sh.Hp + sh.Np) / 16;
+    hipLaunchKernelGGL(k_made_update, dim3((unsigned)(weight_blocks + bias_blocks)), dim3(256), 0, stream, sh, u, splits,
+                       p.Bp / 16, p.off_b1, p.off_W2, p.off_b2, p.padded, weight_blocks, p.wgrad_part, p.bias_part, packed);
     return hipGetLastError();
 }
 
@@ -266,29 +413,6 @@ hipError_t launch_zero(int64_t n, float* p, hipStream_t stream) {
     if (blocks > 2048) blocks = 2048;
     if (blocks < 1) blocks = 1;
     hipLaunchKernelGGL(k_zero, dim3((unsigned)blocks), dim3(256), 0, stream, n, p);
-    return hipGetLastError();
-}
-
-__global__ __launch_bounds__(256) void k_adam(int64_t n, float* __restrict__ p, const float* __restrict__ g,
-                                              float* __restrict__ m, float* __restrict__ v, float c1, float c2,
-                                              float lr, float b1, float b2, float eps) {
-    for (int64_t k = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; k < n; k += (int64_t)gridDim.x * blockDim.x) {
-        const float gk = g[k];
-        const float mk_ = b1 * m[k] + (1.0f - b1) * gk;
-        const float vk = b2 * v[k] + (1.0f - b2) * gk * gk;
-        m[k] = mk_;
-        v[k] = vk;
-        p[k] -= lr * (mk_ * c1) / (sqrtf(vk * c2) + eps);
-    }
-}
-
-hipError_t launch_adam(int64_t n, float* p, const float* g, float* m, float* v, int t, float lr, float b1, float b2,
-                       float eps, hipStream_t stream) {
-    const float c1 = (float)(1.0 / (1.0 - pow((double)b1, t)));
-    const float c2 = (float)(1.0 / (1.0 - pow((double)b2, t)));
-    int64_t blocks = (n + 255) / 256;
-    if (blocks > 2048) blocks = 2048;
-    hipLaunchKernelGGL(k_adam, dim3((unsigned)blocks), dim3(256), 0, stream, n, p, g, m, v, c1, c2, lr, b1, b2, eps);
     return hipGetLastError();
 }
 

@@ -46,56 +46,46 @@ __host__ __device__ inline int made_sorted_unit(int p, int N, int H) {
     return d1 + t * (N - 1);
 }
 
-enum GemmEpi {
-    EPI_STORE = 0,       // C = acc
-    EPI_BIAS_RELU = 1,   // C = acc + bias[n] (pre-activation), C2 = relu(C)
-    EPI_LOGITS = 2,      // l = acc + bias[n]; C = (sigmoid(l) - x) / B on live entries, 0 elsewhere; log-q partials
-    EPI_MASK_W2 = 3,     // C (Np x Hp) = acc where deg(n) <= m < N and n < H, else 0
-    EPI_MASK_W1 = 4,     // C (Hp x Np) = acc where n < deg(m), m < H and n < N, else 0
-    EPI_RELU_GRAD = 5,   // C = acc where aux[m][n] > 0, else 0
-};
-
-struct GemmEpiArgs {
-    const float* bias;   // EPI_BIAS_RELU, EPI_LOGITS
-    float* C2;           // EPI_BIAS_RELU
-    const float* aux;    // EPI_LOGITS: X (B x Np); EPI_RELU_GRAD: pre-activation
-    long ld_aux;
-    int n_live, m_live;  // live columns / rows (N or H, real batch)
+// One training step.  Minibatch row s is sample s of `spins`, or, with draw,
+// floor(u n) with u from Philox(seed; ctr = (step, s, 0, 4)); rows B .. Bp (a
+// multiple of 64) are padding.  Parameters are one padded block [W1 (Hp x Np),
+// b1 (Hp), W2 (Np x Hp), b2 (Np)]; the pass reads the weights from packed copies,
+// W1, W2 and W2t (W2 transposed), that the update keeps.
+// Left by the pass for the weight gradients, per tile of 16 samples: hT and daT
+// [Hp][16], dlT [Np][16], xbits [Np] (bit k of entry i is input i of the tile's
+// sample k), bias_part [Hp + Np] and the log q sum.
+struct MadeStep {
+    int N, B, Bp;
+    int64_t n;
+    int draw;
+    uint32_t step, seed_lo, seed_hi;
+    const uint64_t* spins;
+    const float *W1, *b1, *W2, *b2, *W2t;
     float inv_batch;
-    double* partials;    // EPI_LOGITS: one log-q partial per workgroup
-    int lower_only;      // compute only the 64 x 64 tiles with n0 <= m0 (symmetric products)
+    float *hT, *daT, *dlT;
+    uint16_t* xbits;
+    float* bias_part;     // (Bp / 16) x (Hp + Np)
+    double* loss_part;    // Bp / 16
+    float* wgrad_part;    // splits x padded
+    int64_t off_b1, off_W2, off_b2, padded;
 };
-
-// C[m][n] = sum_k A(m,k) B(k,n), A(m,k) = A[m*sam + k*sak], B(k,n) = B[k*sbk + n*sbn];
-// M, N multiples of 64, K a multiple of 16.
-hipError_t launch_gemm(int epi, int M, int N, int K, const float* A, long sam, long sak, const float* B, long sbk,
-                       long sbn, float* C, long ldc, const GemmEpiArgs& e, hipStream_t stream);
-
-// The same product with K split over `splits` workgroups (K a multiple of
-// 16 * splits): partial products go to scratch (splits x M x N floats) and a
-// second kernel adds them in order and applies EPI_STORE, EPI_MASK_W1 or
-// EPI_MASK_W2.  For the weight gradients, whose M x N is small and K (the batch)
-// long.
-hipError_t launch_gemm_splitk(int epi, int M, int N, int K, const float* A, long sam, long sak, const float* B,
-                              long sbk, long sbn, float* C, long ldc, const GemmEpiArgs& e, int splits, float* scratch,
+// Adam's arrays and the step's constants (c1, c2: bias corrections), or the
+// gradient alone into `grad`
+struct MadeUpdate {
+    float *params, *m, *v, *grad;
+    float c1, c2, lr, beta1, beta2, eps;
+};
+// packed = [W1, W2, W2t] in the order of the pass (3 Np Hp floats)
+hipError_t launch_made_pack(const MadeShape& s, const float* W1, const float* W2, float* packed, hipStream_t stream);
+hipError_t launch_made_pass(const MadeShape& s, const MadeStep& p, hipStream_t stream);
+// sample splits of the weight gradients for Bp / 16 = tiles
+int made_wgrad_splits(const MadeShape& s, int tiles);
+hipError_t launch_made_wgrad(const MadeShape& s, const MadeStep& p, int splits, hipStream_t stream);
+hipError_t launch_made_update(const MadeShape& s, const MadeUpdate& u, const MadeStep& p, int splits, float* packed,
                               hipStream_t stream);
-
-// X[s][i] = bit i of spins[idx[s]] (or of spins[s] without idx) for i < N, 0 for the padding
-// and for rows s >= n_live.
-hipError_t launch_made_gather(int64_t rows, int n_live, int N, int Np, const uint64_t* spins, const int64_t* idx,
-                              float* X, hipStream_t stream);
-// batch indices: idx[s] = floor(u * n) with u from Philox(seed; ctr = (step, s, 0, 4))
-hipError_t launch_made_batch_index(int B, int64_t n, uint32_t step, uint32_t seed_lo, uint32_t seed_hi, int64_t* idx,
-                                   hipStream_t stream);
-// out[n] = sum_m G[m][n] over rows m < rows (ld = cols), fixed order
-constexpr int COLSUM_SLICES = 32;   // row slices of launch_colsum; part holds COLSUM_SLICES x cols floats
-hipError_t launch_colsum(int rows, int cols, int n_live, const float* G, float* out, float* part, hipStream_t stream);
 // p[0 .. n) = 0 (a fill kernel, so the optimiser state can be cleared inside
 // captured work)
 hipError_t launch_zero(int64_t n, float* p, hipStream_t stream);
-// Adam (Kingma & Ba 2015) over n parameters; t is the 1-based step
-hipError_t launch_adam(int64_t n, float* p, const float* g, float* m, float* v, int t, float lr, float b1, float b2,
-                       float eps, hipStream_t stream);
 // bfloat16 inference copies of W1 (transposed) and W2 in the sampler's layout:
 // hidden units in degree-sorted order (made_sorted_unit), row j of either
 // matrix as Hp / 2 words, word 32 t + 2 l + b holding pair v = 2 t + b of
