@@ -1717,7 +1717,8 @@ static cx<double>* s_matrix_centred(Ctx& c, rbmhip_psi* psi, rbmhip_ens* ens, co
 static void cholesky_solve_device(Ctx& c, int n, cx<double>* A, cx<double>* x) {
     int* info = reinterpret_cast<int*>(c.buf("chol_info", 64));
     c.launch("cholesky", [&] { return launch_zero(16, reinterpret_cast<float*>(info), c.stream); });
-    c.launch("cholesky", [&] { return launch_cholesky(n, A, info, c.stream); });
+    cx<double>* D = reinterpret_cast<cx<double>*>(c.buf("chol_D", CHOL_WORK * sizeof(cx<double>)));
+    c.launch("cholesky", [&] { return launch_cholesky(n, A, D, info, c.stream); });
     int h = 0;
     c.d2h(&h, info, sizeof(int));
     c.sync();

@@ -4,14 +4,13 @@
 // builds S).  Matrices are row-major, n x n complex<double>; the factor
 // overwrites the lower triangle (A = L L^H).
 //
-// Blocked right-looking factorisation, panels of NB = 32 in block columns of
-// NB2 = 128:
-//   k_potrf_diag   factor the diagonal block in LDS (one 1024-thread workgroup)
-//   k_trsm_panel   rows below: X L_kk^H = A_ik (32 lanes per row)
-//   k_herk_update  lower-triangle update A_il -= X_i X_l^H (64 x 64 tiles):
-//                  per panel within its block column, per block column
-//                  (rank 128) on the trailing matrix
-// then blocked forward and backward substitution (k_trsv_block, k_trsv_update).
+// Blocked right-looking factorisation, block columns of CB = 128 in panels of
+// NB = 32, with FP64 MFMA for the updates:
+//   k_chol_trail   rank-128 update of the trailing matrix by the last block column
+//   k_chol_panel   a panel's solve X L_kk^H = A_ik and its update of the rest of
+//                  the block column
+// each of which also factors the next 32 x 32 diagonal block (potrf32);
+// then blocked forward and backward substitution (k_trsv_forward, _backward).
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -21,160 +20,372 @@ namespace rbmhip {
 
 constexpr int NB = 32;
 
-RBM_DI cx<double> cmul_conj(cx<double> a, cx<double> b) {   // a * conj(b)
-    return mk(a.re * b.re + a.im * b.im, a.im * b.re - a.re * b.im);
-}
-
-// One workgroup of NB x NB threads factors A[k0:k0+nb, k0:k0+nb] in LDS, one
-// barrier per column: at step j every thread reads the pivot d = A_jj,
-// thread (i, j) writes the finished L_ij (A_ij / sqrt(d), or sqrt(d) on the
-// diagonal) straight to global memory, and threads (i, l) with j < l <= i
-// subtract (A_ij / sqrt d) conj(A_lj / sqrt d) in LDS.  Column j is only read
-// during step j, so the scaled values never need to go back to LDS.
-// A non-positive pivot sets *info = global pivot index + 1 (and is replaced
-// by 1 so that the factorisation runs to the end).
-__global__ __launch_bounds__(1024) void k_potrf_diag(int n, int k0, cx<double>* __restrict__ A, int* __restrict__ info) {
-    __shared__ cx<double> L[NB][NB + 1];
-    const int i = threadIdx.x / NB, l = threadIdx.x % NB;
-    const int nb = n - k0 < NB ? n - k0 : NB;
-    L[i][l] = (i < nb && l < nb && l <= i) ? A[(int64_t)(k0 + i) * n + k0 + l] : mk(0.0, 0.0);
-    __syncthreads();
-    int bad = 0;
-    for (int j = 0; j < nb; j++) {
-        double d = L[j][j].re;
-        if (!(d > 0.0)) {
-            if (!bad) bad = k0 + j + 1;
-            d = 1.0;
-        }
-        const double sd = sqrt(d), rs = 1.0 / sd;
-        if (i < nb && i >= j) {
-            if (l == j) {
-                A[(int64_t)(k0 + i) * n + k0 + j] = i == j ? mk(sd, 0.0) : mk(L[i][j].re * rs, L[i][j].im * rs);
-            } else if (l > j && l <= i) {
-                const cx<double> a = L[i][j], c = L[l][j];
-                const cx<double> u = cmul_conj(mk(a.re * rs, a.im * rs), mk(c.re * rs, c.im * rs));
-                L[i][l] = mk(L[i][l].re - u.re, L[i][l].im - u.im);
-            }
-        }
-        __syncthreads();
-    }
-    if (threadIdx.x == 0 && bad && *info == 0) *info = bad;
-}
-
 // Lane j's value of a complex double, broadcast to the whole wavefront (j is
 // wave-uniform).
-RBM_DI cx<double> lane_bcast(cx<double> v, int j) {
-    const int2 r = *reinterpret_cast<int2*>(&v.re), i = *reinterpret_cast<int2*>(&v.im);
-    int2 rr, ii;
-    rr.x = __builtin_amdgcn_readlane(r.x, j); rr.y = __builtin_amdgcn_readlane(r.y, j);
-    ii.x = __builtin_amdgcn_readlane(i.x, j); ii.y = __builtin_amdgcn_readlane(i.y, j);
-    return mk(*reinterpret_cast<double*>(&rr), *reinterpret_cast<double*>(&ii));
+RBM_DI double lane_bcast(double v, int j) {
+    const int2 r = *reinterpret_cast<int2*>(&v);
+    int2 q;
+    q.x = __builtin_amdgcn_readlane(r.x, j);
+    q.y = __builtin_amdgcn_readlane(r.y, j);
+    return *reinterpret_cast<double*>(&q);
 }
+RBM_DI cx<double> lane_bcast(cx<double> v, int j) { return mk(lane_bcast(v.re, j), lane_bcast(v.im, j)); }
 
-// Rows r >= k0 + nb: solve X L_kk^H = A[r, k0:k0+nb] in place, i.e. for each
-// row x_j = (a_j - sum_{m<j} x_m conj(L_jm)) / L_jj.  32 lanes per row (two
-// rows per wavefront), lane j holding x_j: at step m the row's x_m is final and
-// lanes j > m subtract x_m conj(L_jm), so each x_j receives its terms in the
-// order m = 0, 1, ... as in a sequential solve.
-__global__ __launch_bounds__(256) void k_trsm_panel(int n, int k0, cx<double>* __restrict__ A) {
-    __shared__ cx<double> L[NB][NB + 1];
-    const int nb = n - k0 < NB ? n - k0 : NB;
-    for (int t = threadIdx.x; t < NB * NB; t += blockDim.x) {
-        const int i = t / NB, l = t % NB;
-        L[i][l] = (i < nb && l <= i) ? A[(int64_t)(k0 + i) * n + k0 + l] : mk(0.0, 0.0);
-    }
-    __syncthreads();
-    const int j = threadIdx.x & 31, half = (threadIdx.x >> 5) & 1;
-    const int64_t r = (int64_t)k0 + nb + ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) / 32;
-    const bool live = r < n && j < nb;
-    cx<double>* row = A + (r < n ? r : n - 1) * n + k0;
-    cx<double> x = live ? row[j] : mk(0.0, 0.0);
-    for (int m = 0; m < nb; m++) {
-        if (j == m) {
-            const double rd = 1.0 / L[m][m].re;
-            x = mk(x.re * rd, x.im * rd);
-        }
-        const cx<double> x0 = lane_bcast(x, m), x1 = lane_bcast(x, 32 + m);
-        const cx<double> xm = half ? x1 : x0;
-        if (j > m) {
-            const cx<double> u = cmul_conj(xm, L[j][m]);
-            x = mk(x.re - u.re, x.im - u.im);
-        }
-    }
-    if (live) row[j] = x;
-}
-
-// Trailing update A_il -= sum_m A_im conj(A_lm) over the panel columns
-// m = kc .. kc + kw - 1, for entries with row i >= column l >= base and
-// l < col_end.  One 256-thread workgroup per 64 x 64 tile: thread
-// (tx, ty) = (t % 16, t / 16) owns rows ty + 16 a and columns tx + 16 b
-// (a, b < 4), so each panel value read from LDS serves four products.  The
-// panel is staged 32 columns at a time.  ctiles == 0: the lower-triangle tiles
-// of [base, n)^2, t = bi (bi + 1) / 2 + bj; ctiles > 0: a 2-D grid over a band
-// of ctiles column tiles (bj = blockIdx.x, bi = blockIdx.y), tiles above the
-// diagonal exit.
-constexpr int HT = 64;
-__global__ __launch_bounds__(256) void k_herk_update(int n, int kc, int kw, int base, int col_end, int ctiles,
-                                                     cx<double>* __restrict__ A) {
-    __shared__ cx<double> Pi[HT][NB + 1];
-    __shared__ cx<double> Pl[HT][NB + 1];
-    int bi, bj;
-    if (ctiles == 0) {
-        const int t = blockIdx.x;
-        bi = (int)((sqrt(8.0 * t + 1.0) - 1.0) * 0.5);
-        while ((bi + 1) * (bi + 2) / 2 <= t) bi++;
-        while (bi * (bi + 1) / 2 > t) bi--;
-        bj = t - bi * (bi + 1) / 2;
+// sqrt(d) and 1 / sqrt(d) of a positive d: the hardware's reciprocal square root
+// and one third-order and one second-order correction step, where that can
+// neither overflow nor lose bits, else the library's.
+RBM_DI void sqrt_pair(double d, double& sd, double& rs) {
+    if (d > 1e-200 && d < 1e200) {
+        double y = __builtin_amdgcn_rsq(d);
+        double e = __builtin_fma(-d * y, y, 1.0);
+        y = __builtin_fma(y * e, __builtin_fma(e, 0.375, 0.5), y);
+        e = __builtin_fma(-d * y, y, 1.0);
+        rs = __builtin_fma(y * e, 0.5, y);
+        sd = d * rs;
+        sd = __builtin_fma(__builtin_fma(-sd, sd, d), 0.5 * rs, sd);
     } else {
-        bj = blockIdx.x;
-        bi = blockIdx.y;
-        if (bj > bi) return;
+        sd = sqrt(d);
+        rs = 1.0 / sd;
     }
-    const int r0 = base + bi * HT, c0 = base + bj * HT;
-    const int tx = threadIdx.x & 15, ty = threadIdx.x >> 4;
-    double accr[4][4], acci[4][4];
+}
+
+typedef double doublex4 __attribute__((ext_vector_type(4)));
+// a complex value as one 16-byte word: as a struct, arrays of them that loads
+// fill ahead of their use end up in scratch memory
+typedef double doublex2 __attribute__((ext_vector_type(2)));
+RBM_DI doublex2 load2(const cx<double>* p) { return *reinterpret_cast<const doublex2*>(p); }
+RBM_DI void store2(cx<double>* p, doublex2 v) { *reinterpret_cast<doublex2*>(p) = v; }
+constexpr int CB = 128;        // block column
+constexpr int CLD = NB + 1;    // LDS stride of 32-column panels
+
+// acc += X Y^H for one 16 x 16 tile and 4 columns, x and y this lane's X[l % 16]
+// [l / 16] and Y[l % 16][l / 16]
+RBM_DI void mfma_herk(doublex4& re, doublex4& im, cx<double> x, cx<double> y) {
+    re = __builtin_amdgcn_mfma_f64_16x16x4f64(x.re, y.re, re, 0, 0, 0);
+    im = __builtin_amdgcn_mfma_f64_16x16x4f64(x.im, y.re, im, 0, 0, 0);
+    re = __builtin_amdgcn_mfma_f64_16x16x4f64(x.im, y.im, re, 0, 0, 0);
+    im = __builtin_amdgcn_mfma_f64_16x16x4f64(-x.re, y.im, im, 0, 0, 0);
+}
+
+// 256 threads factor the 32 x 32 block L (lower triangle; rows past the matrix
+// are the identity) in place and write its lower triangle to A[k0:, k0:].
+// Thread (i, g) = (t % 32, t / 32) holds row i, columns 8 q + g; step j = 8 q + g
+// passes the finished column through L, one barrier each.  A pivot that is not
+// positive sets *info = index + 1, if none had, and is replaced by 1 so that the
+// factorisation runs to the end.  Compact loops: unrolled over j the code of one
+// use, 40 KiB, took longer to fetch than to execute (n = 32: 40 us against 12).
+RBM_DI void potrf_store(int n, int k0, cx<double> (*L)[CLD], cx<double>* __restrict__ A, int* __restrict__ info) {
+    const int i = threadIdx.x & 31, g = threadIdx.x >> 5;
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    cx<double> a[4];
 #pragma unroll
-    for (int a = 0; a < 4; a++)
+    for (int q = 0; q < 4; q++) a[q] = L[i][8 * q + g];
+    int bad = 0;
 #pragma unroll
-        for (int b = 0; b < 4; b++) accr[a][b] = acci[a][b] = 0.0;
-    for (int k0 = 0; k0 < kw; k0 += NB) {
-        for (int q = threadIdx.x; q < HT * NB; q += 256) {
-            const int a = q / NB, m = q % NB;
-            const int ri = r0 + a, rl = c0 + a;
-            const bool live = k0 + m < kw;
-            Pi[a][m] = (ri < n && live) ? A[(int64_t)ri * n + kc + k0 + m] : mk(0.0, 0.0);
-            Pl[a][m] = (rl < n && live) ? A[(int64_t)rl * n + kc + k0 + m] : mk(0.0, 0.0);
-        }
-        __syncthreads();
-#pragma unroll 2
-        for (int m = 0; m < NB; m++) {
-            cx<double> pi[4], pl[4];
-#pragma unroll
-            for (int a = 0; a < 4; a++) pi[a] = Pi[ty + 16 * a][m];
-#pragma unroll
-            for (int b = 0; b < 4; b++) pl[b] = Pl[tx + 16 * b][m];
-#pragma unroll
-            for (int a = 0; a < 4; a++)
-#pragma unroll
-                for (int b = 0; b < 4; b++) {
-                    // pi conj(pl)
-                    accr[a][b] = __builtin_fma(pi[a].re, pl[b].re, __builtin_fma(pi[a].im, pl[b].im, accr[a][b]));
-                    acci[a][b] = __builtin_fma(pi[a].im, pl[b].re, __builtin_fma(-pi[a].re, pl[b].im, acci[a][b]));
+    for (int q = 0; q < 4; q++)
+#pragma unroll 1
+        for (int gj = 0; gj < 8; gj++) {
+            const int j = 8 * q + gj;
+            if (wave == gj >> 1) {
+                double d = lane_bcast(a[q].re, j + 32 * (gj & 1)), sd, rs;
+                if (!(d > 0.0)) {
+                    if (!bad) bad = k0 + j + 1;
+                    d = 1.0;
                 }
-        }
-        __syncthreads();
-    }
+                sqrt_pair(d, sd, rs);
+                if (g == gj && i >= j) L[i][j] = i == j ? mk(sd, 0.0) : mk(a[q].re * rs, a[q].im * rs);
+            }
+            __syncthreads();
+            const cx<double> x = L[i][j];
 #pragma unroll
-    for (int a = 0; a < 4; a++) {
-        const int ri = r0 + ty + 16 * a;
-#pragma unroll
-        for (int b = 0; b < 4; b++) {
-            const int cl = c0 + tx + 16 * b;
-            if (ri < n && cl <= ri && cl < col_end) {
-                cx<double>& e = A[(int64_t)ri * n + cl];
-                e = mk(e.re - accr[a][b], e.im - acci[a][b]);
+            for (int u = q; u < 4; u++) {
+                const cx<double> y = L[8 * u + g][j];
+                a[u].re = __builtin_fma(-x.re, y.re, __builtin_fma(-x.im, y.im, a[u].re));
+                a[u].im = __builtin_fma(-x.im, y.re, __builtin_fma(x.re, y.im, a[u].im));
             }
         }
+    // the wavefronts' first bad pivots; the smallest is the block's
+    __shared__ int bads[4];
+    if ((threadIdx.x & 63) == 0) bads[wave] = bad;
+    __syncthreads();
+    if (threadIdx.x == 0 && *info == 0) {
+        int b = 0;
+        for (int w = 0; w < 4; w++)
+            if (bads[w] && (!b || bads[w] < b)) b = bads[w];
+        if (b) *info = b;
+    }
+    for (int t = threadIdx.x; t < NB * NB; t += 256) {
+        const int r = t / NB, l = t % NB;
+        if (k0 + r < n && l <= r) A[(int64_t)(k0 + r) * n + k0 + l] = L[r][l];
+    }
+}
+
+// ROWS x 32 rows of X solve X L^H = X in place (LDS), thread (i, g) as above in
+// rows i, i + 32, ...; rd = 1 / diagonal.  Each x_j gets its terms in the order
+// of a sequential substitution.
+template <int ROWS>
+RBM_DI void trsm32(const cx<double> (*L)[CLD], const double* rd, cx<double> (*X)[CLD]) {
+    const int i = threadIdx.x & 31, g = threadIdx.x >> 5;
+    cx<double> a[ROWS][4];
+#pragma unroll
+    for (int p = 0; p < ROWS; p++)
+#pragma unroll
+        for (int q = 0; q < 4; q++) a[p][q] = X[32 * p + i][8 * q + g];
+#pragma unroll
+    for (int q = 0; q < 4; q++)
+#pragma unroll 1
+        for (int gj = 0; gj < 8; gj++) {
+            const int j = 8 * q + gj;
+            if (g == gj) {
+                const double r = rd[j];
+#pragma unroll
+                for (int p = 0; p < ROWS; p++) X[32 * p + i][j] = mk(a[p][q].re * r, a[p][q].im * r);
+            }
+            __syncthreads();
+            cx<double> y[4];
+#pragma unroll
+            for (int u = q; u < 4; u++) y[u] = L[8 * u + g][j];
+#pragma unroll
+            for (int p = 0; p < ROWS; p++) {
+                const cx<double> x = X[32 * p + i][j];
+#pragma unroll
+                for (int u = q; u < 4; u++) {
+                    a[p][u].re = __builtin_fma(-x.re, y[u].re, __builtin_fma(-x.im, y[u].im, a[p][u].re));
+                    a[p][u].im = __builtin_fma(-x.im, y[u].re, __builtin_fma(x.re, y[u].im, a[p][u].im));
+                }
+            }
+        }
+    __syncthreads();
+}
+
+// Column panel c .. c + 31 (its diagonal block factored): rows below solve
+// X L_cc^H = A, and the rest of the block column, columns c + 32 .. bend,
+// subtracts X X^H.  A workgroup has 32 rows and solves for itself the up to 96
+// rows of the block column's diagonal block that its update needs, all in one
+// sweep of 32 steps; the update is FP64 MFMA, a wavefront 16 rows by
+// half the columns.  Those shared
+// rows live in D (CB x CB, the diagonal block at K0), where every workgroup may
+// read the unsolved columns c .. c + 31 while their owner writes solved ones to
+// A.  Workgroup 0, when the next diagonal block is in this block column, updates
+// and factors that block alone.
+//
+// 5328 x 5328: 19 us a panel, a chain of barriers and LDS round trips (34 with a
+// launch each for factor, solve by 32 lanes a row, and update).
+__global__ __launch_bounds__(256) void k_chol_panel(int n, int c, int K0, int bend, cx<double>* __restrict__ A,
+                                                    cx<double>* __restrict__ D, int* __restrict__ info) {
+    __shared__ cx<double> X[NB + CB - NB][CLD];   // own rows, then the shared ones
+    __shared__ cx<double> Lc[NB][CLD];
+    __shared__ double rdiag[NB];
+    cx<double>(*Xo)[CLD] = X, (*Xt)[CLD] = X + NB;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int c1 = c + NB, nt = bend - c1;
+    const bool has_next = nt > 0;
+    const bool next = has_next && blockIdx.x == 0;
+    const int r0 = next ? c1 : c1 + NB * ((int)blockIdx.x - (has_next ? 1 : 0));
+    const int l = tid & 31;
+    const int passes = has_next ? CB / 8 : NB / 8;
+#pragma unroll 16
+    for (int u = 0; u < passes; u++) {   // 8 rows at a time
+        const int s = 8 * u + (tid >> 5), r = u < NB / 8 ? r0 + s : c1 + s - NB;
+        const bool live = u < NB / 8 ? r < n : r < bend;
+        const doublex2 v = load2(live && r >= bend ? A + (int64_t)r * n + c + l : D + (live ? r - K0 : 0) * CB + (c - K0) + l);
+        store2(&X[s][l], live ? v : doublex2{0.0, 0.0});
+    }
+#pragma unroll
+    for (int u = 0; u < 4; u++) {
+        const int i = 8 * u + (tid >> 5);
+        const doublex2 v = load2(A + (int64_t)(c + i) * n + c + (l <= i ? l : i));
+        store2(&Lc[i][l], l <= i ? v : doublex2{0.0, 0.0});
+        if (i == l) rdiag[i] = 1.0 / Lc[i][i].re;
+    }
+    __syncthreads();
+    if (next || !has_next) trsm32<1>(Lc, rdiag, X);
+    else trsm32<CB / NB>(Lc, rdiag, X);
+    const int row = lane & 15, kq = lane >> 4;
+    if (next) {
+        const int ti = 16 * (wave >> 1), tj = 16 * (wave & 1);
+        doublex4 re{0., 0., 0., 0.}, im{0., 0., 0., 0.};
+        doublex2 d[4];
+#pragma unroll
+        for (int v = 0; v < 4; v++) d[v] = load2(D + (c1 + ti + kq + 4 * v - K0) * CB + (c1 + tj + row - K0));
+#pragma unroll
+        for (int k = 0; k < NB; k += 4) mfma_herk(re, im, Xo[ti + row][k + kq], Xo[tj + row][k + kq]);
+#pragma unroll
+        for (int v = 0; v < 4; v++) {
+            const int i = ti + kq + 4 * v, l = tj + row;
+            cx<double> e = mk(i == l ? 1.0 : 0.0, 0.0);
+            if (c1 + i < bend && l <= i) e = mk(d[v][0] - re[v], d[v][1] - im[v]);
+            Xt[i][l] = e;
+        }
+        __syncthreads();
+        potrf_store(n, c1, Xt, A, info);
+        return;
+    }
+    for (int t = tid; t < NB * NB; t += 256) {
+        const int i = t / NB, l = t % NB;
+        if (r0 + i < n) store2(A + (int64_t)(r0 + i) * n + c + l, load2(&Xo[i][l]));
+    }
+    if (!has_next) return;
+    constexpr int BT = (CB - NB) / 32;
+    const int ti = 16 * (wave & 1), tj = 16 * BT * (wave >> 1);
+    const int i0 = r0 + ti + kq, l0 = c1 + tj + row;
+    doublex2 e[BT][4];   // on their way during the products
+#pragma unroll
+    for (int b = 0; b < BT; b++)
+#pragma unroll
+        for (int v = 0; v < 4; v++) {
+            const int i = i0 + 4 * v, l = l0 + 16 * b;
+            const bool own = i < n && l <= i && l < bend;
+            e[b][v] = load2(own && i >= bend ? A + (int64_t)i * n + l : D + (own ? (i - K0) * CB + (l - K0) : 0));
+        }
+    doublex4 re[BT], im[BT];
+#pragma unroll
+    for (int b = 0; b < BT; b++) re[b] = im[b] = doublex4{0., 0., 0., 0.};
+#pragma unroll 2
+    for (int k = 0; k < NB; k += 4) {
+        const cx<double> xi = Xo[ti + row][k + kq];
+#pragma unroll
+        for (int b = 0; b < BT; b++)
+            if (tj + 16 * b < nt) mfma_herk(re[b], im[b], xi, Xt[tj + 16 * b + row][k + kq]);
+    }
+#pragma unroll
+    for (int b = 0; b < BT; b++)
+#pragma unroll
+        for (int v = 0; v < 4; v++) {
+            const int i = i0 + 4 * v, l = l0 + 16 * b;
+            if (i >= n || l > i || l >= bend || i < c1 + NB) continue;   // the next diagonal block is workgroup 0's
+            store2(i < bend ? D + (i - K0) * CB + (l - K0) : A + (int64_t)i * n + l,
+                   e[b][v] - doublex2{re[b][v], im[b][v]});
+        }
+}
+
+// Trailing update A_il -= X_i X_l^H by the CB columns from kc (kc < 0: none), rows
+// i >= columns l >= base, one 64 x 64 tile of the lower triangle per workgroup:
+// FP64 MFMA, 32 x 32 a wavefront, 16 columns at a time through LDS with the next
+// 16 on their way.  The next block column's diagonal block, rows below bend, goes
+// to D, except its first 32 x 32, which workgroup 0 updates alone and factors
+// while the others work.
+// Above 32 rows of tiles (then the block column, 4 MiB, outgrows a die's L2)
+// squares of 4 x 4 tiles go to one die, the dies in turn along a row of squares.
+// n = 5328: 4.4 ms a factorisation, 51 TFLOP/s for the largest update (of 78.6)
+// falling with its size; as 64 x 64 tiles on the vector units 8.6.
+constexpr int TR_K = 16, TR_LD = TR_K + 1;
+__global__ __launch_bounds__(256, 3) void k_chol_trail(int n, int kc, int base, int bend, int tiles, int group,
+                                                       cx<double>* __restrict__ A,
+                                                    cx<double>* __restrict__ D, int* __restrict__ info) {
+    __shared__ cx<double> P[2][64][TR_LD];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int row = lane & 15, kq = lane >> 4;
+    if (blockIdx.x == 0) {
+        const int ti = 16 * (wave >> 1), tj = 16 * (wave & 1);
+        doublex4 re{0., 0., 0., 0.}, im{0., 0., 0., 0.};
+        doublex2 d[4];
+#pragma unroll
+        for (int v = 0; v < 4; v++) {
+            const int i = ti + kq + 4 * v, l = tj + row;
+            d[v] = load2(A + (base + i < n && l <= i ? (int64_t)(base + i) * n + base + l : 0));
+        }
+        if (kc >= 0) {
+            const cx<double>* xi = A + (int64_t)(base + ti + row < n ? base + ti + row : n - 1) * n + kc + kq;
+            const cx<double>* xj = A + (int64_t)(base + tj + row < n ? base + tj + row : n - 1) * n + kc + kq;
+#pragma unroll 8
+            for (int k = 0; k < CB; k += 4) mfma_herk(re, im, xi[k], xj[k]);
+        }
+        cx<double>(*L)[CLD] = reinterpret_cast<cx<double>(*)[CLD]>(&P[0][0][0]);
+#pragma unroll
+        for (int v = 0; v < 4; v++) {
+            const int i = ti + kq + 4 * v, l = tj + row;
+            cx<double> e = mk(i == l ? 1.0 : 0.0, 0.0);
+            if (base + i < n && l <= i) e = mk(d[v][0] - re[v], d[v][1] - im[v]);
+            L[i][l] = e;
+        }
+        __syncthreads();
+        potrf_store(n, base, L, A, info);
+        return;
+    }
+    int t = (int)blockIdx.x - 1, sub = 0;
+    if (group > 1) {
+        const int per = group * group, seq = t / 8;
+        sub = seq % per;
+        t = seq / per * 8 + t % 8;
+    }
+    int bi = (int)((sqrt(8.0 * t + 1.0) - 1.0) * 0.5);
+    while ((bi + 1) * (bi + 2) / 2 <= t) bi++;
+    while (bi * (bi + 1) / 2 > t) bi--;
+    const int bj = group * (t - bi * (bi + 1) / 2) + sub % group;
+    bi = group * bi + sub / group;
+    if (bj > bi || bi >= tiles) return;
+    const int r0 = base + 64 * bi, c0 = base + 64 * bj;
+    doublex4 re[2][2], im[2][2];
+#pragma unroll
+    for (int a = 0; a < 2; a++)
+#pragma unroll
+        for (int b = 0; b < 2; b++) re[a][b] = im[a][b] = doublex4{0., 0., 0., 0.};
+    if (kc >= 0) {
+        const int k = tid & 15, ri = tid >> 4;
+        const cx<double>*src[2][4];
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+            const int i = r0 + ri + 16 * u, l = c0 + ri + 16 * u;
+            src[0][u] = A + (int64_t)(i < n ? i : n - 1) * n + kc + k;
+            src[1][u] = A + (int64_t)(l < n ? l : n - 1) * n + kc + k;
+        }
+        doublex2 f[2][4];
+#pragma unroll
+        for (int o = 0; o < 2; o++)
+#pragma unroll
+            for (int u = 0; u < 4; u++) f[o][u] = load2(src[o][u]);
+        const int wr = 32 * (wave >> 1), wc = 32 * (wave & 1);
+        for (int k0 = 0; k0 < CB; k0 += TR_K) {
+            __syncthreads();
+#pragma unroll
+            for (int o = 0; o < 2; o++)
+#pragma unroll
+                for (int u = 0; u < 4; u++) store2(&P[o][ri + 16 * u][k], f[o][u]);
+            __syncthreads();
+            const int kn = k0 + TR_K < CB ? k0 + TR_K : 0;   // without a branch, which would make each load wait
+#pragma unroll
+            for (int o = 0; o < 2; o++)
+#pragma unroll
+                for (int u = 0; u < 4; u++) f[o][u] = load2(src[o][u] + kn);
+#pragma unroll
+            for (int kk = 0; kk < TR_K; kk += 4) {
+                cx<double> x[2], y[2];
+#pragma unroll
+                for (int a = 0; a < 2; a++) x[a] = P[0][wr + 16 * a + row][kk + kq];
+#pragma unroll
+                for (int b = 0; b < 2; b++) y[b] = P[1][wc + 16 * b + row][kk + kq];
+#pragma unroll
+                for (int a = 0; a < 2; a++)
+#pragma unroll
+                    for (int b = 0; b < 2; b++) mfma_herk(re[a][b], im[a][b], x[a], y[b]);
+            }
+        }
+    }
+    // eight loads in flight: one at a time the sixteen round trips of a tile cost
+    // as much as its products
+#pragma unroll
+    for (int a = 0; a < 2; a++) {
+        const int i0 = r0 + 32 * (wave >> 1) + 16 * a + kq, l0 = c0 + 32 * (wave & 1) + row;
+        doublex2 e[2][4];
+#pragma unroll
+        for (int b = 0; b < 2; b++)
+#pragma unroll
+            for (int v = 0; v < 4; v++) {
+                const int i = i0 + 4 * v, l = l0 + 16 * b;
+                // in the lower triangle, and not in workgroup 0's block
+                const bool own = i < n && l <= i && i >= base + NB;
+                e[b][v] = load2(A + (own ? (int64_t)i * n + l : 0));
+            }
+#pragma unroll
+        for (int b = 0; b < 2; b++)
+#pragma unroll
+            for (int v = 0; v < 4; v++) {
+                const int i = i0 + 4 * v, l = l0 + 16 * b;
+                if (i >= n || l > i || i < base + NB) continue;
+                store2(i < bend ? D + (i - base) * CB + (l - base) : A + (int64_t)i * n + l,
+                       e[b][v] - doublex2{re[a][b][v], im[a][b][v]});
+            }
     }
 }
 
@@ -286,127 +497,245 @@ hipError_t launch_gemm_tn_splitk(int ldx, int ldy, int64_t K, int splits, const 
     return hipGetLastError();
 }
 
-// Two-level blocking: block columns of NB2 = 128 are factored panel by panel
-// (NB = 32), each panel's update confined to the rest of its block column;
-// then one rank-128 update covers the trailing matrix, which is read and
-// written once per 128 columns instead of once per 32.
-constexpr int NB2 = 128;
-hipError_t launch_cholesky(int n, cx<double>* A, int* info, hipStream_t stream) {
-    for (int K0 = 0; K0 < n; K0 += NB2) {
-        const int bend = n - K0 < NB2 ? n : K0 + NB2;
-        for (int c = K0; c < bend; c += NB) {
-            const int nb = n - c < NB ? n - c : NB;
-            hipLaunchKernelGGL(k_potrf_diag, dim3(1), dim3(NB * NB), 0, stream, n, c, A, info);
-            const int rest = n - c - nb;
-            if (rest <= 0) break;
-            hipLaunchKernelGGL(k_trsm_panel, dim3((unsigned)((rest + 7) / 8)), dim3(256), 0, stream, n, c, A);
-            const int base = c + nb;
-            if (base < bend) {
-                const int ct = (bend - base + HT - 1) / HT, rt = (n - base + HT - 1) / HT;
-                hipLaunchKernelGGL(k_herk_update, dim3((unsigned)ct, (unsigned)rt), dim3(256), 0, stream, n, c, nb,
-                                   base, bend, ct, A);
-            }
-        }
-        const int rest = n - bend;
-        if (rest <= 0) break;
-        const int tiles = (rest + HT - 1) / HT;
-        hipLaunchKernelGGL(k_herk_update, dim3((unsigned)(tiles * (tiles + 1) / 2)), dim3(256), 0, stream, n, K0,
-                           bend - K0, bend, n, 0, A);
+hipError_t launch_cholesky(int n, cx<double>* A, cx<double>* D, int* info, hipStream_t stream) {
+    for (int K0 = 0; K0 < n; K0 += CB) {
+        const int bend = n - K0 < CB ? n : K0 + CB;
+        // the first block column only takes its diagonal block over
+        const int tiles = ((K0 ? n : bend) - K0 + 63) / 64;
+        const int group = tiles > 32 ? 4 : 1, rows = (tiles + group - 1) / group, squares = rows * (rows + 1) / 2;
+        const int blocks = group > 1 ? (squares + 7) / 8 * 8 * group * group : squares;
+        hipLaunchKernelGGL(k_chol_trail, dim3((unsigned)(1 + blocks)), dim3(256), 0, stream, n, K0 ? K0 - CB : -1, K0,
+                           bend, tiles, group, A, D, info);
+        for (int c = K0; c < bend && c + NB < n; c += NB)
+            hipLaunchKernelGGL(k_chol_panel, dim3((unsigned)((n - c - 1) / NB + (c + NB < bend ? 1 : 0))), dim3(256),
+                               0, stream, n, c, K0, bend, A, D, info);
     }
     return hipGetLastError();
 }
 
-// Blocked substitution over all CUs.  Per diagonal block k0 (NB rows):
-//   k_trsv_block   one wavefront solves the block with its 32 x 32 factor,
-//                  one lane per row
-//                  (forward: y_b = L_bb^{-1} x_b; backward: x_b = L_bb^{-H} y_b)
-//   k_trsv_update  the rows outside the block subtract the block's products,
-//                  one wavefront per row pair with coalesced row reads
-//                  (forward: rows below, x_i -= L_ib y_b; backward: rows above,
-//                  x_i -= sum_m conj(L_mi) x_m over the block's rows m).
-__global__ __launch_bounds__(64) void k_trsv_block(int n, int k0, int backward, const cx<double>* __restrict__ A,
-                                                   cx<double>* __restrict__ x) {
-    // lane j < nb holds x_j; at step m the finished x_m is broadcast and the
-    // lanes still to finish subtract its term (forward: L_jm x_m for j > m;
-    // backward: conj(L_mj) x_m for j < m)
-    __shared__ cx<double> Lb[NB][NB + 1];
-    const int nb = n - k0 < NB ? n - k0 : NB;
-    for (int t = threadIdx.x; t < NB * NB; t += 64) {
-        const int i = t / NB, l = t % NB;
-        Lb[i][l] = (i < nb && l < nb && l <= i) ? A[(int64_t)(k0 + i) * n + k0 + l] : mk(0.0, 0.0);
+// Blocked substitution, one launch per block of CB: the rows outside the solved
+// blocks subtract the products of the block solved last (p0 ..; p0 < 0: none),
+// and workgroup 0, which has the next block (k0 ..), then solves that.  Its
+// triangle is in LDS by the time its right-hand side is complete, and wavefront
+// s solves 32 rows with its part of the triangle in registers: a launch of its
+// own for each 32 rows' solve and another for their update took 5.1 ms for
+// n = 5328, this 2.1, most of it the chain through workgroup 0.
+// The triangle is packed by rows; rows past the matrix are the identity.
+RBM_DI int tri(int i, int l) { return i * (i + 1) / 2 + l; }
+constexpr int TRI = CB * (CB + 1) / 2;
+constexpr int TRSV_LDS = (TRI + 4 * CB) * (int)sizeof(cx<double>);
+
+RBM_DI void trsv_load(int n, int k0, const cx<double>* __restrict__ A, cx<double>* Ls) {
+    const int lane = threadIdx.x & 63, wave = (threadIdx.x >> 6) & 3;
+#pragma unroll 16
+    for (int i = wave; i < CB; i += 4) {
+        const int r = k0 + i < n ? k0 + i : n - 1;   // columns stay within row r: l <= i
+        const cx<double>* a = A + (int64_t)r * n + k0;
+        const int l0 = lane < r - k0 ? lane : r - k0, l1 = lane + 64 < r - k0 ? lane + 64 : r - k0;
+        const doublex2 v0 = load2(a + l0), v1 = load2(a + l1);
+        const bool in = k0 + i < n;
+        if (lane <= i) store2(Ls + tri(i, lane), in ? v0 : doublex2{i == lane ? 1.0 : 0.0, 0.0});
+        if (lane + 64 <= i) store2(Ls + tri(i, lane + 64), in ? v1 : doublex2{i == lane + 64 ? 1.0 : 0.0, 0.0});
     }
-    __syncthreads();
-    const int j = threadIdx.x;
-    cx<double> v = j < nb ? x[k0 + j] : mk(0.0, 0.0);
-    if (!backward) {
-        for (int m = 0; m < nb; m++) {
-            if (j == m) {
-                const double r = 1.0 / Lb[m][m].re;
-                v = mk(v.re * r, v.im * r);
-            }
-            const cx<double> y = lane_bcast(v, m);
-            if (j > m && j < nb) {
-                const cx<double> L = Lb[j][m];
-                v = mk(v.re - (L.re * y.re - L.im * y.im), v.im - (L.re * y.im + L.im * y.re));
-            }
-        }
-    } else {
-        for (int m = nb - 1; m >= 0; m--) {
-            if (j == m) {
-                const double r = 1.0 / Lb[m][m].re;
-                v = mk(v.re * r, v.im * r);
-            }
-            const cx<double> y = lane_bcast(v, m);
-            if (j < m) {
-                const cx<double> u = cmul_conj(y, Lb[m][j]);
-                v = mk(v.re - u.re, v.im - u.im);
-            }
-        }
-    }
-    if (j < nb) x[k0 + j] = v;
 }
 
-__global__ __launch_bounds__(256) void k_trsv_update(int n, int k0, int backward, const cx<double>* __restrict__ A,
-                                                     cx<double>* __restrict__ x) {
-    __shared__ cx<double> xb[NB];
-    const int nb = n - k0 < NB ? n - k0 : NB;
-    if (threadIdx.x < NB) xb[threadIdx.x] = threadIdx.x < nb ? x[k0 + threadIdx.x] : mk(0.0, 0.0);
-    __syncthreads();
-    const int lane = threadIdx.x & 31, half = threadIdx.x >> 5;   // 8 rows per workgroup, 32 lanes per row
-    const int64_t row = (int64_t)blockIdx.x * 8 + half;
-    // forward: rows k0 + nb .. n-1; backward: rows 0 .. k0-1
-    const int64_t i = backward ? row : k0 + nb + row;
-    const bool live = backward ? row < k0 : i < n;
-    cx<double> u = mk(0.0, 0.0);
-    if (live && lane < nb) {
-        if (!backward) {
-            const cx<double> L = A[i * n + k0 + lane], y = xb[lane];
-            u = mk(L.re * y.re - L.im * y.im, L.re * y.im + L.im * y.re);
-        } else {
-            u = cmul_conj(xb[lane], A[(int64_t)(k0 + lane) * n + i]);
+// L y = x: x_i -= L_ip y_p below, then block k0
+__global__ __launch_bounds__(512) void k_trsv_forward(int n, int p0, int k0, const cx<double>* __restrict__ A,
+                                                      cx<double>* __restrict__ x) {
+    extern __shared__ cx<double> trsv_lds[];
+    cx<double>*Ls = trsv_lds, *xs = trsv_lds + TRI, *ys = xs + CB;   // block k0's triangle, its x, the solved block's y
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const bool solve = blockIdx.x == 0;
+    const bool first_half = tid < 256;   // subtracts the products, the others load the triangle
+    if (solve) {
+        if (!first_half) trsv_load(n, k0, A, Ls);
+        if (tid < CB) xs[tid] = k0 + tid < n ? x[k0 + tid] : mk(0.0, 0.0);
+    }
+    if (p0 >= 0) {
+        if (tid < CB) ys[tid] = x[p0 + tid];
+        __syncthreads();
+        // 16 lanes a row, 8 columns each
+        const int q = tid & 15, first = solve ? k0 : k0 + CB + 64 * ((int)blockIdx.x - 1);
+        for (int g = 0; first_half && g < (solve ? CB / 64 : 1); g++) {
+            doublex2 f[4][8];
+#pragma unroll
+            for (int u = 0; u < 4; u++) {
+                const int i = first + 64 * g + 16 * u + (tid >> 4);
+                const cx<double>* a = A + (int64_t)(i < n ? i : n - 1) * n + p0 + q;
+#pragma unroll
+                for (int m = 0; m < 8; m++) f[u][m] = load2(a + 16 * m);
+            }
+#pragma unroll
+            for (int u = 0; u < 4; u++) {
+                const int i = first + 64 * g + 16 * u + (tid >> 4);
+                cx<double> s = mk(0.0, 0.0);
+#pragma unroll
+                for (int m = 0; m < 8; m++) {
+                    const cx<double> y = ys[q + 16 * m];
+                    s.re = __builtin_fma(f[u][m][0], y.re, __builtin_fma(-f[u][m][1], y.im, s.re));
+                    s.im = __builtin_fma(f[u][m][0], y.im, __builtin_fma(f[u][m][1], y.re, s.im));
+                }
+                s = row_sum16(s);
+                if (q == 0 && i < n) {
+                    if (solve) xs[i - k0] = mk(xs[i - k0].re - s.re, xs[i - k0].im - s.im);
+                    else x[i] = mk(x[i].re - s.re, x[i].im - s.im);
+                }
+            }
         }
     }
-    // sum over the 32 lanes of the row (lanes 0-31 and 32-63 of a wavefront hold two rows)
+    if (!solve) return;
+    __syncthreads();
+    // rows scaled by their diagonal, so that a step is a broadcast and two FMAs
+    const int j = lane & 31;
+    const double rd = 1.0 / Ls[tri(32 * (wave & 3) + j, 32 * (wave & 3) + j)].re;
+    doublex2 L[NB];
 #pragma unroll
-    for (int off = 16; off > 0; off >>= 1) {
-        u.re += __shfl_xor(u.re, off, 32);
-        u.im += __shfl_xor(u.im, off, 32);
+    for (int m = 0; m < NB; m++) {
+        const doublex2 a = load2(Ls + tri(32 * (wave & 3) + j, 32 * (wave & 3) + (m < j ? m : 0)));
+        L[m] = m < j ? a * rd : doublex2{0.0, 0.0};
     }
-    if (live && lane == 0) x[i] = mk(x[i].re - u.re, x[i].im - u.im);
+    for (int s = 0; s < CB / NB; s++) {
+        if (wave == s) {
+            cx<double> v = mk(xs[32 * s + j].re * rd, xs[32 * s + j].im * rd);
+#pragma unroll
+            for (int m = 0; m < NB; m++) {
+                const cx<double> y = lane_bcast(v, m);
+                v.re = __builtin_fma(-L[m][0], y.re, __builtin_fma(L[m][1], y.im, v.re));
+                v.im = __builtin_fma(-L[m][0], y.im, __builtin_fma(-L[m][1], y.re, v.im));
+            }
+            if (lane < NB) xs[32 * s + j] = v;
+        }
+        __syncthreads();
+        // rows below in the block: 8 lanes a row, 4 columns each
+        for (int i = 32 * (s + 1) + (tid >> 3); i < CB; i += 64) {
+            cx<double> u = mk(0.0, 0.0);
+#pragma unroll
+            for (int m = 0; m < 4; m++) {
+                const int l = 32 * s + (tid & 7) + 8 * m;
+                const cx<double> a = Ls[tri(i, l)], y = xs[l];
+                u.re = __builtin_fma(a.re, y.re, __builtin_fma(-a.im, y.im, u.re));
+                u.im = __builtin_fma(a.re, y.im, __builtin_fma(a.im, y.re, u.im));
+            }
+#pragma unroll
+            for (int off = 4; off > 0; off >>= 1) {
+                u.re += __shfl_xor(u.re, off);
+                u.im += __shfl_xor(u.im, off);
+            }
+            if ((tid & 7) == 0) xs[i] = mk(xs[i].re - u.re, xs[i].im - u.im);
+        }
+        __syncthreads();
+    }
+    if (tid < CB && k0 + tid < n) x[k0 + tid] = xs[tid];
+}
+
+// L^H y = x: x_i -= sum_m conj(L_mi) y_m above, m over the solved block, then
+// block k0
+__global__ __launch_bounds__(512) void k_trsv_backward(int n, int p0, int k0, const cx<double>* __restrict__ A,
+                                                       cx<double>* __restrict__ x) {
+    extern __shared__ cx<double> trsv_lds[];
+    cx<double>*Ls = trsv_lds, *xs = trsv_lds + TRI, *ys = xs + CB, *ps = ys + CB;   // ps: 4 x 64 partial sums
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const bool solve = blockIdx.x == 0;
+    const bool first_half = tid < 256;   // subtracts the products, the others load the triangle
+    if (solve) {
+        if (!first_half) trsv_load(n, k0, A, Ls);
+        if (tid < CB) xs[tid] = k0 + tid < n ? x[k0 + tid] : mk(0.0, 0.0);
+    }
+    if (p0 >= 0) {
+        if (tid < CB) ys[tid] = p0 + tid < n ? x[p0 + tid] : mk(0.0, 0.0);
+        __syncthreads();
+        // a column a lane, 32 rows a wavefront
+        const int first = solve ? k0 : 64 * ((int)blockIdx.x - 1);
+        for (int g = 0; g < (solve ? CB / 64 : 1); g++) {
+            const int i = first + 64 * g + lane;
+            if (first_half) {
+                doublex2 f[NB];
+#pragma unroll
+                for (int m = 0; m < NB; m++) {
+                    const int r = p0 + 32 * wave + m;   // past the matrix: times ys = 0
+                    f[m] = load2(A + (int64_t)(r < n ? r : n - 1) * n + i);
+                }
+                cx<double> s = mk(0.0, 0.0);
+#pragma unroll
+                for (int m = 0; m < NB; m++) {
+                    const cx<double> y = ys[32 * wave + m];
+                    s.re = __builtin_fma(f[m][0], y.re, __builtin_fma(f[m][1], y.im, s.re));
+                    s.im = __builtin_fma(f[m][0], y.im, __builtin_fma(-f[m][1], y.re, s.im));
+                }
+                ps[64 * wave + lane] = s;
+            }
+            __syncthreads();
+            if (wave == 0) {
+                cx<double> t = ps[lane];
+#pragma unroll
+                for (int z = 1; z < 4; z++) t = mk(t.re + ps[64 * z + lane].re, t.im + ps[64 * z + lane].im);
+                if (solve) xs[i - k0] = mk(xs[i - k0].re - t.re, xs[i - k0].im - t.im);
+                else x[i] = mk(x[i].re - t.re, x[i].im - t.im);
+            }
+            __syncthreads();
+        }
+    }
+    if (!solve) return;
+    __syncthreads();
+    // rows scaled by their diagonal, so that a step is a broadcast and two FMAs
+    const int j = lane & 31;
+    const double rd = 1.0 / Ls[tri(32 * (wave & 3) + j, 32 * (wave & 3) + j)].re;
+    doublex2 L[NB];
+#pragma unroll
+    for (int m = 0; m < NB; m++) {
+        const doublex2 a = load2(Ls + tri(32 * (wave & 3) + m, 32 * (wave & 3) + (m > j ? j : 0)));
+        L[m] = m > j ? a * rd : doublex2{0.0, 0.0};
+    }
+    for (int s = CB / NB - 1; s >= 0; s--) {
+        if (wave == s) {
+            cx<double> v = mk(xs[32 * s + j].re * rd, xs[32 * s + j].im * rd);
+#pragma unroll
+            for (int m = NB - 1; m >= 0; m--) {
+                const cx<double> y = lane_bcast(v, m);
+                v.re = __builtin_fma(-L[m][0], y.re, __builtin_fma(-L[m][1], y.im, v.re));
+                v.im = __builtin_fma(-L[m][0], y.im, __builtin_fma(L[m][1], y.re, v.im));
+            }
+            if (lane < NB) xs[32 * s + j] = v;
+        }
+        __syncthreads();
+        // columns above in the block: four threads a column, 8 rows each
+        if (tid < 4 * 32 * s) {
+            const int i = tid >> 2;
+            cx<double> u = mk(0.0, 0.0);
+#pragma unroll
+            for (int m = 0; m < 8; m++) {
+                const int r = 32 * s + 4 * m + (tid & 3);
+                const cx<double> a = Ls[tri(r, i)], y = xs[r];
+                u.re = __builtin_fma(a.re, y.re, __builtin_fma(a.im, y.im, u.re));
+                u.im = __builtin_fma(a.re, y.im, __builtin_fma(-a.im, y.re, u.im));
+            }
+#pragma unroll
+            for (int off = 2; off > 0; off >>= 1) {
+                u.re += __shfl_xor(u.re, off);
+                u.im += __shfl_xor(u.im, off);
+            }
+            if ((tid & 3) == 0) xs[i] = mk(xs[i].re - u.re, xs[i].im - u.im);
+        }
+        __syncthreads();
+    }
+    if (tid < CB && k0 + tid < n) x[k0 + tid] = xs[tid];
 }
 
 hipError_t launch_cholesky_solve(int n, const cx<double>* L, cx<double>* x, hipStream_t stream) {
-    const int nblk = (n + NB - 1) / NB;
-    for (int kb = 0; kb < nblk; kb++) {
-        const int k0 = kb * NB, nb = n - k0 < NB ? n - k0 : NB;
-        hipLaunchKernelGGL(k_trsv_block, dim3(1), dim3(64), 0, stream, n, k0, 0, L, x);
-        const int rest = n - k0 - nb;
-        if (rest > 0) hipLaunchKernelGGL(k_trsv_update, dim3((unsigned)((rest + 7) / 8)), dim3(256), 0, stream, n, k0, 0, L, x);
+    for (const void* f : {(const void*)&k_trsv_forward, (const void*)&k_trsv_backward}) {
+        const hipError_t e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, TRSV_LDS);
+        if (e != hipSuccess) return e;
     }
-    for (int kb = nblk - 1; kb >= 0; kb--) {
-        const int k0 = kb * NB;
-        hipLaunchKernelGGL(k_trsv_block, dim3(1), dim3(64), 0, stream, n, k0, 1, L, x);
-        if (k0 > 0) hipLaunchKernelGGL(k_trsv_update, dim3((unsigned)((k0 + 7) / 8)), dim3(256), 0, stream, n, k0, 1, L, x);
+    const int nblk = (n + CB - 1) / CB;
+    for (int b = 0; b < nblk; b++) {
+        const int k0 = b * CB, rest = b ? n - k0 - CB : 0;
+        hipLaunchKernelGGL(k_trsv_forward, dim3((unsigned)(1 + (rest > 0 ? (rest + 63) / 64 : 0))), dim3(512), TRSV_LDS,
+                           stream, n, b ? k0 - CB : -1, k0, L, x);
+    }
+    for (int b = nblk - 1; b >= 0; b--) {
+        const int k0 = b * CB;
+        hipLaunchKernelGGL(k_trsv_backward, dim3((unsigned)(1 + (b < nblk - 1 ? k0 / 64 : 0))), dim3(512), TRSV_LDS, stream,
+                           n, b < nblk - 1 ? k0 + CB : -1, k0, L, x);
     }
     return hipGetLastError();
 }

@@ -12,7 +12,9 @@ namespace rbmhip {
 
 // A = L L^H in place (lower triangle); *info (zeroed by the caller) receives
 // the 1-based index of the first non-positive pivot, 0 if none.
-hipError_t launch_cholesky(int n, cx<double>* A, int* info, hipStream_t stream);
+// (D: CHOL_WORK elements of scratch)
+constexpr int CHOL_WORK = 128 * 128;
+hipError_t launch_cholesky(int n, cx<double>* A, cx<double>* D, int* info, hipStream_t stream);
 // x <- (L L^H)^{-1} x with the factor from launch_cholesky
 hipError_t launch_cholesky_solve(int n, const cx<double>* L, cx<double>* x, hipStream_t stream);
 // C += A^T A on the lower 128 x 128 tiles of the FP64 matrix C (ld x ld) for
