@@ -1305,21 +1305,38 @@ struct Scalars {
     double v[SC_STRIDE];
 };
 
-static Scalars reduce_scalars(Ctx& c, int64_t n, const double* sc) {
-    int nb = (int)std::min<int64_t>(1024, (n + 255) / 256);
-    if (nb < 1) nb = 1;
-    double* part = reinterpret_cast<double*>(c.buf("scpart", (size_t)nb * SC_STRIDE * sizeof(double)));
-    c.launch("scalar_reduce", [&] { return launch_scalar_partials(n, sc, nb, part, c.stream); });
-    std::vector<double> h((size_t)nb * SC_STRIDE);
-    c.d2h(h.data(), part, h.size() * sizeof(double));
-    c.sync();
-    Scalars r;
-    for (int q = 0; q < SC_STRIDE; q++) {
-        double s = 0.0;
-        for (int b = 0; b < nb; b++) s += h[(size_t)b * SC_STRIDE + q];
-        r.v[q] = s;
+// Sums of the scalar terms over the samples, as the workgroups' partial sums:
+// left on the device for k_coef, and on their way to the host, where total()
+// adds them up after a wait.
+struct ScalarSums {
+    const double* dev = nullptr;
+    int blocks = 0;
+    std::vector<double> host;
+    Scalars total() const {
+        Scalars r;
+        for (int q = 0; q < SC_STRIDE; q++) {
+            double s = 0.0;
+            for (int b = 0; b < blocks; b++) s += host[(size_t)b * SC_STRIDE + q];
+            r.v[q] = s;
+        }
+        return r;
     }
-    return r;
+};
+
+static void scalar_sums(Ctx& c, const CoefArgs& a, ScalarSums& r) {
+    r.blocks = (int)std::max<int64_t>(1, std::min<int64_t>(SC_BLOCKS, (a.n + 255) / 256));
+    double* part = reinterpret_cast<double*>(c.buf("scpart", (size_t)r.blocks * SC_STRIDE * sizeof(double)));
+    c.launch("scalar_reduce", [&] { return launch_scalar_sums(a, r.blocks, part, c.stream); });
+    r.dev = part;
+    r.host.resize((size_t)r.blocks * SC_STRIDE);
+    c.d2h(r.host.data(), part, r.host.size() * sizeof(double));
+}
+
+static Scalars reduce_scalars(Ctx& c, const CoefArgs& a) {
+    ScalarSums r;
+    scalar_sums(c, a, r);
+    c.sync();
+    return r.total();
 }
 
 // R[r][col] = sum_s coef[s] row_r(s) conj(col(s)) for the RBM rows
@@ -1509,15 +1526,29 @@ static void with_precision(int precision, F&& f) {
 static void check_psi(const rbmhip_psi* p) { RBM_REQUIRE(p != nullptr, "null wavefunction handle"); }
 static void check_ens(const rbmhip_ens* e) { RBM_REQUIRE(e != nullptr, "null ensemble handle"); }
 
-template <typename T>
-static Scalars energy_scalars(Ctx& c, rbmhip_psi* psi, const Samples& s, rbmhip_ens* ens, cx<double>* coef) {
-    double* sc = reinterpret_cast<double*>(c.buf("sc", (size_t)s.n * SC_STRIDE * sizeof(double)));
+static CoefArgs energy_args(const rbmhip_psi* psi, const Samples& s, const rbmhip_ens* ens) {
     CoefArgs a;
     std::memset(&a, 0, sizeof(a));
     a.n = s.n; a.mode = 0; a.exact = ens->kind == 0; a.num_configs = (double)ens->num_configs; a.mult = s.mult;
-    a.log_prefactor = std::log(psi->prefactor); a.lp = s.lp; a.el = s.el; a.coef = coef; a.sc = sc;
+    a.log_prefactor = std::log(psi->prefactor); a.lp = s.lp; a.el = s.el;
+    return a;
+}
+
+static Scalars energy_scalars(Ctx& c, rbmhip_psi* psi, const Samples& s, rbmhip_ens* ens) {
+    return reduce_scalars(c, energy_args(psi, s, ens));
+}
+
+// The scalar sums of a (mode 0 or 1) and, from them, the coefficients of mode
+// `centred` (2 or 3), with no wait between; returns coef.
+static const cx<double>* centred_coef(Ctx& c, CoefArgs a, int centred, double n, cx<double>* coef, ScalarSums& sums) {
+    scalar_sums(c, a, sums);
+    a.mode = centred;
+    a.coef = coef;
+    a.sums = sums.dev;
+    a.n_sums = sums.blocks;
+    a.n_steps = n;
     c.launch("coef", [&] { return launch_coef(a, c.stream); });
-    return reduce_scalars(c, s.n, sc);
+    return coef;
 }
 
 // Allocation-free local energies: rbmhip_local_energy with every device
@@ -2286,7 +2317,7 @@ int rbmhip_expectation(rbmhip_psi* psi, rbmhip_op* op, rbmhip_ens* ens, double* 
         with_precision(psi->precision, [&](auto tag) {
             using T = decltype(tag);
             Samples s = sample<T>(c, psi, op, ens, false, false);
-            Scalars r = energy_scalars<T>(c, psi, s, ens, nullptr);
+            Scalars r = energy_scalars(c, psi, s, ens);
             const double inv = 1.0 / (double)ens->num_steps();
             out[0] = r.v[1] * inv;
             out[1] = r.v[2] * inv;
@@ -2316,7 +2347,7 @@ int rbmhip_expectation_list(rbmhip_psi* psi, rbmhip_op* const* ops, int n_ops, r
                 eval_model<T>(c, psi, ops[i], s.n, configs, 0, rec);
                 Samples si = s;
                 si.el = el;
-                Scalars r = energy_scalars<T>(c, psi, si, ens, nullptr);
+                Scalars r = energy_scalars(c, psi, si, ens);
                 out[2 * i] = r.v[1] * inv;
                 out[2 * i + 1] = r.v[2] * inv;
             }
@@ -2333,7 +2364,7 @@ int rbmhip_fluctuation(rbmhip_psi* psi, rbmhip_op* op, rbmhip_ens* ens, double* 
         with_precision(psi->precision, [&](auto tag) {
             using T = decltype(tag);
             Samples s = sample<T>(c, psi, op, ens, false, false);
-            Scalars r = energy_scalars<T>(c, psi, s, ens, nullptr);
+            Scalars r = energy_scalars(c, psi, s, ens);
             const double inv = 1.0 / (double)ens->num_steps();
             const double Er = r.v[1] * inv, Ei = r.v[2] * inv, E2 = r.v[3] * inv;
             expectation[0] = Er;
@@ -2403,11 +2434,12 @@ static int gradient_impl(rbmhip_psi* psi, rbmhip_op* op, rbmhip_ens* ens, int es
         with_precision(psi->precision, [&](auto tag) {
             using T = decltype(tag);
             Samples s = sample<T>(c, psi, op, ens, true, true);
-            Scalars r = energy_scalars<T>(c, psi, s, ens, nullptr);
             const int64_t P = psi->num_params();
             const double n = (double)ens->num_steps();
-            const cd E(r.v[1] / n, r.v[2] / n);
+            CoefArgs a = energy_args(psi, s, ens);
             if (use_ek) {
+                const Scalars r = reduce_scalars(c, a);
+                const cd E(r.v[1] / n, r.v[2] / n);
                 const std::vector<cd> R = gradient_ek_sums<T>(c, psi, op, ens, s, cd(1, 0), -2.0 * E, cd(0, 0), cd(1, 0));
                 for (int64_t k = 0; k < P; k++) {
                     const cd g = R[(size_t)k] / n;
@@ -2421,13 +2453,11 @@ static int gradient_impl(rbmhip_psi* psi, rbmhip_op* op, rbmhip_ens* ens, int es
             // ExpectationValue.cu:243-253 with conj<E_k> = <E conj(O_k)> (Hermitian):
             // g_k = 2 <E conj O_k> - 2 <E> conj<O_k> = (2/n) sum_s w (E - <E>) conj(O_k)
             cx<double>* coef = reinterpret_cast<cx<double>*>(c.buf("coef", (size_t)s.n * sizeof(cx<double>)));
-            CoefArgs a;
-            std::memset(&a, 0, sizeof(a));
-            a.n = s.n; a.mode = 2; a.exact = ens->kind == 0; a.num_configs = (double)ens->num_configs; a.mult = s.mult;
-            a.log_prefactor = std::log(psi->prefactor); a.lp = s.lp; a.el = s.el; a.coef = coef;
-            a.e_mean = mk(E.real(), E.imag());
-            c.launch("coef", [&] { return launch_coef(a, c.stream); });
-            std::vector<cd> R = contract_params<T>(c, psi, s.n, s.tanh, s.spins, coef);
+            ScalarSums sums;
+            const cx<double>* ready = centred_coef(c, a, 2, n, coef, sums);
+            std::vector<cd> R = contract_params<T>(c, psi, s.n, s.tanh, s.spins, ready);
+            const Scalars r = sums.total();
+            const cd E(r.v[1] / n, r.v[2] / n);
             for (int64_t k = 0; k < P; k++) {
                 const cd g = (2.0 / n) * R[(size_t)k];
                 grad[2 * k] = g.real();
@@ -2461,7 +2491,7 @@ int rbmhip_fluctuation_gradient(rbmhip_psi* psi, rbmhip_op* op, rbmhip_ens* ens,
         with_precision(psi->precision, [&](auto tag) {
             using T = decltype(tag);
             Samples s = sample<T>(c, psi, op, ens, true, true);
-            Scalars r = energy_scalars<T>(c, psi, s, ens, nullptr);
+            Scalars r = energy_scalars(c, psi, s, ens);
             const int64_t P = psi->num_params();
             const double n = (double)ens->num_steps();
             const cd E(r.v[1] / n, r.v[2] / n);
@@ -2490,13 +2520,11 @@ int rbmhip_corrected(rbmhip_psi* psi, rbmhip_op* op, rbmhip_op* op2, rbmhip_ens*
         with_precision(psi->precision, [&](auto tag) {
             using T = decltype(tag);
             Samples s = sample<T>(c, psi, op, ens, false, false);
-            double* sc = reinterpret_cast<double*>(c.buf("sc", (size_t)s.n * SC_STRIDE * sizeof(double)));
             CoefArgs a;
             std::memset(&a, 0, sizeof(a));
             a.n = s.n; a.mode = 6; a.exact = ens->kind == 0; a.num_configs = (double)ens->num_configs; a.mult = s.mult;
-            a.log_prefactor = std::log(psi->prefactor); a.lp = s.lp; a.el = s.el; a.sc = sc;
-            c.launch("coef", [&] { return launch_coef(a, c.stream); });
-            Scalars r = reduce_scalars(c, s.n, sc);
+            a.log_prefactor = std::log(psi->prefactor); a.lp = s.lp; a.el = s.el;
+            Scalars r = reduce_scalars(c, a);
             const double n = (double)ens->num_steps();
             const cd A(r.v[0] / n, r.v[1] / n);
             const double X = r.v[2] / n;
@@ -2529,7 +2557,6 @@ int rbmhip_difference(rbmhip_psi* psi, rbmhip_psi* psi_prime, rbmhip_op* const* 
         cx<double>* lp2 = reinterpret_cast<cx<double>*>(c.buf("lp2", (size_t)s.n * sizeof(cx<double>)));
         cx<double>* el = reinterpret_cast<cx<double>*>(c.buf("diff_el", (size_t)s.n * sizeof(cx<double>)));
         cx<double>* el2 = reinterpret_cast<cx<double>*>(c.buf("diff_el2", (size_t)s.n * sizeof(cx<double>)));
-        double* sc = reinterpret_cast<double*>(c.buf("sc", (size_t)s.n * SC_STRIDE * sizeof(double)));
         with_precision(psi_prime->precision, [&](auto tag) {
             using T = decltype(tag);
             Records rec{nullptr, lp2, nullptr, nullptr};
@@ -2538,11 +2565,10 @@ int rbmhip_difference(rbmhip_psi* psi, rbmhip_psi* psi_prime, rbmhip_op* const* 
         CoefArgs a;
         std::memset(&a, 0, sizeof(a));
         a.n = s.n; a.exact = ens->kind == 0; a.num_configs = (double)ens->num_configs; a.mult = s.mult;
-        a.log_prefactor = std::log(psi->prefactor); a.lp = s.lp; a.lp2 = lp2; a.sc = sc;
+        a.log_prefactor = std::log(psi->prefactor); a.lp = s.lp; a.lp2 = lp2;
         a.mode = 8;
-        c.launch("coef", [&] { return launch_coef(a, c.stream); });
         const double n = (double)ens->num_steps();
-        const double ravg = reduce_scalars(c, s.n, sc).v[0] / n;
+        const double ravg = reduce_scalars(c, a).v[0] / n;
         for (int i = 0; i < n_ops; i++) {
             with_precision(psi->precision, [&](auto tag) {
                 using T = decltype(tag);
@@ -2555,8 +2581,7 @@ int rbmhip_difference(rbmhip_psi* psi, rbmhip_psi* psi_prime, rbmhip_op* const* 
                 eval_model<T>(c, psi_prime, ops[i], s.n, configs, 0, rec);
             });
             a.mode = 7; a.el = el; a.el2 = el2;
-            c.launch("coef", [&] { return launch_coef(a, c.stream); });
-            Scalars r = reduce_scalars(c, s.n, sc);
+            Scalars r = reduce_scalars(c, a);
             const cd av(r.v[0] / n, r.v[1] / n), bv(r.v[2] / n, r.v[3] / n);
             const cd d = av - bv / ravg;
             out[2 * i] = d.real();
@@ -2642,20 +2667,16 @@ int rbmhip_sr_update(rbmhip_psi* psi, rbmhip_op* op, rbmhip_ens* ens, double eps
         with_precision(psi->precision, [&](auto tag) {
             using T = decltype(tag);
             Samples s = sample<T>(c, psi, op, ens, true, true);
-            Scalars r = energy_scalars<T>(c, psi, s, ens, nullptr);
             const int64_t Pall = psi->num_params();
             const int N = psi->N;
             const int P = (int)(Pall - 2 * (int64_t)N);
             const double n = (double)ens->num_steps();
-            const cd E(r.v[1] / n, r.v[2] / n);
             cx<double>* coef = reinterpret_cast<cx<double>*>(c.buf("coef", (size_t)s.n * sizeof(cx<double>)));
-            CoefArgs a;
-            std::memset(&a, 0, sizeof(a));
-            a.n = s.n; a.mode = 2; a.exact = ens->kind == 0; a.num_configs = (double)ens->num_configs; a.mult = s.mult;
-            a.log_prefactor = std::log(psi->prefactor); a.lp = s.lp; a.el = s.el; a.coef = coef;
-            a.e_mean = mk(E.real(), E.imag());
-            c.launch("coef", [&] { return launch_coef(a, c.stream); });
-            const std::vector<cd> R = contract_params<T>(c, psi, s.n, s.tanh, s.spins, coef);
+            ScalarSums sums;
+            const cx<double>* ready = centred_coef(c, energy_args(psi, s, ens), 2, n, coef, sums);
+            const std::vector<cd> R = contract_params<T>(c, psi, s.n, s.tanh, s.spins, ready);
+            const Scalars r = sums.total();
+            const cd E(r.v[1] / n, r.v[2] / n);
             std::vector<cd> g((size_t)P);
             for (int k = 0; k < P; k++) g[(size_t)k] = (2.0 / n) * R[(size_t)(2 * N + k)];
             cx<double>* S = s_matrix_centred<T>(c, psi, ens, s, eps);
@@ -2765,15 +2786,29 @@ static int hs_distance_impl(rbmhip_psi* psi, rbmhip_psi* psi_prime, rbmhip_op* o
             }
             c.launch("axis_log_psi", [&] { return launch_axis_log_psi(s.n, N, configs, 0, axis_dev, lp2, flip_r, c.stream); });
         }
-        double* sc = reinterpret_cast<double*>(c.buf("sc", (size_t)s.n * SC_STRIDE * sizeof(double)));
         CoefArgs a;
         std::memset(&a, 0, sizeof(a));
         a.n = s.n; a.mode = 1; a.exact = ens->kind == 0; a.is_unitary = is_unitary ? 1 : 0; a.mult = s.mult;
         a.num_configs = (double)ens->num_configs; a.log_prefactor = std::log(psi->prefactor);
-        a.lp = s.lp; a.el = s.el; a.lp2 = lp2; a.sc = sc;
-        c.launch("coef", [&] { return launch_coef(a, c.stream); });
-        Scalars r = reduce_scalars(c, s.n, sc);
+        a.lp = s.lp; a.el = s.el; a.lp2 = lp2;
         const double n = (double)ens->num_steps();
+        ScalarSums sums;
+        cx<double>* coef = nullptr;
+        std::vector<cd> R;
+        if (want_grad) {
+            // g_k = -(conj(w) <w O*> v - u n <r O*>) / v^2 / d^nu
+            //     = -conj(w) n_avg / (n v^2 d^nu) * sum_s w (r_avg omega - omega_avg r) conj(O_k)
+            coef = reinterpret_cast<cx<double>*>(c.buf("coef", (size_t)s.n * sizeof(cx<double>)));
+            centred_coef(c, a, 3, n, coef, sums);
+            with_precision(psi_prime->precision, [&](auto tag) {
+                using T = decltype(tag);
+                R = contract_params<T>(c, psi_prime, s.n, tanh2, spins_for_grad, coef);
+            });
+        } else {
+            scalar_sums(c, a, sums);
+            c.sync();
+        }
+        const Scalars r = sums.total();
         const cd omega(r.v[0] / n, r.v[1] / n);
         const double ratio = r.v[2] / n, nrm = r.v[3] / n;
         // HilbertSpaceDistance.cu:216-220, 248-262
@@ -2782,18 +2817,6 @@ static int hs_distance_impl(rbmhip_psi* psi, rbmhip_psi* psi_prime, rbmhip_op* o
         const double d = std::sqrt(1.0 - u / v);
         *distance = d;
         if (want_grad) {
-            // g_k = -(conj(w) <w O*> v - u n <r O*>) / v^2 / d^nu
-            //     = -conj(w) n_avg / (n v^2 d^nu) * sum_s w (r_avg omega - omega_avg r) conj(O_k)
-            cx<double>* coef = reinterpret_cast<cx<double>*>(c.buf("coef", (size_t)s.n * sizeof(cx<double>)));
-            a.mode = 3; a.coef = coef; a.sc = nullptr;
-            a.omega_mean = mk(omega.real(), omega.imag());
-            a.ratio_mean = ratio;
-            c.launch("coef", [&] { return launch_coef(a, c.stream); });
-            std::vector<cd> R;
-            with_precision(psi_prime->precision, [&](auto tag) {
-                using T = decltype(tag);
-                R = contract_params<T>(c, psi_prime, s.n, tanh2, spins_for_grad, coef);
-            });
             if (axis) {
                 const int slices = (int)std::max<int64_t>(1, std::min<int64_t>(256, s.n / 4096));
                 cx<double>* part = reinterpret_cast<cx<double>*>(c.buf("axis_part", (size_t)slices * 2 * N * sizeof(cx<double>)));

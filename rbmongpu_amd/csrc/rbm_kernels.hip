@@ -3,7 +3,7 @@
 //   k_eval_rbm  log psi / E_loc / tanh(theta) for given configurations
 //               (ExactSummation, psi_vector, psi_O_k_vector, batched calls)
 //   k_ok_reduce + k_partials_sum   FP64 O_k contractions
-//   k_coef, k_scalar_partials, k_lse_partials   per-sample FP64 reductions
+//   k_coef, k_scalar_sums, k_lse_partials   per-sample FP64 reductions
 //
 // Execution model: a chain (or a basis state) is owned by a 16-lane DPP row;
 // a wavefront holds four chains and a 256-thread workgroup sixteen.  Hidden
@@ -445,68 +445,114 @@ __global__ __launch_bounds__(256) void k_eval_rbm(RbmDev<T> md, OpDev op, int ha
 //   mode 1 (distance): HilbertSpaceDistance.cu:83-105 with log psi' in lp2:
 //     coef0 = w omega, coef1 = w ratio; sc = {w omega, w ratio, w norm}
 // ---------------------------------------------------------------------------
+// Weight of sample s
+RBM_DI double coef_weight(const CoefArgs& a, int64_t s, double lp_re) {
+    return a.mult ? a.mult[s] : a.exact ? a.num_configs * exp(2.0 * (a.log_prefactor + lp_re)) : 1.0;
+}
+
+// Modes 1 and 3: the distance's overlap and norm of one sample
+RBM_DI void distance_terms(const CoefArgs& a, cx<double> lp, cx<double> lpp, cx<double> E, cx<double>& omega, double& ratio,
+                           double& nrm) {
+    const cx<double> dl = conj(lpp - lp);
+    if (a.is_unitary) {
+        omega = cexp(dl) * E;
+        nrm = E.re * E.re + E.im * E.im;
+    } else {
+        omega = cexp(E + dl);
+        nrm = exp(2.0 * E.re);
+    }
+    ratio = exp(2.0 * (lpp.re - lp.re));
+}
+
+// Scalar terms of one sample (modes 0, 1, 6, 7, 8)
+RBM_DI void scalar_terms(const CoefArgs& a, int64_t s, double* v) {
+    const cx<double> lp = a.lp[s];
+    const double w = coef_weight(a, s, lp.re);
+    const cx<double> E = a.el ? a.el[s] : mk(0.0, 0.0);
+    if (a.mode == 6) {
+        // ExpectationValue.cu:100-110: X = exp(2 Im E + Re(E^2 - E))
+        const cx<double> q = E * E - E;
+        v[0] = w * E.re; v[1] = w * E.im; v[2] = w * exp(2.0 * E.im + q.re); v[3] = 0.0;
+    } else if (a.mode == 7 || a.mode == 8) {
+        // ExpectationValue.cu:392-412: r = |psi / psi'|^2 on samples of psi
+        const double r = exp(2.0 * (lp.re - a.lp2[s].re));
+        if (a.mode == 8) {
+            v[0] = w * r; v[1] = 0.0; v[2] = 0.0; v[3] = 0.0;
+        } else {
+            const cx<double> Ep = a.el2[s];
+            v[0] = w * Ep.re; v[1] = w * Ep.im; v[2] = w * r * E.re; v[3] = w * r * E.im;
+        }
+    } else if (a.mode == 0) {
+        v[0] = w; v[1] = w * E.re; v[2] = w * E.im; v[3] = w * (E.re * E.re + E.im * E.im);
+    } else {
+        cx<double> omega;
+        double ratio, nrm;
+        distance_terms(a, lp, a.lp2[s], E, omega, ratio, nrm);
+        v[0] = w * omega.re; v[1] = w * omega.im; v[2] = w * ratio; v[3] = w * nrm;
+    }
+}
+
+// partials[b] = sums of the scalar terms over workgroup b's samples.  A small
+// ensemble's call is made of launches and waits (norm and gradient of N = 10, all
+// 1024 states, FP32: 87 us, 30 of them in kernels), so the terms are summed where
+// they are formed and k_coef finishes the sums by itself, without a wait on the
+// host between: 74 us.
+__global__ __launch_bounds__(256) void k_scalar_sums(CoefArgs a, double* __restrict__ partials) {
+    __shared__ double red[SC_STRIDE][256];
+    double acc[SC_STRIDE], v[SC_STRIDE];
+#pragma unroll
+    for (int q = 0; q < SC_STRIDE; q++) acc[q] = 0.0;
+    for (int64_t s = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; s < a.n; s += (int64_t)gridDim.x * blockDim.x) {
+        scalar_terms(a, s, v);
+#pragma unroll
+        for (int q = 0; q < SC_STRIDE; q++) acc[q] += v[q];
+    }
+#pragma unroll
+    for (int q = 0; q < SC_STRIDE; q++) red[q][threadIdx.x] = acc[q];
+    __syncthreads();
+    for (int w = 128; w > 0; w >>= 1) {
+        if ((int)threadIdx.x < w)
+#pragma unroll
+            for (int q = 0; q < SC_STRIDE; q++) red[q][threadIdx.x] += red[q][threadIdx.x + w];
+        __syncthreads();
+    }
+    if (threadIdx.x < SC_STRIDE) partials[blockIdx.x * SC_STRIDE + threadIdx.x] = red[threadIdx.x][0];
+}
+
+// Per-sample coefficients (modes 2 .. 5).  Modes 2 and 3 subtract means: every
+// workgroup adds up the partial sums, at most SC_BLOCKS of them, in their order.
 __global__ __launch_bounds__(256) void k_coef(CoefArgs a) {
+    __shared__ double part[SC_BLOCKS * SC_STRIDE], mean[SC_STRIDE];
+    if (a.mode == 2 || a.mode == 3) {
+        for (int k = threadIdx.x; k < a.n_sums * SC_STRIDE; k += blockDim.x) part[k] = a.sums[k];
+        __syncthreads();
+        if (threadIdx.x < SC_STRIDE) {
+            double sum = 0.0;
+#pragma unroll 8
+            for (int b = 0; b < a.n_sums; b++) sum += part[b * SC_STRIDE + threadIdx.x];
+            mean[threadIdx.x] = sum / a.n_steps;
+        }
+        __syncthreads();
+    }
     for (int64_t s = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; s < a.n; s += (int64_t)gridDim.x * blockDim.x) {
         const cx<double> lp = a.lp[s];
-        const double w = a.mult ? a.mult[s] : a.exact ? a.num_configs * exp(2.0 * (a.log_prefactor + lp.re)) : 1.0;
+        const double w = coef_weight(a, s, lp.re);
         const cx<double> E = a.el ? a.el[s] : mk(0.0, 0.0);
         if (a.mode == 4) {
             // the weight itself: sum_s coef conj(O_k) = n <conj O_k>
             a.coef[s] = mk(w, 0.0);
-            continue;
-        }
-        if (a.mode == 5) {
+        } else if (a.mode == 5) {
             a.coef[s] = w * (a.alpha * E + a.e_mean);
-            continue;
-        }
-        if (a.mode == 6) {
-            // ExpectationValue.cu:100-110: X = exp(2 Im E + Re(E^2 - E))
-            double* sc = a.sc + s * SC_STRIDE;
-            const cx<double> q = E * E - E;
-            sc[0] = w * E.re; sc[1] = w * E.im; sc[2] = w * exp(2.0 * E.im + q.re); sc[3] = 0.0;
-            continue;
-        }
-        if (a.mode == 7 || a.mode == 8) {
-            // ExpectationValue.cu:392-412: r = |psi / psi'|^2 on samples of psi
-            const double r = exp(2.0 * (lp.re - a.lp2[s].re));
-            double* sc = a.sc + s * SC_STRIDE;
-            if (a.mode == 8) {
-                sc[0] = w * r; sc[1] = 0.0; sc[2] = 0.0; sc[3] = 0.0;
-            } else {
-                const cx<double> Ep = a.el2[s];
-                sc[0] = w * Ep.re; sc[1] = w * Ep.im; sc[2] = w * r * E.re; sc[3] = w * r * E.im;
-            }
-            continue;
-        }
-        if (a.mode == 0 || a.mode == 2) {
-            if (a.mode == 2) {
-                // w (E - <E>): sum_s coef conj(O_k) = n (<E conj O_k> - <E> conj<O_k>)
-                a.coef[s] = w * (E - a.e_mean);
-                continue;
-            }
-            double* sc = a.sc + s * SC_STRIDE;
-            sc[0] = w; sc[1] = w * E.re; sc[2] = w * E.im; sc[3] = w * (E.re * E.re + E.im * E.im);
+        } else if (a.mode == 2) {
+            // w (E - <E>): sum_s coef conj(O_k) = n (<E conj O_k> - <E> conj<O_k>)
+            a.coef[s] = w * (E - mk(mean[1], mean[2]));
         } else {
-            const cx<double> lpp = a.lp2[s];
-            const cx<double> dl = conj(lpp - lp);
+            // w (r_mean omega - omega_mean r): the numerator of the distance
+            // gradient in one coefficient (HilbertSpaceDistance.cu:257-262)
             cx<double> omega;
-            double nrm;
-            if (a.is_unitary) {
-                omega = cexp(dl) * E;
-                nrm = E.re * E.re + E.im * E.im;
-            } else {
-                omega = cexp(E + dl);
-                nrm = exp(2.0 * E.re);
-            }
-            const double ratio = exp(2.0 * (lpp.re - lp.re));
-            if (a.mode == 3) {
-                // w (r_mean omega - omega_mean r): the numerator of the distance
-                // gradient in one coefficient (HilbertSpaceDistance.cu:257-262)
-                a.coef[s] = w * (a.ratio_mean * omega - ratio * a.omega_mean);
-                continue;
-            }
-            double* sc = a.sc + s * SC_STRIDE;
-            sc[0] = w * omega.re; sc[1] = w * omega.im; sc[2] = w * ratio; sc[3] = w * nrm;
+            double ratio, nrm;
+            distance_terms(a, lp, a.lp2[s], E, omega, ratio, nrm);
+            a.coef[s] = w * (mean[2] * omega - ratio * mk(mean[0], mean[1]));
         }
     }
 }
@@ -633,28 +679,6 @@ __global__ __launch_bounds__(256) void k_axis_contract(int64_t n, int N, const u
         partials[(int64_t)blockIdx.y * 2 * N + i] = mk(red[0][0], red[1][0]);
         partials[(int64_t)blockIdx.y * 2 * N + N + i] = mk(red[2][0], red[3][0]);
     }
-}
-
-// Block partial sums of the SC_STRIDE scalar records, fixed order.
-__global__ __launch_bounds__(256) void k_scalar_partials(int64_t n, const double* __restrict__ sc,
-                                                         double* __restrict__ partials) {
-    __shared__ double red[SC_STRIDE][256];
-    double acc[SC_STRIDE];
-#pragma unroll
-    for (int q = 0; q < SC_STRIDE; q++) acc[q] = 0.0;
-    for (int64_t s = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; s < n; s += (int64_t)gridDim.x * blockDim.x)
-#pragma unroll
-        for (int q = 0; q < SC_STRIDE; q++) acc[q] += sc[s * SC_STRIDE + q];
-#pragma unroll
-    for (int q = 0; q < SC_STRIDE; q++) red[q][threadIdx.x] = acc[q];
-    __syncthreads();
-    for (int w = 128; w > 0; w >>= 1) {
-        if ((int)threadIdx.x < w)
-#pragma unroll
-            for (int q = 0; q < SC_STRIDE; q++) red[q][threadIdx.x] += red[q][threadIdx.x + w];
-        __syncthreads();
-    }
-    if (threadIdx.x < SC_STRIDE) partials[blockIdx.x * SC_STRIDE + threadIdx.x] = red[threadIdx.x][0];
 }
 
 // Log-sum-exp partials of x_s = 2 (log prefactor + Re log psi_s): per block
@@ -1474,6 +1498,7 @@ hipError_t launch_partials_sum(int nblocks, int64_t len, const cx<double>* parti
 }
 
 hipError_t launch_coef(const CoefArgs& a, hipStream_t stream) {
+    if ((a.mode == 2 || a.mode == 3) && (!a.sums || a.n_sums < 1 || a.n_sums > SC_BLOCKS)) return hipErrorInvalidValue;
     int64_t g = (a.n + 255) / 256;
     if (g > 4096) g = 4096;
     if (g < 1) g = 1;
@@ -1527,8 +1552,9 @@ hipError_t launch_axis_contract(int64_t n, int N, const uint64_t* configs, uint6
     return hipGetLastError();
 }
 
-hipError_t launch_scalar_partials(int64_t n, const double* sc, int nblocks, double* partials, hipStream_t stream) {
-    hipLaunchKernelGGL(k_scalar_partials, dim3(nblocks), dim3(256), 0, stream, n, sc, partials);
+hipError_t launch_scalar_sums(const CoefArgs& a, int nblocks, double* partials, hipStream_t stream) {
+    if (nblocks < 1 || nblocks > SC_BLOCKS) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(k_scalar_sums, dim3(nblocks), dim3(256), 0, stream, a, partials);
     return hipGetLastError();
 }
 

@@ -70,10 +70,12 @@ constexpr int MC_RESYNC_SWEEPS = 16;
 
 constexpr int SC_STRIDE = 4;
 
+constexpr int SC_BLOCKS = 1024;   // most workgroups of k_scalar_sums
 struct CoefArgs {
     int64_t n;
-    int mode;            // 0 energy, 1 Hilbert-space distance, 2 centred energy, 3 centred distance, 4 weight,
-                         // 5 affine w (alpha E + e_mean), 6 corrected, 7 difference, 8 probability ratio
+    int mode;            // scalar terms: 0 energy, 1 Hilbert-space distance, 6 corrected, 7 difference,
+                         // 8 probability ratio; coefficients: 2 centred energy, 3 centred distance, 4 weight,
+                         // 5 affine w (alpha E + e_mean)
     int exact;           // ExactSummation weights
     const double* mult;  // per-configuration multiplicity weights (runs of equal samples), may be null
     int is_unitary;
@@ -82,13 +84,13 @@ struct CoefArgs {
     const cx<double>* lp;
     const cx<double>* el;
     const cx<double>* lp2;
-    const cx<double>* el2;  // modes 7: local energy of the second wavefunction
+    const cx<double>* el2;  // mode 7: local energy of the second wavefunction
     cx<double> alpha;       // mode 5
-    cx<double>* coef;    // n (modes 2, 3), may be null
-    double* sc;          // SC_STRIDE x n (modes 0, 1)
-    cx<double> e_mean;   // mode 2: sum w E / n
-    cx<double> omega_mean;  // mode 3
-    double ratio_mean;      // mode 3
+    cx<double> e_mean;      // mode 5
+    cx<double>* coef;       // n (modes 2 .. 5)
+    const double* sums;     // modes 2, 3: the partial sums of modes 0, 1, divided by n_steps
+    int n_sums;
+    double n_steps;
 };
 
 int max_hidden_units();
@@ -156,7 +158,7 @@ hipError_t launch_axis_log_psi(int64_t n, int N, const uint64_t* configs, uint64
 hipError_t launch_axis_contract(int64_t n, int N, const uint64_t* configs, uint64_t index_base, const double* axis,
                                 const cx<double>* r, const cx<double>* coef, int slices, cx<double>* partials,
                                 hipStream_t stream);
-hipError_t launch_scalar_partials(int64_t n, const double* sc, int nblocks, double* partials, hipStream_t stream);
+hipError_t launch_scalar_sums(const CoefArgs& a, int nblocks, double* partials, hipStream_t stream);
 hipError_t launch_lse_partials(int64_t n, const cx<double>* lp, double log_prefactor, int nblocks, double* partials,
                                hipStream_t stream);
 hipError_t launch_activation(int64_t n, const cx<double>* z, cx<double>* out, int deriv, hipStream_t stream);
