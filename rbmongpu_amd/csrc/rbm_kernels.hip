@@ -520,18 +520,22 @@ __global__ __launch_bounds__(256) void k_scalar_sums(CoefArgs a, double* __restr
 }
 
 // Per-sample coefficients (modes 2 .. 5).  Modes 2 and 3 subtract means: every
-// workgroup adds up the partial sums, at most SC_BLOCKS of them, in their order.
+// workgroup adds up the partial sums, 64 threads a term (one thread a term over
+// 1024 of them took as long as the coefficients of 300 000 samples).
 __global__ __launch_bounds__(256) void k_coef(CoefArgs a) {
-    __shared__ double part[SC_BLOCKS * SC_STRIDE], mean[SC_STRIDE];
+    __shared__ double mean[64][SC_STRIDE];
     if (a.mode == 2 || a.mode == 3) {
-        for (int k = threadIdx.x; k < a.n_sums * SC_STRIDE; k += blockDim.x) part[k] = a.sums[k];
-        __syncthreads();
-        if (threadIdx.x < SC_STRIDE) {
-            double sum = 0.0;
+        const int q = threadIdx.x % SC_STRIDE, z = threadIdx.x / SC_STRIDE;
+        double sum = 0.0;
 #pragma unroll 8
-            for (int b = 0; b < a.n_sums; b++) sum += part[b * SC_STRIDE + threadIdx.x];
-            mean[threadIdx.x] = sum / a.n_steps;
+        for (int b = z; b < a.n_sums; b += 64) sum += a.sums[b * SC_STRIDE + q];
+        mean[z][q] = sum;
+        __syncthreads();
+        for (int w = 32; w > 0; w >>= 1) {
+            if (z < w) mean[z][q] += mean[z + w][q];
+            __syncthreads();
         }
+        if (z == 0) mean[0][q] /= a.n_steps;
         __syncthreads();
     }
     for (int64_t s = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; s < a.n; s += (int64_t)gridDim.x * blockDim.x) {
@@ -545,14 +549,14 @@ __global__ __launch_bounds__(256) void k_coef(CoefArgs a) {
             a.coef[s] = w * (a.alpha * E + a.e_mean);
         } else if (a.mode == 2) {
             // w (E - <E>): sum_s coef conj(O_k) = n (<E conj O_k> - <E> conj<O_k>)
-            a.coef[s] = w * (E - mk(mean[1], mean[2]));
+            a.coef[s] = w * (E - mk(mean[0][1], mean[0][2]));
         } else {
             // w (r_mean omega - omega_mean r): the numerator of the distance
             // gradient in one coefficient (HilbertSpaceDistance.cu:257-262)
             cx<double> omega;
             double ratio, nrm;
             distance_terms(a, lp, a.lp2[s], E, omega, ratio, nrm);
-            a.coef[s] = w * (mean[2] * omega - ratio * mk(mean[0], mean[1]));
+            a.coef[s] = w * (mean[0][2] * omega - ratio * mk(mean[0][0], mean[0][1]));
         }
     }
 }
