@@ -1507,7 +1507,7 @@ static std::vector<cd> contract_params(Ctx& c, rbmhip_psi* psi, int64_t n, const
         nb = std::min<int64_t>(nb, std::max<int64_t>(1, (cur + 63) / 64));
         const int64_t chunk = (cur + nb - 1) / nb;
         cx<double>* part = reinterpret_cast<cx<double>*>(c.buf("okpart", (size_t)(nb * K) * sizeof(cx<double>)));
-        c.launch("ok_reduce", [&] { return launch_rows_reduce<T>(cur, K, rows, coef + s0, 1, chunk, (int)nb, part, c.stream); });
+        c.launch("ok_reduce", [&] { return launch_rows_reduce<T>(cur, K, rows, coef + s0, chunk, (int)nb, part, c.stream); });
         c.launch("partials_sum", [&] { return launch_partials_sum((int)nb, K, part, out, c.stream); });
         c.d2h(h.data(), out, h.size() * sizeof(cx<double>));
         c.sync();

@@ -48,7 +48,7 @@ hipError_t launch_deep_mc(const DeepDev<T>& md, const OpDev& op, int has_op, con
                           uint32_t* counts, hipStream_t stream);
 // R[q][k] = sum_s coef_q[s] conj(O[s][k]) over materialised O rows (K per sample)
 template <typename T>
-hipError_t launch_rows_reduce(int64_t n, int64_t K, const void* O, const cx<double>* coef, int nc, int64_t chunk,
+hipError_t launch_rows_reduce(int64_t n, int64_t K, const void* O, const cx<double>* coef, int64_t chunk,
                               int nblocks, cx<double>* partials, hipStream_t stream);
 // PsiDeep as dense BF16 MFMA layers (deep_mfma.hip).  Layer l has in_p[l]
 // inputs (padded to 32; layer 0's inputs are the spins) and out_p[l] units
