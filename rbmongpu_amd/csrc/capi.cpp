@@ -162,7 +162,8 @@ struct Ctx {
     // Pinned staging for copies between the host's arrays and the device.  A
     // copy from or to pageable memory goes through the runtime's own staging
     // and blocks (10-20 us each, and an exact gradient of 10 spins makes 8); a
-    // copy of at most STAGE_COPY bytes goes through this buffer instead and is
+    // copy of at most STAGE_COPY bytes goes through this buffer instead, by a
+    // kernel (launch_copy), and is
     // ordered by the stream alone: h2d takes its bytes at once, d2h delivers
     // them at the next sync().  The buffer is used from its start again after
     // each sync(); when it is full, and for larger copies, the runtime's path
@@ -188,6 +189,10 @@ struct Ctx {
         if (at + bytes > STAGE_BYTES) return nullptr;
         stage_used = at + bytes;
         return stage + at;
+    }
+    void stage_copy(void* dst, const void* src, size_t bytes, hipMemcpyKind kind) {
+        if (((uintptr_t)dst | (uintptr_t)src) & 15u) RBM_HIPCHK(hipMemcpyAsync(dst, src, bytes, kind, stream));
+        else RBM_HIPCHK(launch_copy(dst, src, bytes, stream));
     }
     // Forgets what a call that failed half-way left in the staging buffer.
     void stage_reset() {
@@ -216,7 +221,7 @@ struct Ctx {
 
     void d2h(void* dst, const void* src, size_t bytes) {
         if (void* s = stage_take(bytes)) {
-            RBM_HIPCHK(hipMemcpyAsync(s, src, bytes, hipMemcpyDeviceToHost, stream));
+            stage_copy(s, src, bytes, hipMemcpyDeviceToHost);
             deliveries.push_back({dst, s, bytes});
             return;
         }
@@ -225,7 +230,7 @@ struct Ctx {
     void h2d(void* dst, const void* src, size_t bytes) {
         if (void* s = stage_take(bytes)) {
             std::memcpy(s, src, bytes);
-            RBM_HIPCHK(hipMemcpyAsync(dst, s, bytes, hipMemcpyHostToDevice, stream));
+            stage_copy(dst, s, bytes, hipMemcpyHostToDevice);
             return;
         }
         RBM_HIPCHK(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, stream));
@@ -236,7 +241,7 @@ struct Ctx {
         if (n == 0) return;
         if (void* s = stage_take(n * sizeof(V))) {
             fill(reinterpret_cast<V*>(s));
-            RBM_HIPCHK(hipMemcpyAsync(dst, s, n * sizeof(V), hipMemcpyHostToDevice, stream));
+            stage_copy(dst, s, n * sizeof(V), hipMemcpyHostToDevice);
             return;
         }
         std::vector<V> h(n);

@@ -158,6 +158,8 @@ hipError_t launch_axis_log_psi(int64_t n, int N, const uint64_t* configs, uint64
 hipError_t launch_axis_contract(int64_t n, int N, const uint64_t* configs, uint64_t index_base, const double* axis,
                                 const cx<double>* r, const cx<double>* coef, int slices, cx<double>* partials,
                                 hipStream_t stream);
+// bytes between device and pinned host memory, both 16-byte aligned
+hipError_t launch_copy(void* dst, const void* src, size_t bytes, hipStream_t stream);
 hipError_t launch_scalar_sums(const CoefArgs& a, int nblocks, double* partials, hipStream_t stream);
 hipError_t launch_lse_partials(int64_t n, const cx<double>* lp, double log_prefactor, int nblocks, double* partials,
                                hipStream_t stream);
