@@ -162,8 +162,7 @@ struct Ctx {
     // Pinned staging for copies between the host's arrays and the device.  A
     // copy from or to pageable memory goes through the runtime's own staging
     // and blocks (10-20 us each, and an exact gradient of 10 spins makes 8); a
-    // copy of at most STAGE_COPY bytes goes through this buffer instead, by a
-    // kernel (launch_copy), and is
+    // copy of at most STAGE_COPY bytes goes through this buffer instead and is
     // ordered by the stream alone: h2d takes its bytes at once, d2h delivers
     // them at the next sync().  The buffer is used from its start again after
     // each sync(); when it is full, and for larger copies, the runtime's path
@@ -190,8 +189,11 @@ struct Ctx {
         stage_used = at + bytes;
         return stage + at;
     }
+    // Up to 16 KiB the runtime's pinned copy is the cheaper by 0.5 us, above it
+    // costs 10 us more than the kernel (log psi of 1024 configurations 19.4 against
+    // 20.0 us, of 1353 29.6 against 20.7).
     void stage_copy(void* dst, const void* src, size_t bytes, hipMemcpyKind kind) {
-        if (((uintptr_t)dst | (uintptr_t)src) & 15u) RBM_HIPCHK(hipMemcpyAsync(dst, src, bytes, kind, stream));
+        if (bytes <= 16384 || (((uintptr_t)dst | (uintptr_t)src) & 15u)) RBM_HIPCHK(hipMemcpyAsync(dst, src, bytes, kind, stream));
         else RBM_HIPCHK(launch_copy(dst, src, bytes, stream));
     }
     // Forgets what a call that failed half-way left in the staging buffer.
