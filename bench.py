@@ -611,7 +611,7 @@ def run_j1j2_deep(args, R, HAM, F):
 
 def run_heisenberg6x6_sr(args, R, HAM, F):
     """6x6 Heisenberg, RBM M = 144: one stochastic-reconfiguration step
-    (sampling, E_loc, O_k, gradient, centred S on FP32 MFMA with FP64
+    (sampling, E_loc, O_k, gradient, centred S on BF16 MFMA with FP64
     accumulation, FP64 Cholesky solve of S + 1e-4 I).  Errors of S, the
     gradient and the update are stated against an FP64 recomputation from the
     same samples of a 2048-chain ensemble (8192 samples)."""
@@ -640,12 +640,12 @@ def run_heisenberg6x6_sr(args, R, HAM, F):
     P = M + N * M
     n = CH * spc
     gram_ms, gram_n = kms["s_gram"]
-    flop = F.s_matrix_flops(P, n)
-    # the Gram product runs every FP32 product as six bfloat16 part products
-    # on the matrix cores: priced as those products against the BF16 peak,
-    # with the FP32-equivalent rate beside it
+    flop = F.pair_moment_flops(N, M, n)
+    # the moments' products of exact signs with FP32 values run as three
+    # bfloat16 part products on the matrix cores: priced as those products
+    # against the BF16 peak, with the FP32-equivalent rate beside it
     fp32_equiv = flop / (gram_ms / args.steps / 1e3) / 1e12
-    achieved = 6 * fp32_equiv
+    achieved = 3 * fp32_equiv
     # FP64 recomputation on the samples of one 2048-chain call with 4 samples
     # per chain: 8192 samples, more than the P parameters with an O_k, so
     # S + eps I is not rank-deficient
@@ -686,18 +686,17 @@ def run_heisenberg6x6_sr(args, R, HAM, F):
         "data": "synthetic (seeded N(0, 0.01^2) RBM parameters)",
         "config": {"workload": f"2-D Heisenberg 6x6 periodic (72 bonds, 216 Pauli strings), RBM M=144, {CH} chains x "
                                f"({THERM} therm + {spc} measurement sweeps), SR step with S ({P}x{P} complex) on "
-                               f"the BF16 matrix cores at FP32 accuracy (three-part split, six products) and the FP64 "
+                               f"the BF16 matrix cores at FP32 accuracy (three-part split) and the FP64 "
                                f"Cholesky solve of S + {EPS} I",
                    "chains": CH, "samples_per_chain": spc, "P": P, "eps": EPS},
         "tau_int": tau, "energy": E.real, "energy_se": se,
         "kernel_ms_per_step": {k: v[0] / max(args.steps, 1) for k, v in kms.items()},
         "roofline": {"bound": "mfma", "achieved": achieved, "peak": PEAK_BF16_TFLOPS, "unit": "TFLOP/s",
                      "frac": achieved / PEAK_BF16_TFLOPS,
-                     # HBM bytes of one Gram dispatch (one batch of 12 480 samples)
-                     "traffic": stored_traffic("k_gram_lower_bf3@heisenberg6x6-sr"),
-                     "kernel": "k_gram_lower_bf3 (S Gram, lower 128x128 tiles, FP32 products as six bfloat16 part "
-                               "products)",
-                     "flop_per_step": 6 * flop, "fp32_flop_per_step": flop, "fp32_equivalent_tflops": fp32_equiv,
+                     "traffic": stored_traffic("k_pair_moments@heisenberg6x6-sr"),
+                     "kernel": "k_pair_moments (moments of spin pairs by unit pairs, FP32 values as three bfloat16 "
+                               "parts)",
+                     "flop_per_step": 3 * flop, "fp32_flop_per_step": flop, "fp32_equivalent_tflops": fp32_equiv,
                      "ms_per_step": gram_ms / args.steps},
         "fp64_recomputation": {
             "samples": len(s), "S_rel_err": rel(S_gpu, S_ref),

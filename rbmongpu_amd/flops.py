@@ -73,11 +73,11 @@ def deep_mc_launch_flops(N, sizes, chains, proposals_per_chain):
     return chains * (proposals_per_chain + 1) * deep_forward_mfma_flops(N, sizes)
 
 
-def s_matrix_flops(P, samples):
-    """FP32 matrix-core FLOP of the centred S-matrix Gram product on real rows
-    of 2P values per sample: the symmetric product needs its lower triangle,
-    2 (2P)(2P + 1) / 2 FLOP per sample."""
-    return float(2 * P) * (2 * P + 1) * samples
+def pair_moment_flops(N, M, samples):
+    """FLOP of the moments that the centred S-matrix is assembled from: the
+    sums over the samples of 1 + N (N + 1) / 2 sign rows times the
+    (M + 1)(M + 2) / 2 complex products of two units (2 real columns each)."""
+    return 2.0 * (1 + N * (N + 1) // 2) * ((M + 1) * (M + 2)) * samples
 
 
 def cholesky_flops(n):
