@@ -494,7 +494,7 @@ RBM_DI void scalar_terms(const CoefArgs& a, int64_t s, double* v) {
 
 // partials[b] = sums of the scalar terms over workgroup b's samples.  A small
 // ensemble's call is made of launches and waits (norm and gradient of N = 10, all
-// 1024 states, FP32: 87 us, 30 of them in kernels), so the terms are summed where
+// 1024 states, FP32: 87 us, 47 of them in kernels), so the terms are summed where
 // they are formed and k_coef finishes the sums by itself, without a wait on the
 // host between: 74 us.
 __global__ __launch_bounds__(256) void k_scalar_sums(CoefArgs a, double* __restrict__ partials) {
