@@ -1659,11 +1659,11 @@ constexpr int PAIR_MIN_P = 2048;
 
 template <typename T>
 static bool s_matrix_pairs(Ctx& c, rbmhip_psi* psi, const Samples& s, double n, double eps, const cx<double>* w,
-                           const std::vector<cd>& R, int P, cx<double>* S) {
+                           bool weighted, const std::vector<cd>& R, int P, cx<double>* S) {
     const int N = psi->N, M = psi->M;
-    // R[r][j] = sum_s w row_r conj(col_j)
+    // R[r][j] = sum_s w row_r conj(col_j), R[0][M] = sum_s w
     std::vector<cx<double>> mean((size_t)M);
-    for (int j = 0; j < M; j++) mean[(size_t)j] = cxd(std::conj(R[(size_t)j]) / n);
+    for (int j = 0; j < M; j++) mean[(size_t)j] = cxd(std::conj(R[(size_t)j]) / R[(size_t)M].real());
     cx<double>* dmean = reinterpret_cast<cx<double>*>(c.buf("pair_mean", mean.size() * sizeof(cx<double>)));
     c.h2d(dmean, mean.data(), mean.size() * sizeof(cx<double>));
     const PairShape sh = pair_shape(N, M);
@@ -1684,16 +1684,22 @@ static bool s_matrix_pairs(Ctx& c, rbmhip_psi* psi, const Samples& s, double n, 
     float* units = reinterpret_cast<float*>(c.buf("pair_units", (size_t)batch * (M + 1) * 64 * sizeof(float)));
     double* C = reinterpret_cast<double*>(c.buf("pair_moments", (size_t)splits * len * sizeof(double)));
     double* ratio = reinterpret_cast<double*>(c.buf("pair_ratio", 16));
+    const int csplits = pair_const_splits(sh, M, nblk, c.num_cus);
+    const int64_t clen = csplits * pair_const_len(sh, M);
+    double* cpart = weighted ? reinterpret_cast<double*>(c.buf("pair_const", (size_t)clen * sizeof(double))) : nullptr;
     cx<double>* first = reinterpret_cast<cx<double>*>(c.buf("pair_first", (size_t)(N + 1) * (M + 1) * sizeof(cx<double>)));
     c.launch("s_matrix", [&] { return launch_zero(2 * splits * len, reinterpret_cast<float*>(C), c.stream); });
+    if (weighted) c.launch("s_matrix", [&] { return launch_zero(2 * clen, reinterpret_cast<float*>(cpart), c.stream); });
     c.launch("s_matrix", [&] { return launch_spin_planes(s.n, N, s.spins, planes, c.stream); });
     for (int64_t b0 = 0; b0 < nblk; b0 += batch) {
         const int64_t cur = std::min(batch, nblk - b0);
         c.launch("s_matrix", [&] { return launch_pair_planes(cur, N, sh.rows_p, planes + b0 * N, signs, c.stream); });
         c.launch("s_matrix", [&] { return launch_pair_units<T>(b0 * 32, s.n, cur, M, s.tanh, w, dmean, units, c.stream); });
         c.launch("s_gram", [&] { return launch_pair_moments(sh, cur, splits, M, signs, units, C, c.stream); });
+        if (weighted) c.launch("s_const", [&] { return launch_pair_const(sh, cur, csplits, M, signs, units, cpart, c.stream); });
     }
     c.launch("s_matrix", [&] { return launch_pair_finish(sh, N, M, splits, 1.0 / n, C, ratio, c.stream); });
+    if (weighted) c.launch("s_const", [&] { return launch_pair_const_sum(sh, csplits, M, cpart, C, c.stream); });
     double r = 0.0;
     c.d2h(&r, ratio, sizeof(double));
     c.sync();
@@ -1716,7 +1722,7 @@ static cx<double>* s_matrix_centred(Ctx& c, rbmhip_psi* psi, rbmhip_ens* ens, co
     c.launch("coef", [&] { return launch_coef(a, c.stream); });
     const std::vector<cd> R = ok_contract<T>(c, N, M, s.n, s.tanh, s.spins, w);
     cx<double>* S = reinterpret_cast<cx<double>*>(c.buf("s_centred", (size_t)P * P * sizeof(cx<double>)));
-    if (P >= PAIR_MIN_P && s_matrix_pairs<T>(c, psi, s, n, eps, w, R, P, S)) return S;
+    if (P >= PAIR_MIN_P && s_matrix_pairs<T>(c, psi, s, n, eps, w, a.exact || a.mult, R, P, S)) return S;
     std::vector<cd> osum;
     rbm_params_from_R(psi, R.data(), osum);
     std::vector<cx<float>> obar((size_t)P);

@@ -449,13 +449,145 @@ __global__ __launch_bounds__(256) void k_pair_first(int N, int M, int cols_p, co
     first[e] = j < M ? t + pair_moment(C, cols_p, r, M, M).re * mean[j] : t;
 }
 
-// S_kl = <conj(O_k) O_l> - conj(<O_k>) <O_l> with O_(p,j) = s_p (t_j + mean_j);
-// the upper triangle is the conjugate of the lower one
+// The columns of the constant unit, sum s_r sqrt(w) conj(t_j) and, for j = M,
+// sum s_r w, in FP64 for ensembles whose weights are not all 1.  The assembly
+// multiplies them by unit means and takes their products away again, so a
+// relative error e of them leaves e |mean|^2 in S, however small the entry.  As
+// FP32 sums of FP32-rounded weights they left 9e-5 of sqrt(S_kk S_ll) for a
+// plain state with biases around 0.5, 8e-4 at <s> = 0.999 and 0.2 at 0.9999 (12
+// spins, 170 units, exact sum), now 3e-7; the Gram product leaves 1e-6 to 6e-6.
+// Here every product is exact (two FP32 factors and a sign) and the sums are
+// FP64, of the same rounded sqrt(w) and t as the other columns, so that S is the
+// covariance of those values.  Weights of 1 don't need it: their sums are whole
+// numbers, which the FP32 sums of 4096 samples hold exactly.
+// v_mfma_f64_16x16x4f64 as below; MFMA e of a 32-sample block takes samples
+// 8 (l / 16) + e, so that a lane's 8 samples are two 16-byte words.  A wavefront
+// owns 4 row tiles and 2 column tiles of one sample split; part holds
+// splits x rows_p x cols, cols = 2 (M + 1) rounded up to 32.  36 spins, 144
+// units, 51 155 samples: 0.8 ms with the sum of the splits beside 5.5 ms of
+// k_pair_moments, 30 TFLOP/s with about one wavefront a SIMD (the Gram product
+// took 30.6 ms).
+typedef double gbf64x4 __attribute__((ext_vector_type(4)));
+constexpr int PAIRC_RT = 4, PAIRC_CT = 2;
+static int pair_const_cols(int M) { return (2 * (M + 1) + 16 * PAIRC_CT - 1) / (16 * PAIRC_CT) * (16 * PAIRC_CT); }
+
+__global__ __launch_bounds__(64) void k_pair_const(int64_t nblk, int splits, int groups, int M, int rows_p, int cols,
+                                                   const uint32_t* __restrict__ planes, const float* __restrict__ units,
+                                                   double* __restrict__ part) {
+    constexpr int RT = PAIRC_RT, CT = PAIRC_CT;
+    const int lane = threadIdx.x, kk = lane >> 4, ii = lane & 15;
+    const int col_groups = cols / (16 * CT);
+    const int grp = blockIdx.x % groups, rest = blockIdx.x / groups;
+    const int col0 = (rest % col_groups) * 16 * CT, z = rest / col_groups;
+    const int im = ii & 1;
+    int row[RT], off[CT];
+#pragma unroll
+    for (int a = 0; a < RT; a++) {
+        const int r = 16 * (grp * RT + a) + ii;
+        row[a] = r < rows_p ? r : ii;   // tiles past the last repeat the first; they are not stored
+    }
+#pragma unroll
+    for (int b = 0; b < CT; b++) {
+        const int j = (col0 + 16 * b + ii) >> 1;
+        off[b] = (j < M ? j : M) * 64 + 32 * im;
+    }
+    gbf64x4 acc[RT][CT];
+#pragma unroll
+    for (int a = 0; a < RT; a++)
+#pragma unroll
+        for (int b = 0; b < CT; b++) acc[a][b] = gbf64x4{0.0, 0.0, 0.0, 0.0};
+    const int64_t per = (nblk + splits - 1) / splits;
+    const int64_t b0 = z * per, b1 = b0 + per < nblk ? b0 + per : nblk;
+    const int64_t ustride = (int64_t)(M + 1) * 64;
+    for (int64_t blk = b0; blk < b1; blk++) {
+        const float* U = units + blk * ustride + 8 * kk;
+        float sw[8], t[CT][8];
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+            *reinterpret_cast<float4*>(sw + 4 * h) = *reinterpret_cast<const float4*>(U + M * 64 + 4 * h);
+#pragma unroll
+            for (int b = 0; b < CT; b++)
+                *reinterpret_cast<float4*>(t[b] + 4 * h) = *reinterpret_cast<const float4*>(U + off[b] + 4 * h);
+        }
+        uint32_t byte[RT];
+#pragma unroll
+        for (int a = 0; a < RT; a++) byte[a] = planes[blk * rows_p + row[a]] >> (8 * kk);
+#pragma unroll
+        for (int e = 0; e < 8; e++) {
+            double bv[CT];
+#pragma unroll
+            for (int b = 0; b < CT; b++) bv[b] = (double)sw[e] * (double)(im ? -t[b][e] : t[b][e]);
+#pragma unroll
+            for (int a = 0; a < RT; a++) {
+                const double av = (byte[a] >> e) & 1u ? 1.0 : -1.0;
+#pragma unroll
+                for (int b = 0; b < CT; b++) acc[a][b] = __builtin_amdgcn_mfma_f64_16x16x4f64(av, bv[b], acc[a][b], 0, 0, 0);
+            }
+        }
+    }
+    double* out = part + (int64_t)z * rows_p * cols;
+#pragma unroll
+    for (int a = 0; a < RT; a++) {
+        const int tile = grp * RT + a;
+        if (16 * tile >= rows_p) break;
+#pragma unroll
+        for (int b = 0; b < CT; b++)
+#pragma unroll
+            for (int v = 0; v < 4; v++) out[(int64_t)(16 * tile + kk + 4 * v) * cols + col0 + 16 * b + ii] += acc[a][b][v];
+    }
+}
+
+// The splits added in order into the constant unit's columns of C
+__global__ __launch_bounds__(256) void k_pair_const_sum(int splits, int M, int rows_p, int cols, int cols_p,
+                                                        const double* __restrict__ part, double* __restrict__ C) {
+    const int live = 2 * (M + 1);
+    const int64_t e = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+    if (e >= (int64_t)rows_p * live) return;
+    const int64_t r = e / live;
+    const int col = (int)(e % live);
+    double s = 0.0;
+    for (int z = 0; z < splits; z++) s += part[((int64_t)z * rows_p + r) * cols + col];
+    C[r * cols_p + M * (M + 1) + col] = s;
+}
+
+int64_t pair_const_len(const PairShape& s, int M) { return (int64_t)s.rows_p * pair_const_cols(M); }
+
+int pair_const_splits(const PairShape& s, int M, int64_t nblk, int num_cus) {
+    // about a wavefront per SIMD, at least 8 blocks each and at most 256 MiB of partials
+    const int64_t wp = (int64_t)((s.rows_p / 16 + PAIRC_RT - 1) / PAIRC_RT) * (pair_const_cols(M) / (16 * PAIRC_CT));
+    int64_t z = (4ll * num_cus + wp - 1) / wp;
+    if (z > nblk / 8) z = nblk / 8;
+    if (z > (256ll << 20) / (pair_const_len(s, M) * 8)) z = (256ll << 20) / (pair_const_len(s, M) * 8);
+    return z < 1 ? 1 : (int)z;
+}
+
+hipError_t launch_pair_const(const PairShape& s, int64_t nblk, int splits, int M, const uint32_t* planes, const float* units,
+                             double* part, hipStream_t stream) {
+    if (nblk <= 0 || splits < 1 || s.rows_p <= 0 || s.rows_p % 16) return hipErrorInvalidValue;
+    const int cols = pair_const_cols(M), groups = (s.rows_p / 16 + PAIRC_RT - 1) / PAIRC_RT;
+    hipLaunchKernelGGL(k_pair_const, dim3((unsigned)(groups * (cols / (16 * PAIRC_CT)) * splits)), dim3(64), 0, stream, nblk,
+                       splits, groups, M, s.rows_p, cols, planes, units, part);
+    return hipGetLastError();
+}
+
+hipError_t launch_pair_const_sum(const PairShape& s, int splits, int M, const double* part, double* C, hipStream_t stream) {
+    if (splits < 1) return hipErrorInvalidValue;
+    const int64_t len = (int64_t)s.rows_p * 2 * (M + 1);
+    hipLaunchKernelGGL(k_pair_const_sum, dim3((unsigned)((len + 255) / 256)), dim3(256), 0, stream, splits, M, s.rows_p,
+                       pair_const_cols(M), s.cols_p, part, C);
+    return hipGetLastError();
+}
+
+// S_kl = <conj(O_k - <O_k>) (O_l - <O_l>)> = <conj(O_k) O_l> - (2 - <1>)
+// conj(<O_k>) <O_l> with O_(p,j) = s_p (t_j + mean_j), averages over n and <1> =
+// sum w / n (1 where psi is normalised); the upper triangle is the conjugate of
+// the lower one
 __global__ __launch_bounds__(256) void k_pair_assemble(int N, int M, int P, int cols_p, double inv, double eps,
                                                        const cx<double>* __restrict__ mean,
                                                        const cx<double>* __restrict__ first,
                                                        const double* __restrict__ C, cx<double>* __restrict__ S) {
     const int row = blockIdx.y, WN = M + N * M;
+    const double twice = 2.0 - inv * pair_moment(C, cols_p, 0, M, M).re;
     auto spin = [&](int k) { return k < M ? 0 : k < WN ? 1 + (k - M) / M : 1 + k - WN; };
     auto unit = [&](int k) { return k < M ? k : k < WN ? (k - M) % M : M; };
     const int rp = spin(row), rj = unit(row);
@@ -470,7 +602,7 @@ __global__ __launch_bounds__(256) void k_pair_assemble(int N, int M, int P, int 
         if (jl < M) m = m + pair_moment(C, cols_p, r, j, M) * ml;
         if (j < M) m = m + mj * pair_moment(C, cols_p, r, M, jl);
         if (j < M && jl < M) m = m + pair_moment(C, cols_p, r, M, M).re * (mj * ml);
-        cx<double> v = inv * m - (inv * conj(first[p * (M + 1) + j])) * (inv * first[pl * (M + 1) + jl]);
+        cx<double> v = inv * m - (twice * inv * conj(first[p * (M + 1) + j])) * (inv * first[pl * (M + 1) + jl]);
         if (row == col) v = mk(v.re + eps, 0.0);
         S[(int64_t)row * P + col] = lower ? v : conj(v);
     }
@@ -532,7 +664,6 @@ hipError_t launch_pair_assemble(const PairShape& s, int N, int M, int P, double 
 // N = 10, M = 20 (1024 states, 240 x 240): moments, sum and assembly 30 us, where
 // one thread per entry running down all states took 608.
 // ---------------------------------------------------------------------------
-typedef double gbf64x4 __attribute__((ext_vector_type(4)));
 constexpr int PAIR64_RT_MAX = 4, PAIR64_CT = 2;
 
 template <typename T, int RT>

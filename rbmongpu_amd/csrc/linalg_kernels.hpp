@@ -48,6 +48,14 @@ hipError_t launch_pair_units(int64_t s0, int64_t n, int64_t nblk, int M, const v
 // C[z][row][col] += sum over the blocks of split z (splits equal ranges of the nblk blocks)
 hipError_t launch_pair_moments(const PairShape& s, int64_t nblk, int splits, int M, const uint32_t* planes,
                                const float* units, double* C, hipStream_t stream);
+// The constant unit's columns in FP64, for weights other than 1: part (splits x
+// pair_const_len, zeroed by the caller) += the blocks' sums, and their total into
+// C[0] after launch_pair_finish
+int64_t pair_const_len(const PairShape& s, int M);
+int pair_const_splits(const PairShape& s, int M, int64_t nblk, int num_cus);
+hipError_t launch_pair_const(const PairShape& s, int64_t nblk, int splits, int M, const uint32_t* planes, const float* units,
+                             double* part, hipStream_t stream);
+hipError_t launch_pair_const_sum(const PairShape& s, int splits, int M, const double* part, double* C, hipStream_t stream);
 // Adds the splits into C[0]; *ratio = max |<s_p t_j>|^2 / <|t_j|^2> (inv = 1 / n)
 hipError_t launch_pair_finish(const PairShape& s, int N, int M, int splits, double inv, double* C, double* ratio,
                               hipStream_t stream);
