@@ -1650,15 +1650,47 @@ static cx<double> cxd(cd z) { return mk(z.real(), z.imag()); }
 // (up to 5e-5 of it at eps = 1e-2 below a thousand parameters), so smaller
 // models, whose Gram product takes 1.7 to 4.9 ms (32 768 samples), keep it and the
 // updates they had.
-// S_kl from pairs is a difference of two sums, <conj(O_k) O_l> -
-// conj(<O_k>) <O_l>, which loses 1 / (1 - r) of the accuracy for r =
-// |<s_p t_j>|^2 / <|t_j|^2> (1 where a unit follows one spin); beyond
-// PAIR_RATIO the O_k rows are centred before the product (k_gram_lower_bf3).
-constexpr double PAIR_RATIO = 0.9;
+// S_kl from pairs is a difference of moments, whose rounding is in proportion to
+// the spreads V_j = <|T_j - <T_j>|^2> of its units, whatever is left of them in
+// the variance of O_k = s_p T_j: little where a unit follows one spin, also a
+// polarised one.  From V_j / 10 (PAIR_KEEP) the pairs are still the more accurate
+// (45 spins, 45 units: 3.6e-6 of sqrt(S_kk S_ll) against the Gram product's 7.4e-6
+// at 65 536 samples, 2.2e-6 against 3.6e-6 at 2 048; at V_j / 20 7.9e-6 against
+// 7.4e-6, 4.0e-6 against 3.4e-6); below it the O_k rows are centred before the
+// product (k_gram_lower_bf3).
+constexpr double PAIR_KEEP = 0.1;
 constexpr int PAIR_MIN_P = 2048;
 
+// Whether every O_(p,j) = s_p T_j keeps PAIR_KEEP of its unit's spread, from the
+// contraction R of the weights and sum w |T_j|^2, both in FP64: before the moments
+// are formed, so that a model that has to take the Gram product pays for that
+// alone.
 template <typename T>
-static bool s_matrix_pairs(Ctx& c, rbmhip_psi* psi, const Samples& s, double n, double eps, const cx<double>* w,
+static bool pairs_keep_accuracy(Ctx& c, int N, int M, const Samples& s, double n, const cx<double>* w,
+                                const std::vector<cd>& R) {
+    const int64_t chunk = std::max<int64_t>(64, (s.n + 1023) / 1024), nb = (s.n + chunk - 1) / chunk;
+    cx<double>* part = reinterpret_cast<cx<double>*>(c.buf("okpart", (size_t)(nb * M) * sizeof(cx<double>)));
+    cx<double>* out = reinterpret_cast<cx<double>*>(c.buf("okout", (size_t)M * sizeof(cx<double>)));
+    c.launch("s_matrix", [&] { return launch_unit_squares<T>(s.n, M, chunk, s.tanh, w, part, c.stream); });
+    c.launch("s_matrix", [&] { return launch_partials_sum((int)nb, M, part, out, c.stream); });
+    std::vector<cd> Q((size_t)M);
+    c.d2h(Q.data(), out, Q.size() * sizeof(cx<double>));
+    c.sync();
+    const double z = R[(size_t)M].real() / n;   // sum w / n
+    if (!(z > 0.0)) return false;
+    for (int j = 0; j < M; j++) {
+        const double q = Q[(size_t)j].real() / n, V = q - std::norm(R[(size_t)j]) / (n * n * z);
+        if (V <= 1e-12 * q) continue;   // constant to complex64
+        for (int p = 1; p <= N; p++) {
+            const double var = q - (2.0 - z) * std::norm(R[(size_t)p * (M + 1) + j]) / (n * n);
+            if (!(var >= PAIR_KEEP * V)) return false;
+        }
+    }
+    return true;
+}
+
+template <typename T>
+static void s_matrix_pairs(Ctx& c, rbmhip_psi* psi, const Samples& s, double n, double eps, const cx<double>* w,
                            bool weighted, const std::vector<cd>& R, int P, cx<double>* S) {
     const int N = psi->N, M = psi->M;
     // R[r][j] = sum_s w row_r conj(col_j), R[0][M] = sum_s w
@@ -1683,7 +1715,6 @@ static bool s_matrix_pairs(Ctx& c, rbmhip_psi* psi, const Samples& s, double n, 
     uint32_t* signs = reinterpret_cast<uint32_t*>(c.buf("pair_signs", (size_t)batch * sh.rows_p * sizeof(uint32_t)));
     float* units = reinterpret_cast<float*>(c.buf("pair_units", (size_t)batch * (M + 1) * 64 * sizeof(float)));
     double* C = reinterpret_cast<double*>(c.buf("pair_moments", (size_t)splits * len * sizeof(double)));
-    double* ratio = reinterpret_cast<double*>(c.buf("pair_ratio", 16));
     const int csplits = pair_const_splits(sh, M, nblk, c.num_cus);
     const int64_t clen = csplits * pair_const_len(sh, M);
     double* cpart = weighted ? reinterpret_cast<double*>(c.buf("pair_const", (size_t)clen * sizeof(double))) : nullptr;
@@ -1698,14 +1729,9 @@ static bool s_matrix_pairs(Ctx& c, rbmhip_psi* psi, const Samples& s, double n, 
         c.launch("s_gram", [&] { return launch_pair_moments(sh, cur, splits, M, signs, units, C, c.stream); });
         if (weighted) c.launch("s_const", [&] { return launch_pair_const(sh, cur, csplits, M, signs, units, cpart, c.stream); });
     }
-    c.launch("s_matrix", [&] { return launch_pair_finish(sh, N, M, splits, 1.0 / n, C, ratio, c.stream); });
+    c.launch("s_matrix", [&] { return launch_pair_sum(sh, splits, C, c.stream); });
     if (weighted) c.launch("s_const", [&] { return launch_pair_const_sum(sh, csplits, M, cpart, C, c.stream); });
-    double r = 0.0;
-    c.d2h(&r, ratio, sizeof(double));
-    c.sync();
-    if (!(r <= PAIR_RATIO)) return false;
     c.launch("s_matrix", [&] { return launch_pair_assemble(sh, N, M, P, 1.0 / n, eps, dmean, C, first, S, c.stream); });
-    return true;
 }
 
 template <typename T>
@@ -1720,11 +1746,15 @@ static cx<double>* s_matrix_centred(Ctx& c, rbmhip_psi* psi, rbmhip_ens* ens, co
     a.n = s.n; a.mode = 4; a.exact = ens->kind == 0; a.num_configs = (double)ens->num_configs; a.mult = s.mult;
     a.log_prefactor = std::log(psi->prefactor); a.lp = s.lp; a.coef = w;
     c.launch("coef", [&] { return launch_coef(a, c.stream); });
-    const std::vector<cd> R = ok_contract<T>(c, N, M, s.n, s.tanh, s.spins, w);
     cx<double>* S = reinterpret_cast<cx<double>*>(c.buf("s_centred", (size_t)P * P * sizeof(cx<double>)));
-    if (P >= PAIR_MIN_P && s_matrix_pairs<T>(c, psi, s, n, eps, w, a.exact || a.mult, R, P, S)) return S;
-    std::vector<cd> osum;
-    rbm_params_from_R(psi, R.data(), osum);
+    if (P >= PAIR_MIN_P) {
+        const std::vector<cd> R = ok_contract<T>(c, N, M, s.n, s.tanh, s.spins, w, true);
+        if (pairs_keep_accuracy<T>(c, N, M, s, n, w, R)) {
+            s_matrix_pairs<T>(c, psi, s, n, eps, w, a.exact || a.mult, R, P, S);
+            return S;
+        }
+    }
+    const std::vector<cd> osum = contract_params<T>(c, psi, s.n, s.tanh, s.spins, w);
     std::vector<cx<float>> obar((size_t)P);
     for (int k = 0; k < P; k++) {
         // the contraction gives sum_s w conj(O_k)

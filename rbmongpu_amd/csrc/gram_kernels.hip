@@ -1,7 +1,7 @@
 // The centred S of a stochastic-reconfiguration step on the bfloat16 matrix
 // cores (the reference only builds S, S_matrix.cu:10-58): second moments by
 // pairs of spins and pairs of units (k_pair_moments), and the Gram product of
-// the O_k rows (k_gram_lower_bf3) for models whose moments cancel.
+// the O_k rows (k_gram_lower_bf3) for small models and where moments cancel.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -608,41 +608,41 @@ __global__ __launch_bounds__(256) void k_pair_assemble(int N, int M, int P, int 
     }
 }
 
-// *ratio = the largest |<s_p t_j>|^2 / <|t_j|^2>: 1 where a unit follows one
-// spin, whose O_k = s_p T_j then hardly varies.  One workgroup.
-__global__ __launch_bounds__(256) void k_pair_ratio(int N, int M, int cols_p, double inv, const double* __restrict__ C,
-                                                    double* __restrict__ ratio) {
-    __shared__ double red[256];
-    double m = 0.0;
-    for (int e = threadIdx.x; e < N * M; e += 256) {
-        const int p = 1 + e / M, j = e % M;
-        const cx<double> f = pair_moment(C, cols_p, pair_row(0, p), j, M);
-        const double v = pair_moment(C, cols_p, 0, j, j).re;
-        const double r = v > 0.0 ? inv * (f.re * f.re + f.im * f.im) / v : 0.0;
-        m = r > m || r != r ? r : m;   // a NaN is kept
-    }
-    red[threadIdx.x] = m;
-    __syncthreads();
-    for (int w = 128; w > 0; w >>= 1) {
-        if ((int)threadIdx.x < w) {
-            const double a = red[threadIdx.x], b = red[threadIdx.x + w];
-            red[threadIdx.x] = b > a || b != b ? b : a;
-        }
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) *ratio = red[0];
-}
-
-hipError_t launch_pair_finish(const PairShape& s, int N, int M, int splits, double inv, double* C, double* ratio,
-                              hipStream_t stream) {
+hipError_t launch_pair_sum(const PairShape& s, int splits, double* C, hipStream_t stream) {
     const int64_t len = (int64_t)s.rows_p * s.cols_p;
-    if (splits > 1) {
-        const unsigned g = (unsigned)((len + 255) / 256 < 8192 ? (len + 255) / 256 : 8192);
-        hipLaunchKernelGGL(k_pair_sum, dim3(g), dim3(256), 0, stream, len, splits, C);
-    }
-    hipLaunchKernelGGL(k_pair_ratio, dim3(1), dim3(256), 0, stream, N, M, s.cols_p, inv, C, ratio);
+    if (splits < 2) return hipSuccess;
+    const unsigned g = (unsigned)((len + 255) / 256 < 8192 ? (len + 255) / 256 : 8192);
+    hipLaunchKernelGGL(k_pair_sum, dim3(g), dim3(256), 0, stream, len, splits, C);
     return hipGetLastError();
 }
+
+// partials[b][j] = sum over chunk b of w |T_j|^2, a thread per unit with eight
+// rows' loads in flight
+template <typename T>
+__global__ __launch_bounds__(256) void k_unit_squares(int64_t n, int M, int64_t chunk, const cx<T>* __restrict__ Trec,
+                                                      const cx<double>* __restrict__ w, cx<double>* __restrict__ partials) {
+    const int j = threadIdx.x;
+    if (j >= M) return;
+    const int64_t s0 = blockIdx.x * chunk, s1 = s0 + chunk < n ? s0 + chunk : n;
+    double q = 0.0;
+#pragma unroll 8
+    for (int64_t s = s0; s < s1; s++) {
+        const cx<double> t = to_d(Trec[s * M + j]);
+        q = fm(w[s].re, fm(t.re, t.re, t.im * t.im), q);
+    }
+    partials[(int64_t)blockIdx.x * M + j] = mk(q, 0.0);
+}
+
+template <typename T>
+hipError_t launch_unit_squares(int64_t n, int M, int64_t chunk, const void* Trec, const cx<double>* w, cx<double>* partials,
+                               hipStream_t stream) {
+    if (n <= 0 || chunk <= 0 || M <= 0 || M > 256) return hipErrorInvalidValue;
+    hipLaunchKernelGGL((k_unit_squares<T>), dim3((unsigned)((n + chunk - 1) / chunk)), dim3(256), 0, stream, n, M, chunk,
+                       reinterpret_cast<const cx<T>*>(Trec), w, partials);
+    return hipGetLastError();
+}
+template hipError_t launch_unit_squares<float>(int64_t, int, int64_t, const void*, const cx<double>*, cx<double>*, hipStream_t);
+template hipError_t launch_unit_squares<double>(int64_t, int, int64_t, const void*, const cx<double>*, cx<double>*, hipStream_t);
 
 hipError_t launch_pair_assemble(const PairShape& s, int N, int M, int P, double inv, double eps, const cx<double>* mean,
                                 const double* C, cx<double>* first, cx<double>* S, hipStream_t stream) {

@@ -50,15 +50,19 @@ hipError_t launch_pair_moments(const PairShape& s, int64_t nblk, int splits, int
                                const float* units, double* C, hipStream_t stream);
 // The constant unit's columns in FP64, for weights other than 1: part (splits x
 // pair_const_len, zeroed by the caller) += the blocks' sums, and their total into
-// C[0] after launch_pair_finish
+// C[0] after launch_pair_sum
 int64_t pair_const_len(const PairShape& s, int M);
 int pair_const_splits(const PairShape& s, int M, int64_t nblk, int num_cus);
 hipError_t launch_pair_const(const PairShape& s, int64_t nblk, int splits, int M, const uint32_t* planes, const float* units,
                              double* part, hipStream_t stream);
 hipError_t launch_pair_const_sum(const PairShape& s, int splits, int M, const double* part, double* C, hipStream_t stream);
-// Adds the splits into C[0]; *ratio = max |<s_p t_j>|^2 / <|t_j|^2> (inv = 1 / n)
-hipError_t launch_pair_finish(const PairShape& s, int N, int M, int splits, double inv, double* C, double* ratio,
-                              hipStream_t stream);
+// Adds the splits into C[0]
+hipError_t launch_pair_sum(const PairShape& s, int splits, double* C, hipStream_t stream);
+// partials[b][j] = sum of w |T_j|^2 over samples b chunk .. (M <= 256 units);
+// partials holds ceil(n / chunk) x M
+template <typename T>
+hipError_t launch_unit_squares(int64_t n, int M, int64_t chunk, const void* Trec, const cx<double>* w, cx<double>* partials,
+                               hipStream_t stream);
 // S (P x P, eps added on the diagonal) from C[0]; mean holds M values, first
 // (N + 1) x (M + 1) scratch
 hipError_t launch_pair_assemble(const PairShape& s, int N, int M, int P, double inv, double eps, const cx<double>* mean,
