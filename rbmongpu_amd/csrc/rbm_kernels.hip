@@ -748,12 +748,13 @@ __global__ __launch_bounds__(64) void k_ok_mfma_f64(int64_t n, int N, int M, con
         for (int b = 0; b < CT; b++) acc[a][b] = doublex4{0.0, 0.0, 0.0, 0.0};
     const int part = ii & 1;
     int coff[CT];
-    double cload[CT], cfix[CT];
+    bool cload[CT];
+    double cfix[CT];
 #pragma unroll
     for (int b = 0; b < CT; b++) {
         const int j = (16 * (ct0 + b) + ii) >> 1;
         coff[b] = j < M ? j : 0;               // clamped: always a valid load
-        cload[b] = j < M ? 1.0 : 0.0;          // take the loaded value
+        cload[b] = j < M;                      // take the loaded value
         cfix[b] = j == M ? 1.0 : 0.0;          // the constant column
     }
     const int64_t s_begin = chunk_id * chunk;
@@ -773,7 +774,8 @@ __global__ __launch_bounds__(64) void k_ok_mfma_f64(int64_t n, int N, int M, con
 #pragma unroll
         for (int b = 0; b < CT; b++) {
             const cx<T> t = Tr[coff[b]];
-            bv[b] = fm(p, fm((double)t.re, cload[b], cfix[b]), q * ((double)t.im * cload[b]));
+            // selected, not multiplied by zero: my_tanh overflows long before log psi
+            bv[b] = fm(p, cload[b] ? (double)t.re : cfix[b], cload[b] ? q * (double)t.im : 0.0);
         }
 #pragma unroll
         for (int a = 0; a < RT; a++) {
