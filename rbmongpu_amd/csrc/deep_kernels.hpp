@@ -46,7 +46,7 @@ hipError_t launch_deep_eval(const DeepDev<T>& md, const OpDev& op, int has_op, i
 template <typename T>
 hipError_t launch_deep_mc(const DeepDev<T>& md, const OpDev& op, int has_op, const McParams& mp, const Records& rec,
                           uint32_t* counts, hipStream_t stream);
-// R[q][k] = sum_s coef_q[s] conj(O[s][k]) over materialised O rows (K per sample)
+// partials[b][k] = sum over chunk b of coef[s] conj(O[s][k]), materialised O rows (K per sample)
 template <typename T>
 hipError_t launch_rows_reduce(int64_t n, int64_t K, const void* O, const cx<double>* coef, int64_t chunk,
                               int nblocks, cx<double>* partials, hipStream_t stream);

@@ -437,13 +437,15 @@ __global__ __launch_bounds__(256) void k_eval_rbm(RbmDev<T> md, OpDev op, int ha
 }
 
 // ---------------------------------------------------------------------------
-// Per-sample coefficients and scalar records (FP64).
+// Scalar sums over the samples and per-sample coefficients (FP64).
 //   weight w = mult[s] for runs of equal samples, else
 //            exact ? num_configs * exp(2 (log prefactor + Re log psi)) : 1
 //     (ExactSummation.hpp:75, Psi.hpp:133-136)
-//   mode 0 (energy):   coef0 = w, coef1 = w E;  sc = {w, w E, w |E|^2}
-//   mode 1 (distance): HilbertSpaceDistance.cu:83-105 with log psi' in lp2:
-//     coef0 = w omega, coef1 = w ratio; sc = {w omega, w ratio, w norm}
+// k_scalar_sums, modes 0 (energy), 1 (distance, HilbertSpaceDistance.cu:83-105
+// with log psi' in lp2), 6 (corrected), 7 (difference), 8 (probability ratio):
+// sums of up to four terms of a sample (scalar_terms).
+// k_coef, modes 2 and 3 (centred energy and distance, from the partial sums of
+// modes 0 and 1), 4 (weight), 5 (affine): one complex coefficient a sample.
 // ---------------------------------------------------------------------------
 // Weight of sample s
 RBM_DI double coef_weight(const CoefArgs& a, int64_t s, double lp_re) {
@@ -1504,6 +1506,7 @@ hipError_t launch_partials_sum(int nblocks, int64_t len, const cx<double>* parti
 }
 
 hipError_t launch_coef(const CoefArgs& a, hipStream_t stream) {
+    if (a.mode < 2 || a.mode > 5 || !a.coef || (a.mode == 3 && !a.lp2)) return hipErrorInvalidValue;
     if ((a.mode == 2 || a.mode == 3) && (!a.sums || a.n_sums < 1 || a.n_sums > SC_BLOCKS)) return hipErrorInvalidValue;
     int64_t g = (a.n + 255) / 256;
     if (g > 4096) g = 4096;
@@ -1582,6 +1585,8 @@ hipError_t launch_copy(void* dst, const void* src, size_t bytes, hipStream_t str
 
 hipError_t launch_scalar_sums(const CoefArgs& a, int nblocks, double* partials, hipStream_t stream) {
     if (nblocks < 1 || nblocks > SC_BLOCKS) return hipErrorInvalidValue;
+    if (a.mode != 0 && a.mode != 1 && (a.mode < 6 || a.mode > 8)) return hipErrorInvalidValue;
+    if ((a.mode != 0 && a.mode != 6 && !a.lp2) || (a.mode == 7 && !a.el2)) return hipErrorInvalidValue;
     hipLaunchKernelGGL(k_scalar_sums, dim3(nblocks), dim3(256), 0, stream, a, partials);
     return hipGetLastError();
 }
