@@ -850,54 +850,85 @@ static MadeInf made_inf(Ctx& c, rbmhip_made* md) {
     return mi;
 }
 
-// Launch extents of one training step (pass, weight gradients, update): for
-// every buffer a kernel of the step touches, the largest element offset its
-// launch arguments allow, against the size the step allocates for that buffer.
-// Pure host arithmetic, run before every training call and by
-// rbmhip_made_check_launches without a GPU.
+// One training step (pass, weight gradients, update): its shape, its offsets into
+// the parameters, and the elements of every buffer it uses, which the step
+// allocates from here.  (External linkage: the checks run without a GPU too.)
+namespace rbmhip {
 struct MadeStepPlan {
     MadeShape s;
     int B, Bp, tiles, splits;
     int64_t n, off_b1, off_W2, off_b2, padded;
+    // spins: 64-bit words; packed: the weights in the pass's order; loss: one step's
+    int64_t spins, params, packed, h, da, dl, xbits, bias, loss, wgrad;
 };
 
-static MadeStepPlan made_plan(int N, int H, int64_t n, int batch) {
+void made_plan(int N, int H, int64_t n, int batch, MadeStepPlan* out) {
     MadeStepPlan p{};
     p.s.N = N; p.s.H = H; p.s.Np = made_pad(N); p.s.Hp = made_pad(H);
     p.B = batch; p.Bp = made_pad(batch); p.n = n;
     p.tiles = p.Bp / 16;
     p.splits = made_wgrad_splits(p.s, p.tiles);
-    p.off_b1 = (int64_t)p.s.Hp * p.s.Np;
-    p.off_W2 = p.off_b1 + p.s.Hp;
-    p.off_b2 = p.off_W2 + (int64_t)p.s.Np * p.s.Hp;
-    p.padded = p.off_b2 + p.s.Np;
-    return p;
+    const int64_t Np = p.s.Np, Hp = p.s.Hp;
+    p.off_b1 = Hp * Np;
+    p.off_W2 = p.off_b1 + Hp;
+    p.off_b2 = p.off_W2 + Np * Hp;
+    p.padded = p.off_b2 + Np;
+    p.spins = 2 * n;
+    p.params = p.padded;
+    p.packed = 3 * Np * Hp;
+    p.h = p.da = Hp * p.Bp;
+    p.dl = Np * p.Bp;
+    p.xbits = p.tiles * Np;
+    p.bias = p.tiles * (Hp + Np);
+    p.loss = p.tiles;
+    p.wgrad = p.splits * p.padded;
+    *out = p;
 }
 
-static void made_check_extents(const MadeStepPlan& p) {
-    auto need = [](int64_t touched, int64_t size, const char* what) {
-        if (touched > size)
-            throw Error(RBMHIP_ERR_ARG, std::string("launch extent exceeds its buffer: ") + what + " touches " +
-                                            std::to_string(touched) + " elements of " + std::to_string(size));
+// The largest element that a kernel of the step touches in each buffer, from the
+// kernels' index expressions at their last workgroup and lane, against the
+// buffer's size: the first buffer that is too small, or null.  Pure host
+// arithmetic, run before every training call and by rbmhip_made_check_launches.
+const char* made_extent_fault(const MadeStepPlan& p) {
+    const int64_t Np = p.s.Np, Hp = p.s.Hp, W = Np * Hp, tile = p.tiles - 1;
+    if (!((Np == 64 || Np == 128) && Hp >= 64 && Hp <= 512 && Hp % 64 == 0)) return "padded shape of the training pass";
+    if (p.B > p.Bp || p.tiles * 16 != p.Bp) return "sample tiles";
+    if (p.splits < 1 || p.splits > p.tiles) return "an empty split of the weight gradients";
+    // row s is sample s of the whole set, or a drawn one, n - 1 at most
+    const int64_t row = p.B == p.n ? p.B - 1 : p.n - 1;
+    // lane 63's four weights of the last 16 x 16 tile of rows x cols
+    auto packed = [](int64_t rows, int64_t cols) { return ((rows / 16 - 1) * (cols / 16) + cols / 16 - 1) * 256 + 4 * 63 + 3; };
+    // v = 3 of the last 16-unit tile, sample 15, in the last tile of 16 samples
+    auto units = [&](int64_t rows) { return tile * rows * 16 + 256 * (rows / 16 - 1) + 64 * 3 + 16 * 3 + 15; };
+    // the weight gradients' 16-byte reads, 4 row tiles of the last 64-row block
+    auto rows64 = [&](int64_t rows) { return (tile * rows + rows - 64 + 48 + 15) * 16 + 4 * 3 + 3; };
+    const struct { const char* what; int64_t last, size; } use[] = {
+        {"spin words", 2 * row + 1, p.spins},
+        {"b1", p.off_b1 + Hp - 1, p.off_W2},
+        {"W2", p.off_W2 + W - 1, p.off_b2},
+        {"parameters", p.off_b2 + Np - 1, p.params},
+        {"W1, packed", packed(Hp, Np), W},
+        {"W2, packed", W + packed(Np, Hp), 2 * W},
+        {"packed weights", 2 * W + packed(Hp, Np), p.packed},
+        {"hidden activations", std::max(units(Hp), rows64(Hp)), p.h},
+        {"hidden derivatives", std::max(units(Hp), rows64(Hp)), p.da},
+        {"logit derivatives", std::max(units(Np), rows64(Np)), p.dl},
+        {"input bits", tile * Np + Np - 1, p.xbits},
+        {"bias sums", tile * (Hp + Np) + 16 * ((Hp + Np) / 16 - 1) + 15, p.bias},
+        {"loss partials", tile, p.loss},
+        {"weight-gradient partials", (int64_t)(p.splits - 1) * p.padded + p.off_W2 + (Np - 1) * Hp + Hp - 1, p.wgrad},
     };
-    const int64_t Np = p.s.Np, Hp = p.s.Hp, Bp = p.Bp, W = Np * Hp;
-    RBM_REQUIRE((Np == 64 || Np == 128) && Hp >= 64 && Hp <= 512 && Hp % 64 == 0, "padded shape of the training pass");
-    RBM_REQUIRE(p.B <= p.Bp && p.tiles * 16 == p.Bp, "sample tiles");
-    // pass: tile blk of 16 samples
-    const int64_t last = 15;
-    need(2 * p.n, 2 * p.n, "spin words");
-    need(((Hp / 16 - 1) * (Np / 16) + Np / 16 - 1) * 256 + 4 * 63 + 4, W, "W1 and W2 transposed, packed");
-    need(((Np / 16 - 1) * (Hp / 16) + Hp / 16 - 1) * 256 + 4 * 63 + 4, W, "W2, packed");
-    need(p.off_b1 + Hp, p.off_W2, "b1");
-    need(p.off_b2 + Np, p.padded, "b2");
-    need((p.tiles - 1) * Hp * 16 + 256 * (Hp / 16 - 1) + 16 * 3 + 64 * 3 + last + 1, Hp * Bp, "hidden activations");
-    need((p.tiles - 1) * Np * 16 + 256 * (Np / 16 - 1) + 16 * 3 + 64 * 3 + last + 1, Np * Bp, "logit derivatives");
-    need((p.tiles - 1) * Np + Np, p.tiles * Np, "input bits");
-    need((p.tiles - 1) * (Hp + Np) + Hp + Np, p.tiles * (Hp + Np), "bias sums");
-    // weight gradients: 64 x 64 blocks, sample tiles z, z + splits, ...
-    RBM_REQUIRE(p.splits >= 1 && p.splits <= p.tiles, "an empty split of the weight gradients");
-    need(((p.tiles - 1) * Hp + Hp - 64 + 48 + last) * 16 + 4 * 3 + 4, Hp * Bp, "rows of the weight gradients");
-    need((int64_t)(p.splits - 1) * p.padded + p.off_W2 + W, (int64_t)p.splits * p.padded, "weight-gradient partials");
+    for (const auto& u : use)
+        if (u.last >= u.size) return u.what;
+    return nullptr;
+}
+}  // namespace rbmhip
+
+static MadeStepPlan made_checked_plan(int N, int H, int64_t n, int batch) {
+    MadeStepPlan p;
+    made_plan(N, H, n, batch, &p);
+    if (const char* what = made_extent_fault(p)) throw Error(RBMHIP_ERR_ARG, std::string("launch extent exceeds its buffer: ") + what);
+    return p;
 }
 
 // The step's buffers and constant arguments.
@@ -907,16 +938,16 @@ static MadeStep made_step_args(Ctx& c, rbmhip_made* md, const MadeStepPlan& p, c
     a.N = p.s.N; a.B = p.B; a.Bp = p.Bp; a.n = p.n;
     a.spins = spins;
     const float* P = md->P();
-    float* packed = reinterpret_cast<float*>(c.buf("made_packed", (size_t)(3 * Np * Hp) * sizeof(float)));
+    float* packed = reinterpret_cast<float*>(c.buf("made_packed", (size_t)p.packed * sizeof(float)));
     a.W1 = packed; a.b1 = P + p.off_b1; a.W2 = packed + Np * Hp; a.b2 = P + p.off_b2; a.W2t = packed + 2 * Np * Hp;
     a.inv_batch = 1.0f / (float)p.B;
-    a.hT = reinterpret_cast<float*>(c.buf("made_h", (size_t)(Hp * p.Bp) * sizeof(float)));
-    a.daT = reinterpret_cast<float*>(c.buf("made_da", (size_t)(Hp * p.Bp) * sizeof(float)));
-    a.dlT = reinterpret_cast<float*>(c.buf("made_dl", (size_t)(Np * p.Bp) * sizeof(float)));
-    a.xbits = reinterpret_cast<uint16_t*>(c.buf("made_x", (size_t)(p.tiles * Np) * sizeof(uint16_t)));
-    a.bias_part = reinterpret_cast<float*>(c.buf("made_bias", (size_t)(p.tiles * (Hp + Np)) * sizeof(float)));
+    a.hT = reinterpret_cast<float*>(c.buf("made_h", (size_t)p.h * sizeof(float)));
+    a.daT = reinterpret_cast<float*>(c.buf("made_da", (size_t)p.da * sizeof(float)));
+    a.dlT = reinterpret_cast<float*>(c.buf("made_dl", (size_t)p.dl * sizeof(float)));
+    a.xbits = reinterpret_cast<uint16_t*>(c.buf("made_x", (size_t)p.xbits * sizeof(uint16_t)));
+    a.bias_part = reinterpret_cast<float*>(c.buf("made_bias", (size_t)p.bias * sizeof(float)));
     a.loss_part = loss_part;
-    a.wgrad_part = reinterpret_cast<float*>(c.buf("made_wgrad", (size_t)(p.splits * p.padded) * sizeof(float)));
+    a.wgrad_part = reinterpret_cast<float*>(c.buf("made_wgrad", (size_t)p.wgrad * sizeof(float)));
     a.off_b1 = p.off_b1; a.off_W2 = p.off_W2; a.off_b2 = p.off_b2; a.padded = p.padded;
     c.launch("made_pack", [&] { return launch_made_pack(p.s, P, P + p.off_W2, packed, c.stream); });
     return a;
@@ -2999,7 +3030,7 @@ int rbmhip_made_check_launches(int N, int H, int64_t n, int batch) {
     return guard([&] {
         RBM_REQUIRE(N >= 1 && N <= 128 && H >= 1 && made_pad(H) <= 512 && n > 0 && batch > 0 && batch <= (1 << 24),
                     "bad arguments");
-        made_check_extents(made_plan(N, H, n, batch));
+        (void)made_checked_plan(N, H, n, batch);
     });
 }
 
@@ -3023,12 +3054,11 @@ int rbmhip_made_loss_grad(rbmhip_made* made, const uint64_t* spins, int64_t n, d
         Ctx& c = ctx();
         made_check_device(c, made);
         const int B = (int)n;
-        const MadeStepPlan plan = made_plan(made->s.N, made->s.H, n, B);
-        made_check_extents(plan);
-        uint64_t* ds = reinterpret_cast<uint64_t*>(c.buf("made_in", (size_t)n * 2 * sizeof(uint64_t)));
+        const MadeStepPlan plan = made_checked_plan(made->s.N, made->s.H, n, B);
+        uint64_t* ds = reinterpret_cast<uint64_t*>(c.buf("made_in", (size_t)plan.spins * sizeof(uint64_t)));
         c.h2d(ds, spins, (size_t)n * 2 * sizeof(uint64_t));
         const int tiles = plan.tiles;
-        double* part = reinterpret_cast<double*>(c.buf("made_part", (size_t)tiles * sizeof(double)));
+        double* part = reinterpret_cast<double*>(c.buf("made_part", (size_t)plan.loss * sizeof(double)));
         const MadeStep a = made_step_args(c, made, plan, ds, part);
         MadeUpdate u{};
         u.grad = made->G();
@@ -3058,12 +3088,11 @@ int rbmhip_made_train(rbmhip_made* made, const uint64_t* spins, int64_t n, int s
         made_check_device(c, made);
         if (steps == 0) return;
         const int B = batch;
-        const MadeStepPlan plan = made_plan(made->s.N, made->s.H, n, B);
-        made_check_extents(plan);
-        uint64_t* ds = reinterpret_cast<uint64_t*>(c.buf("made_train_in", (size_t)n * 2 * sizeof(uint64_t)));
+        const MadeStepPlan plan = made_checked_plan(made->s.N, made->s.H, n, B);
+        uint64_t* ds = reinterpret_cast<uint64_t*>(c.buf("made_train_in", (size_t)plan.spins * sizeof(uint64_t)));
         c.h2d(ds, spins, (size_t)n * 2 * sizeof(uint64_t));
         const int tiles = plan.tiles;
-        double* part = reinterpret_cast<double*>(c.buf("made_train_part", (size_t)steps * tiles * sizeof(double)));
+        double* part = reinterpret_cast<double*>(c.buf("made_train_part", (size_t)steps * plan.loss * sizeof(double)));
         MadeStep a = made_step_args(c, made, plan, ds, part);
         a.draw = (int64_t)batch != n;   // else the whole sample set, in order, every step
         a.seed_lo = (uint32_t)seed;
