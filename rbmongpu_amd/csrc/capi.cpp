@@ -1692,21 +1692,23 @@ static cx<double> cxd(cd z) { return mk(z.real(), z.imag()); }
 constexpr double PAIR_KEEP = 0.1;
 constexpr int PAIR_MIN_P = 2048;
 
+// Q[j] = sum w |T_j|^2 in FP64, on its way to the host until the next sync()
+template <typename T>
+static void unit_squares(Ctx& c, int M, const Samples& s, const cx<double>* w, std::vector<cd>& Q) {
+    const int64_t chunk = std::max<int64_t>(64, (s.n + 1023) / 1024), nb = (s.n + chunk - 1) / chunk;
+    cx<double>* part = reinterpret_cast<cx<double>*>(c.buf("sqpart", (size_t)(nb * M) * sizeof(cx<double>)));
+    cx<double>* out = reinterpret_cast<cx<double>*>(c.buf("sqout", (size_t)M * sizeof(cx<double>)));
+    c.launch("s_matrix", [&] { return launch_unit_squares<T>(s.n, M, chunk, s.tanh, w, part, c.stream); });
+    c.launch("s_matrix", [&] { return launch_partials_sum((int)nb, M, part, out, c.stream); });
+    Q.resize((size_t)M);
+    c.d2h(Q.data(), out, Q.size() * sizeof(cx<double>));
+}
+
 // Whether every O_(p,j) = s_p T_j keeps PAIR_KEEP of its unit's spread, from the
 // contraction R of the weights and sum w |T_j|^2, both in FP64: before the moments
 // are formed, so that a model that has to take the Gram product pays for that
 // alone.
-template <typename T>
-static bool pairs_keep_accuracy(Ctx& c, int N, int M, const Samples& s, double n, const cx<double>* w,
-                                const std::vector<cd>& R) {
-    const int64_t chunk = std::max<int64_t>(64, (s.n + 1023) / 1024), nb = (s.n + chunk - 1) / chunk;
-    cx<double>* part = reinterpret_cast<cx<double>*>(c.buf("okpart", (size_t)(nb * M) * sizeof(cx<double>)));
-    cx<double>* out = reinterpret_cast<cx<double>*>(c.buf("okout", (size_t)M * sizeof(cx<double>)));
-    c.launch("s_matrix", [&] { return launch_unit_squares<T>(s.n, M, chunk, s.tanh, w, part, c.stream); });
-    c.launch("s_matrix", [&] { return launch_partials_sum((int)nb, M, part, out, c.stream); });
-    std::vector<cd> Q((size_t)M);
-    c.d2h(Q.data(), out, Q.size() * sizeof(cx<double>));
-    c.sync();
+static bool pairs_keep_accuracy(int N, int M, double n, const std::vector<cd>& R, const std::vector<cd>& Q) {
     const double z = R[(size_t)M].real() / n;   // sum w / n
     if (!(z > 0.0)) return false;
     for (int j = 0; j < M; j++) {
@@ -1779,8 +1781,10 @@ static cx<double>* s_matrix_centred(Ctx& c, rbmhip_psi* psi, rbmhip_ens* ens, co
     c.launch("coef", [&] { return launch_coef(a, c.stream); });
     cx<double>* S = reinterpret_cast<cx<double>*>(c.buf("s_centred", (size_t)P * P * sizeof(cx<double>)));
     if (P >= PAIR_MIN_P) {
-        const std::vector<cd> R = ok_contract<T>(c, N, M, s.n, s.tanh, s.spins, w, true);
-        if (pairs_keep_accuracy<T>(c, N, M, s, n, w, R)) {
+        std::vector<cd> Q;
+        unit_squares<T>(c, M, s, w, Q);
+        const std::vector<cd> R = ok_contract<T>(c, N, M, s.n, s.tanh, s.spins, w, true);   // waits for both
+        if (pairs_keep_accuracy(N, M, n, R, Q)) {
             s_matrix_pairs<T>(c, psi, s, n, eps, w, a.exact || a.mult, R, P, S);
             return S;
         }
