@@ -211,7 +211,11 @@ int rbmhip_difference(rbmhip_psi* psi, rbmhip_psi* psi_prime, rbmhip_op* const* 
 int rbmhip_s_matrix(rbmhip_psi* psi, rbmhip_ens* ens, double* out);
 /* Centred, weighted S-matrix S_kl = <conj(O_k - <O_k>) (O_l - <O_l>)> over the
  * parameters that have an O_k (the num_params - 2N entries of `params` after
- * alpha and beta), P x P complex, FP32 MFMA products accumulated in FP64.  No
+ * alpha and beta), P x P complex, with the averages over num_steps as they are
+ * (an exact sum of a psi that is not normalised is not rescaled).  FP32 products
+ * on the matrix cores accumulated in FP64: second moments by pairs of spins and
+ * pairs of units from 2048 parameters, where no O_k loses more than nine tenths
+ * of its unit's spread, else the Gram product of the centred O_k rows.  No
  * reference counterpart: the reference's S (get_S_matrix above) is unweighted
  * and uncentred and feeds no solver. */
 int rbmhip_s_matrix_centred(rbmhip_psi* psi, rbmhip_ens* ens, double* out);

@@ -1673,14 +1673,19 @@ static cx<double> cxd(cd z) { return mk(z.real(), z.imag()); }
 //
 // From PAIR_MIN_P parameters the second moments come from pairs of spins and
 // pairs of units (k_pair_moments), an eighth of the Gram product's matrix work
-// at 36 spins and 144 units: 7.4 ms against 40.3 ms on 65 536 samples.  They
-// are also the more accurate (1.1e-7 of the largest entry against 5.6e-6, 18
-// spins, 36 units, 28 700 samples): the FP32 sums of the matrix cores round
-// toward zero, and the Gram product's longer ones lose 3.4e-6 of the diagonal
-// on average.  Divided by a small eps that difference is visible in an update
-// (up to 5e-5 of it at eps = 1e-2 below a thousand parameters), so smaller
-// models, whose Gram product takes 1.7 to 4.9 ms (32 768 samples), keep it and the
-// updates they had.
+// at 36 spins and 144 units: 7.2 ms against 40.3 ms on 65 536 samples.  They are
+// also the more accurate: the Gram product's FP32 sums over up to 30 000 samples
+// lose 3e-6 of a variance on average and up to 7e-5 where one value repeats
+// (visible biases), the pairs' over 4 096 2e-7 to 4e-6 of sqrt(S_kk S_ll).
+//
+// PAIR_MIN_P is not where the two cost the same: S takes, pairs and Gram product,
+// 0.23 and 1.88 ms at 816 parameters, 0.57 and 2.98 at 1 800, 0.83 and 5.69 at
+// 2 200, 1.19 and 6.19 at 2 664, 4.2 and 22.0 at 5 328 (32 768 samples), and pairs
+// are ahead down to 216.  Below it a model keeps the S, and with it the updates,
+// that it had before there were pairs: they would move by 3e-5 to 5e-5 at
+// eps = 1e-2, which is the Gram product's rounding divided by eps, for at most
+// 2.4 ms of a step.
+//
 // S_kl from pairs is a difference of moments, whose rounding is in proportion to
 // the spreads V_j = <|T_j - <T_j>|^2> of its units, whatever is left of them in
 // the variance of O_k = s_p T_j: little where a unit follows one spin, also a

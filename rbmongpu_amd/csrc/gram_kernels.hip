@@ -177,8 +177,10 @@ hipError_t launch_gram_lower(int ld, int K, const uint32_t* A, double* C, const 
 // A wavefront owns RT <= 12 row tiles and CT = 3 column tiles of one sample
 // split: B is formed once for RT row tiles (about 65 vector instructions per
 // column tile and K step against RT x 3 MFMAs of 16 cycles), and the 4 RT CT
-// accumulators leave two wavefronts per SIMD.  6x6 Heisenberg, M = 144, 65 536
-// samples: 6.6 ms, 43 % of the MFMA issue rate of its 2.36 ms, and 0.8 ms for
+// accumulators leave two wavefronts per SIMD; from nine row tiles up some of
+// the other registers go to scratch (18, 38, 60, 80 a lane at 9, 10, 11, 12).
+// 6x6 Heisenberg, M = 144 (11 row tiles), 65 536 samples: 6.4 ms, 0.92 PFLOP/s of
+// bfloat16 products, the matrix pipes busy 39 % of the cycles, and 0.8 ms for
 // the operands and the assembly, where the Gram product took 37.6 + 2.7 ms;
 // what it waits for now is the loads and vector work of B, formed again by
 // each of the 4 row groups.  Every PAIR_FLUSH blocks the FP32
