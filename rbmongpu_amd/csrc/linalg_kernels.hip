@@ -74,6 +74,8 @@ RBM_DI void mfma_herk(doublex4& re, doublex4& im, cx<double> x, cx<double> y) {
 // positive sets *info = index + 1, if none had, and is replaced by 1 so that the
 // factorisation runs to the end.  Compact loops: unrolled over j the code of one
 // use, 40 KiB, took longer to fetch than to execute (n = 32: 40 us against 12).
+// Columns past the matrix are left out, as in the substitutions (n = 1, a whole
+// call: 70 us with all of them, 54 so).
 RBM_DI void potrf_store(int n, int k0, cx<double> (*L)[CLD], cx<double>* __restrict__ A, int* __restrict__ info) {
     const int i = threadIdx.x & 31, g = threadIdx.x >> 5;
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
@@ -84,7 +86,7 @@ RBM_DI void potrf_store(int n, int k0, cx<double> (*L)[CLD], cx<double>* __restr
 #pragma unroll
     for (int q = 0; q < 4; q++)
 #pragma unroll 1
-        for (int gj = 0; gj < 8; gj++) {
+        for (int gj = 0; gj < (n - k0 - 8 * q < 8 ? n - k0 - 8 * q : 8); gj++) {   // the identity's columns are done
             const int j = 8 * q + gj;
             if (wave == gj >> 1) {
                 double d = lane_bcast(a[q].re, j + 32 * (gj & 1)), sd, rs;
@@ -594,7 +596,7 @@ __global__ __launch_bounds__(512) void k_trsv_forward(int n, int p0, int k0, con
         const doublex2 a = load2(Ls + tri(32 * (wave & 3) + j, 32 * (wave & 3) + (m < j ? m : 0)));
         L[m] = m < j ? a * rd : doublex2{0.0, 0.0};
     }
-    for (int s = 0; s < CB / NB; s++) {
+    for (int s = 0; s < CB / NB && k0 + NB * s < n; s++) {   // identity rows past the matrix are left
         if (wave == s) {
             cx<double> v = mk(xs[32 * s + j].re * rd, xs[32 * s + j].im * rd);
 #pragma unroll
@@ -607,7 +609,7 @@ __global__ __launch_bounds__(512) void k_trsv_forward(int n, int p0, int k0, con
         }
         __syncthreads();
         // rows below in the block: 8 lanes a row, 4 columns each
-        for (int i = 32 * (s + 1) + (tid >> 3); i < CB; i += 64) {
+        for (int i = 32 * (s + 1) + (tid >> 3); i < CB && k0 + i < n; i += 64) {
             cx<double> u = mk(0.0, 0.0);
 #pragma unroll
             for (int m = 0; m < 4; m++) {
@@ -686,7 +688,7 @@ __global__ __launch_bounds__(512) void k_trsv_backward(int n, int p0, int k0, co
         const doublex2 a = load2(Ls + tri(32 * (wave & 3) + m, 32 * (wave & 3) + (m > j ? j : 0)));
         L[m] = m > j ? a * rd : doublex2{0.0, 0.0};
     }
-    for (int s = CB / NB - 1; s >= 0; s--) {
+    for (int s = (n - k0 < CB ? n - k0 - 1 : CB - 1) / NB; s >= 0; s--) {
         if (wave == s) {
             cx<double> v = mk(xs[32 * s + j].re * rd, xs[32 * s + j].im * rd);
 #pragma unroll
