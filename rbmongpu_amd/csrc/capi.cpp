@@ -237,6 +237,13 @@ struct Ctx {
         }
         RBM_HIPCHK(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, stream));
     }
+    // A copy with nothing before it, waited for at once (parameters in or out):
+    // the runtime's own staging is 2 to 4 us the cheaper there (a 20 x 64 proposal
+    // network's parameters 11.8 us in and 10.8 out against 15.9 and 14.0).
+    void copy_alone(void* dst, const void* src, size_t bytes, hipMemcpyKind kind) {
+        RBM_HIPCHK(hipMemcpyAsync(dst, src, bytes, kind, stream));
+        sync();
+    }
     // n values of V at dst, formed by fill(V*)
     template <class V, class F>
     void upload(void* dst, size_t n, F&& fill) {
@@ -3016,8 +3023,7 @@ int rbmhip_made_get_params(rbmhip_made* made, float* out) {
         Ctx& c = ctx();
         made_check_device(c, made);
         std::vector<float> dev((size_t)made->padded);
-        c.d2h(dev.data(), made->params.p, dev.size() * sizeof(float));
-        c.sync();
+        c.copy_alone(dev.data(), made->params.p, dev.size() * sizeof(float), hipMemcpyDeviceToHost);
         const std::vector<float> flat = made_unpad_params(made, dev);
         std::memcpy(out, flat.data(), flat.size() * sizeof(float));
     });
@@ -3029,8 +3035,7 @@ int rbmhip_made_set_params(rbmhip_made* made, const float* params) {
         Ctx& c = ctx();
         made_check_device(c, made);
         const std::vector<float> dev = made_pad_params(made, params);
-        c.h2d(made->params.p, dev.data(), dev.size() * sizeof(float));
-        c.sync();
+        c.copy_alone(made->params.p, dev.data(), dev.size() * sizeof(float), hipMemcpyHostToDevice);
         made->inf_valid = false;
     });
 }
